@@ -1475,15 +1475,15 @@ int jw_batch_evolve(jw_batch* b, int coupling, int kernel, double step, const jw
     // from here on the tables (and the graph, once built) are this key's
     b->key = key;
     b->have_key = true;
-    // every group's stream must be idle before the origin stream forks to it
+    // coupling tables first: they are built on the groups' streams, their builds are
+    // not captured, and a launch over all groups runs on the origin stream alone.
+    // Every group's stream must be idle before the origin stream forks to it.
+    for (auto& g : b->g) {
+        const double *p, *k;
+        if (int e = batch_tables(g, coupling, al, &p, &k)) return e;
+    }
     for (auto& g : b->g) HIP_CHECK(hipStreamSynchronize(g.ctx->stream));
     if (!b->graph && nsteps >= K) {
-        // coupling tables first: their builds are not captured
-        for (auto& g : b->g) {
-            const double *p, *k;
-            if (int e = batch_tables(g, coupling, al, &p, &k)) return e;
-            HIP_CHECK(hipStreamSynchronize(g.ctx->stream));
-        }
         hipGraph_t graph = nullptr;
         HIP_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         int rc = JW_OK;
