@@ -115,20 +115,15 @@ int check_field(const jw_field* f, const jw_ctx* c, int t, const char* name) {
     return JW_OK;
 }
 
-// the fused step's intermediate layout when none is selected.  Measured at
-// N = 2048 (steps/s, FP64 / FP32 storage, correlated / fixed coupling):
-// row-major 382 / 568, 418 / 653; 4-row blocks 363 / 474, 415 / 536; 8-row
-// blocks 345 / 507, 407 / 559.  Row-major everywhere.
 // the column passes of layouts 1, 4 and 8 read the 16-row-blocked sqrt(alpha) table
 bool uses_sa16(int layout) { return layout == 1 || layout == 4 || layout == 8 || layout >= 16; }
 
-// N = 8192: 16-byte strips (the only ones that fit LDS); N = 4096: 16-byte
-// strips in FP32 (measured 143 against 125 steps/s for the X + Y column tiles,
-// correlated, momentum-space noise), the X + Y tiles in FP64 (89 against 85);
-// otherwise row-major X + Y column tiles
-int default_layout(int N, int corr, int fp32) {
-    (void)corr;
-    return N == 8192 || (N == 4096 && fp32) ? 32 : 0;
+// the intermediate layout when none is selected: row-major planes, whose column pass holds its strip in registers; 16-byte strips
+// one plane at a time for FP64 at N = 8192 (two planes of one column take the
+// registers of more than a CU) and for the matrix-core stages of the large lattices
+int default_layout(int N, int fp32, int mfma) {
+    if (!fp32) return N == 8192 ? 32 : 0;
+    return N >= 4096 && mfma ? 32 : 0;
 }
 
 // nsteps generator-basis steps: the fused passes or the unfused kernel sequence
@@ -190,7 +185,7 @@ int evolve_sin(jw_ctx* c, jw_field* U, int coupling, double step, const jw_alpha
     const bool large = jw::large_supported(c->N) && !c->unfused;
     if (int e = check_kspace(c, coupling, fused || large)) return e;
     const int saved_layout = c->layout;
-    if (c->layout < 0) c->layout = default_layout(c->N, corr, 0);
+    if (c->layout < 0) c->layout = default_layout(c->N, 0, c->fft_mfma);
     if ((fused || large) && sa_k && uses_sa16(c->layout)) {
         if (tabs) {
             const hipError_t he = jw::block16(c, tabs + V, tabs);
@@ -1071,7 +1066,7 @@ int jw_evolve_mixed(jw_ctx* c, jw_field* U, int coupling, int kernel, double ste
     const bool large = jw::large_supported(c->N) && !c->unfused;
     if (int e = check_kspace(c, coupling, fused || large)) return e;
     const int saved_layout = c->layout;
-    if (c->layout < 0) c->layout = default_layout(c->N, corr, 1);
+    if (c->layout < 0) c->layout = default_layout(c->N, 1, c->fft_mfma);
     int rc = JW_OK;
     if ((fused || large) && sa_k && uses_sa16(c->layout)) {
         rc = ensure_sa16(c);

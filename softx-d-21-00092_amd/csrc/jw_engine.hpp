@@ -32,6 +32,7 @@
 #pragma once
 
 #include "jw_common.hpp"
+#include "jw_regfft.hpp"
 
 namespace jw {
 
@@ -454,7 +455,165 @@ __global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_uxiu_co
 }
 
 // ---------------------------------------------------------------------------
-// column pass: Z[p] = F_col^-1[ i (kx X^[p] + ky Y^[p]) / V ], X^ = F_col X
+// column pass on row-major planes, transforms in registers (jw_regfft.hpp):
+//   Z[p] = F_col^-1[ i (kx X^[p] + ky Y^[p]) / V ], X^ = F_col X
+//   kx = -2 pi c pbarX / phat2 (c = sa(k) for MODE 1, else 1), zero at k = 0.
+//   CORR: X^, Y^ are first multiplied by sa(k) (MODE 2) and F_col^-1[X^ / V] is
+//   written back over X (likewise Y).
+//   GEN (with CORR): X^, Y^ are not transformed from X, Y but drawn per mode
+//   (kspace_normals4, plane pair p = bi.by, noise key from ns); X and Y then
+//   receive the row spectra of the position-space noise.
+// X, Y: row spectra of plane p; one workgroup per strip of W columns and plane
+// pair.  A thread holds PT points of one column of X and of Y; LDS holds one
+// plane of the strip for the exchanges, and the (4 sin^2, sin) table of kx.
+//
+// What bounds it: the loaded pass moves 12 planes at 3.1-3.2 TB/s (FP64 and FP32
+// at N = 2048; the bare access pattern reaches 4.6 TB/s), the drawing pass is
+// bound by the noise's instructions.  64-byte row segments (W = 4 FP64, 8 FP32)
+// take the bare pattern from 2.7 TB/s (16 bytes) and 3.7 (32 bytes) to 4.6, and
+// the registers of a CU hold four times the strip that the LDS-resident form
+// (k_col_kmult) could, with 4 workgroup barriers instead of about 20.
+// N = 2048, us per launch, k_col_kmult -> this: loaded FP64 420 -> 258, FP32 241 ->
+// 135; correlated FP64 660 -> 485, FP32 445 -> 212; drawing FP64 490 -> 355, FP32
+// 295 -> 171.
+// ---------------------------------------------------------------------------
+template <int N, typename C>
+struct ColR {
+    static constexpr bool F64 = sizeof(C) == sizeof(double2);
+    static constexpr int WSEG = 64 / (int)sizeof(C);                     // columns of a 64-byte segment
+    // the widest strip whose X and Y fit the registers of one CU (FP64 8192, FP32
+    // 16384 points), 64-byte segments at most
+    static constexpr int WMAX = (F64 ? 8192 : 16384) / N;
+    static constexpr int W = WMAX < WSEG ? WMAX : (N / RegFft<N>::PT * WSEG < 64 ? 64 / (N / RegFft<N>::PT) : WSEG);
+    static constexpr int NT = N / RegFft<N>::PT * W;
+    static constexpr int ELEMS = N * W;                                  // of C in LDS
+    static constexpr bool TAB = ELEMS * (int)sizeof(C) + N * 16 <= 160 * 1024;
+    static constexpr int LDS = ELEMS + (TAB ? N * 16 / (int)sizeof(C) : 0);
+    // registers: 256 (FP64; 32 points a thread) or 128 a thread
+    static constexpr int REGS = F64 || RegFft<N>::PT > 16 ? 256 : 128;
+    static constexpr int WAVES = 512 / REGS;
+    static_assert(W >= 1 && NT >= 64 && NT * REGS <= 512 * 256, "column strip");
+};
+
+// v, defined only once d is: what is computed from it is not started before
+template <typename T>
+__device__ __forceinline__ int after(int v, T d) {
+    asm volatile("" : "+v"(v) : "v"(d));
+    return v;
+}
+
+// lds: N W elements; kt: N (q4, sb) pairs (TAB), filled here by the whole workgroup
+template <int N, int CORR, int GEN, int MODE, typename C>
+__device__ __forceinline__ void col_reg_body(C* lds, double2* kt, BlockIx bi, C* __restrict__ Z, C* __restrict__ X,
+                                             C* __restrict__ Y, size_t V, const double* __restrict__ q4,
+                                             const double* __restrict__ sb, const double* __restrict__ sa,
+                                             const C* __restrict__ tw, NoiseSrc ns) {
+    static_assert(!GEN || CORR, "drawn spectra are written back as position-space noise");
+    static_assert(!CORR || GEN || MODE == 2, "transformed noise is written back only where it is scaled");
+    typedef typename scalar_of<C>::type T;
+    typedef RegFft<N> F;
+    typedef ColR<N, C> CR;
+    constexpr int PT = F::PT, W = CR::W;
+    constexpr size_t RS = (size_t)F::T * N;             // elements between a thread's points
+    const int col0 = xcd_strip(bi.bx, N / W) * W;
+    Z += zofs_z(bi.bz, 4, V) + (size_t)bi.by * V;
+    X += zofs_z(bi.bz, 8, V) + (size_t)bi.by * V;
+    Y += zofs_z(bi.bz, 8, V) + (size_t)bi.by * V;
+    // the thread's first element: uniform plane and row offsets, one 32-bit offset per thread
+    auto at = [&]() -> unsigned {
+        const int t = opaque_v(bi.tid);
+        return (unsigned)((t / W) * N + col0 + t % W);
+    };
+    if constexpr (CR::TAB) {
+        for (int i = threadIdx.x; i < N; i += blockDim.x) kt[i] = make_double2(q4[i], sb[i]);
+        if constexpr (GEN) __syncthreads();             // otherwise the transforms' barriers do
+    }
+    C x[PT], y[PT], z[CORR ? PT : 1];
+    int tk = bi.tid;
+    if constexpr (!GEN) {
+        const unsigned o = at();
+#pragma unroll
+        for (int r = 0; r < PT; r++) x[r] = (X + r * RS)[o];
+#pragma unroll
+        for (int r = 0; r < PT; r++) y[r] = (Y + r * RS)[o];        // in flight under the transform of X
+        reg_fft_fwd<N, W, true>(x, lds, tw_fft(tw), opaque_v(bi.tid));
+        reg_fft_fwd<N, W, false>(y, lds, tw_fft(tw), opaque_v(bi.tid));
+        tk = after(tk, y[PT - 1].x);
+    }
+    const NoiseSrc nk = batch_noise_z(ns, V, bi.bz);
+    const double invV = 1.0 / ((double)N * (double)N);
+    const int j = tk / W, ky = col0 + tk % W;
+    const int kx0 = reg_freq<N>(j / F::N3, j % F::N3, 0);
+    const unsigned k0 = (unsigned)(kx0 * N + ky);
+    const double q4y = q4[ky];
+    const T sby = (T)sb[ky];
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+        const int dk = reg_freq<N>(0, 0, q);            // kx = kx0 + dk
+        if constexpr (GEN) {
+            T g[4];
+            kspace_normals4(k0 + (unsigned)(dk * N), nk.step, nk.tag, bi.by, nk.seed, nk.traj, g);
+            x[q] = mkc<C>(g[0] * (T)N, g[1] * (T)N);            // sqrt(V) = N
+            y[q] = mkc<C>(g[2] * (T)N, g[3] * (T)N);
+        }
+        double2 kq;
+        if constexpr (CR::TAB) kq = kt[kx0 + dk];
+        else kq = make_double2((q4 + dk)[kx0], (sb + dk)[kx0]);
+        // kernel factors in the element type: one FP64 division per pair in FP64,
+        // one FP32 division in the mixed form (whose spectra are FP32)
+        const double cc = MODE == 1 ? (sa + (size_t)dk * N)[k0] : 1.0;
+        T f = (T)(-2.0 * M_PI * invV * cc) / (T)(kq.x + q4y);
+        if (q == 0 && k0 == 0) f = 0;
+        const T fx = f * (T)kq.y, fy = f * sby;
+        if constexpr (MODE == 2) {
+            const T s = (T)(sa + (size_t)dk * N)[k0];
+            x[q] = cscale(x[q], s);
+            y[q] = cscale(y[q], s);
+        }
+        const C zq = mkc<C>(-(fx * x[q].y + fy * y[q].y), fx * x[q].x + fy * y[q].x);   // i (fx x + fy y)
+        // the fences end each element before the next (an interleaved order spills)
+        if constexpr (CORR) {
+            z[q] = zq;
+            x[q] = cscale(x[q], (T)invV);
+            y[q] = cscale(y[q], (T)invV);
+            fence(y[q]);
+            fence(z[q]);
+        } else {
+            x[q] = zq;
+        }
+        fence(x[q]);
+    }
+    reg_fft_inv<N, W, true>(x, lds, tw_fft(tw), opaque_v(bi.tid));
+    {
+        C* const O = CORR ? X : Z;
+        const unsigned o = at();
+#pragma unroll
+        for (int r = 0; r < PT; r++) (O + r * RS)[o] = x[r];
+    }
+    if constexpr (CORR) {
+        reg_fft_inv<N, W, false>(y, lds, tw_fft(tw), opaque_v(bi.tid));
+        const unsigned oy = at();
+#pragma unroll
+        for (int r = 0; r < PT; r++) (Y + r * RS)[oy] = y[r];
+        reg_fft_inv<N, W, false>(z, lds, tw_fft(tw), opaque_v(bi.tid));
+        const unsigned oz = at();
+#pragma unroll
+        for (int r = 0; r < PT; r++) (Z + r * RS)[oz] = z[r];
+    }
+}
+
+template <int N, int CORR, int GEN, int MODE, typename C>
+__global__ __launch_bounds__((ColR<N, C>::NT), (ColR<N, C>::WAVES)) void k_col_reg(
+    C* __restrict__ Z, C* __restrict__ X, C* __restrict__ Y, size_t V, const double* __restrict__ q4,
+    const double* __restrict__ sb, const double* __restrict__ sa, const C* __restrict__ tw, NoiseSrc ns) {
+    __shared__ __align__(16) C lds[ColR<N, C>::LDS];
+    col_reg_body<N, CORR, GEN, MODE, C>(lds, reinterpret_cast<double2*>(lds + ColR<N, C>::ELEMS), own_block(), Z, X, Y,
+                                        V, q4, sb, sa, tw, ns);
+}
+
+// ---------------------------------------------------------------------------
+// column pass in LDS (the pair-interleaved layout, and the matrix-core stages on
+// row-major planes): Z[p] = F_col^-1[ i (kx X^[p] + ky Y^[p]) / V ], X^ = F_col X
 //   kx = -2 pi c pbarX / phat2 (c = sa(k) for SQRT, else 1), zero at k = 0.
 //   CORR: X^, Y^ are first multiplied by sa(k) (per-mode correlated noise;
 //   by 1 when noise_scale is 0) and F_col^-1[sa X^ / V] is written back over X
@@ -925,7 +1084,11 @@ __device__ __forceinline__ void dispatch_group(const MultiRun<C>& m, F&& f) {
 }
 template <int N> struct RowNT { static constexpr int value = RowE<N>::NT; };
 template <typename C>
-struct ColNT { template <int N> struct of { static constexpr int value = ColE<N, C, 1>::NT; }; };
+struct ColNT { template <int N> struct of { static constexpr int value = ColR<N, C>::NT; }; };
+// threads of a column launch: the strips of every size have at most that many,
+// at the registers of ColR
+template <typename C>
+struct ColMultiT { static constexpr int value = sizeof(C) == sizeof(double2) ? 512 : 1024; };
 
 // LDS of a row launch of T threads: T / NT bodies of `planes` padded rows
 template <int T, int planes, typename C>
@@ -938,15 +1101,19 @@ struct RowMultiLds {
     static constexpr int ab = a > b ? a : b;
     static constexpr int value = ab > c ? ab : c;
 };
+// LDS of a column launch: the bodies' tiles, then the (q4, sb) table they share
 template <typename C>
 struct ColMultiLds {
     template <int N>
-    static constexpr int need() { return (1024 / ColE<N, C, 1>::NT) * padded<N, 3>::value * 2 * ColE<N, C, 1>::W; }
+    static constexpr int need() {
+        return (ColMultiT<C>::value / ColR<N, C>::NT) * ColR<N, C>::ELEMS + N * 16 / (int)sizeof(C);
+    }
     static constexpr int a = need<64>() > need<128>() ? need<64>() : need<128>();
     static constexpr int b = need<256>() > need<512>() ? need<256>() : need<512>();
     static constexpr int c = need<1024>() > need<2048>() ? need<1024>() : need<2048>();
     static constexpr int ab = a > b ? a : b;
     static constexpr int value = ab > c ? ab : c;
+    static_assert(value * sizeof(C) <= 160 * 1024, "LDS of a column launch");
 };
 
 // the row (x), trajectory (z) and thread of a row body in block b of its group
@@ -995,22 +1162,21 @@ __global__ __launch_bounds__(T, RowWaves<C>::value) void k_row_update_multi(Mult
                                  g.V, ss, reunit, g.tw, 0, g.Xi, g.ns, g.sa_pos);
     });
 }
-// column passes: T = 1024; block b of a group: strip block, plane pair, trajectory
-// in that order (the order of the grouped launch's grid)
-template <typename C, int CORR, int GEN>
-__global__ __launch_bounds__(1024, 1) void k_col_kmult_multi(MultiRun<C> m, int use_v, int sqrt_coupling,
-                                                             int noise_scale) {
-    __shared__ C lds[ColMultiLds<C>::value];
-    dispatch_group<1024, ColNT<C>::template of>(m, [&](auto n, const GroupRun<C>& g, int b) {
+// column passes: the strips of a group in the order strip, plane pair, trajectory
+// (the order of the grouped launch's grid), T / NT of one trajectory in a block
+template <typename C, int CORR, int GEN, int MODE>
+__global__ __launch_bounds__((ColMultiT<C>::value), (ColR<2048, C>::WAVES)) void k_col_reg_multi(MultiRun<C> m, int use_v) {
+    __shared__ __align__(16) C lds[ColMultiLds<C>::value];
+    constexpr int T = ColMultiT<C>::value;
+    dispatch_group<T, ColNT<C>::template of>(m, [&](auto n, const GroupRun<C>& g, int b) {
         constexpr int N = decltype(n)::value;
-        typedef ColE<N, C, CORR> CE;
-        constexpr int SPB = 1024 / CE::NT, NSB = N / CE::W / SPB;
-        const int s = threadIdx.x / CE::NT;
-        const BlockIx bi{(b % NSB) * SPB + s, (b / NSB) % 4, b / (NSB * 4), (int)threadIdx.x % CE::NT};
+        typedef ColR<N, C> CR;
+        constexpr int SPB = T / CR::NT, NS = N / CR::W, NB = 4 * NS / SPB;      // blocks of a trajectory
+        const int s = threadIdx.x / CR::NT, u = (b % NB) * SPB + s;
+        const BlockIx bi{u % NS, u / NS, b / NB, (int)threadIdx.x % CR::NT};
         C* X = use_v ? g.Vv : g.Xi;
-        col_kmult_body<N, CORR, C, 0, 0, GEN>(lds + s * padded<N, 3>::value * 2 * CE::W, bi, use_v ? g.ZB : g.ZA, X,
-                                              X + 4 * g.V, g.V, sqrt_coupling, g.q4, g.sb, g.sa_k, g.tw, g.ns,
-                                              noise_scale);
+        col_reg_body<N, CORR, GEN, MODE, C>(lds + s * CR::ELEMS, reinterpret_cast<double2*>(lds + SPB * CR::ELEMS), bi,
+                                            use_v ? g.ZB : g.ZA, X, X + 4 * g.V, g.V, g.q4, g.sb, g.sa_k, g.tw, g.ns);
     });
 }
 
@@ -1022,9 +1188,21 @@ inline int row_blocks(int N, int count, int T) {
 }
 template <typename C>
 inline int col_blocks(int N, int count) {
-    const int W = 4096 / N > 16 ? 16 : 4096 / N;                          // ColE<N>::W
-    const int elems = 2 * W * N, nt = elems / 8 < 64 ? 64 : (elems / 8 > 1024 ? 1024 : elems / 8);
-    return count * 4 * (N / W) / (1024 / nt);
+    auto blocks = [&](auto n) {
+        constexpr int M = decltype(n)::value;
+        constexpr int SPB = ColMultiT<C>::value / ColR<M, C>::NT;
+        constexpr int units = 4 * (M / ColR<M, C>::W);      // strips of the four plane pairs
+        static_assert(SPB >= 1 && units % SPB == 0, "strips of a block");
+        return count * (units / SPB);
+    };
+    switch (N) {
+        case 64: return blocks(int_c<64>{});
+        case 128: return blocks(int_c<128>{});
+        case 256: return blocks(int_c<256>{});
+        case 512: return blocks(int_c<512>{});
+        case 1024: return blocks(int_c<1024>{});
+        default: return blocks(int_c<2048>{});
+    }
 }
 
 // one step of every group of a batch, one launch per kernel class (row-major
@@ -1052,12 +1230,20 @@ static hipError_t step_multi_t(hipStream_t st, MultiRun<C> m, const int* counts,
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     set_blocks(true);
-    if (a.kspace)
-        hipLaunchKernelGGL((k_col_kmult_multi<C, 1, 1>), dim3(ncol), dim3(1024), 0, st, m, 0, a.sqrt_coupling, a.corr);
-    else if (a.corr)
-        hipLaunchKernelGGL((k_col_kmult_multi<C, 1, 0>), dim3(ncol), dim3(1024), 0, st, m, 0, a.sqrt_coupling, 1);
-    else
-        hipLaunchKernelGGL((k_col_kmult_multi<C, 0, 0>), dim3(ncol), dim3(1024), 0, st, m, 0, a.sqrt_coupling, 0);
+    constexpr int TC = ColMultiT<C>::value;
+#define JW_COL_MULTI(corr, gen, mode, use_v) \
+    hipLaunchKernelGGL((k_col_reg_multi<C, corr, gen, mode>), dim3(ncol), dim3(TC), 0, st, m, use_v)
+    if (a.kspace) {
+        if (a.corr) JW_COL_MULTI(1, 1, 2, 0);
+        else if (a.sqrt_coupling) JW_COL_MULTI(1, 1, 1, 0);
+        else JW_COL_MULTI(1, 1, 0, 0);
+    } else if (a.corr) {
+        JW_COL_MULTI(1, 0, 2, 0);
+    } else if (a.sqrt_coupling) {
+        JW_COL_MULTI(0, 0, 1, 0);
+    } else {
+        JW_COL_MULTI(0, 0, 0, 0);
+    }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     set_blocks(false);
     if (wb) {
@@ -1069,7 +1255,9 @@ static hipError_t step_multi_t(hipStream_t st, MultiRun<C> m, const int* counts,
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     set_blocks(true);
-    hipLaunchKernelGGL((k_col_kmult_multi<C, 0, 0>), dim3(ncol), dim3(1024), 0, st, m, 1, a.sqrt_coupling, 0);
+    if (a.sqrt_coupling) JW_COL_MULTI(0, 0, 1, 1);
+    else JW_COL_MULTI(0, 0, 0, 1);
+#undef JW_COL_MULTI
     if ((e = hipGetLastError()) != hipSuccess) return e;
     set_blocks(false);
     if (T == 256)
@@ -1114,12 +1302,11 @@ static hipError_t col_pass(jw_ctx* c, C* Z, C* X, C* Y, const double* sa_k, int 
     const size_t V = c->V;
     const C* tw = twiddles<C>(c);
 #define JW_COL_ARGS Z, X, Y, V, sqrt_coupling, c->q4, c->sb, sa_k, tw, ns, noise_scale
-    if constexpr (BF == 0 || BF == 2) {
-        constexpr int W = ColE<N, C>::W, PI = BF == 2;
-        const dim3 grid(N / W, 4, nbatch);
-        // split-BF16 matrix-core radix-16 stages: FP32 storage, row-major layout
-        if constexpr (sizeof(C) == sizeof(float2) && BF == 0) {
+    if constexpr (BF == 0) {
+        // split-BF16 matrix-core radix-16 stages (FP32 storage)
+        if constexpr (sizeof(C) == sizeof(float2) && N <= 2048) {
             if (c->fft_mfma) {
+                const dim3 grid(N / ColE<N, C>::W, 4, nbatch);
                 if (gen)
                     hipLaunchKernelGGL((k_col_kmult<N, 1, C, 0, 1, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream,
                                        JW_COL_ARGS);
@@ -1132,12 +1319,31 @@ static hipError_t col_pass(jw_ctx* c, C* Z, C* X, C* Y, const double* sa_k, int 
                 return hipGetLastError();
             }
         }
+        typedef ColR<N, C> CR;
+        const dim3 grid(N / CR::W, 4, nbatch);
+#define JW_COL_REG(corr_, gen_, mode_)                                                                               \
+    hipLaunchKernelGGL((k_col_reg<N, corr_, gen_, mode_, C>), grid, dim3(CR::NT), 0, c->stream, Z, X, Y, V, c->q4, \
+                       c->sb, sa_k, tw, ns)
+        if (gen) {
+            if (noise_scale) JW_COL_REG(1, 1, 2);
+            else if (sqrt_coupling) JW_COL_REG(1, 1, 1);
+            else JW_COL_REG(1, 1, 0);
+        } else if (corr) {
+            JW_COL_REG(1, 0, 2);
+        } else if (sqrt_coupling) {
+            JW_COL_REG(0, 0, 1);
+        } else {
+            JW_COL_REG(0, 0, 0);
+        }
+#undef JW_COL_REG
+    } else if constexpr (BF == 2) {
+        const dim3 grid(N / ColE<N, C>::W, 4, nbatch);
         if (gen)
-            hipLaunchKernelGGL((k_col_kmult<N, 1, C, PI, 0, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream, JW_COL_ARGS);
+            hipLaunchKernelGGL((k_col_kmult<N, 1, C, 1, 0, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream, JW_COL_ARGS);
         else if (corr)
-            hipLaunchKernelGGL((k_col_kmult<N, 1, C, PI>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream, JW_COL_ARGS);
+            hipLaunchKernelGGL((k_col_kmult<N, 1, C, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream, JW_COL_ARGS);
         else
-            hipLaunchKernelGGL((k_col_kmult<N, 0, C, PI>), grid, dim3(ColE<N, C, 0>::NT), 0, c->stream, JW_COL_ARGS);
+            hipLaunchKernelGGL((k_col_kmult<N, 0, C, 1>), grid, dim3(ColE<N, C, 0>::NT), 0, c->stream, JW_COL_ARGS);
     } else {
         constexpr int CPB = ColB<N, BF, C>::CPB, NT = ColB<N, BF, C>::NT;
         const dim3 grid(N / CPB, 4, nbatch);

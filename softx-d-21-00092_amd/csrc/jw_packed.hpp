@@ -452,14 +452,17 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     return hipSuccess;
 }
 
-// the column strips of a large lattice: 16-byte segments one plane at a time
-// at N = 8192 (the only strip that fits LDS); at N = 4096 the X + Y tiles of
-// one column (layout 0, default) or one plane at a time over 16-byte segments
-// (layout 32)
+// the column strips of a large lattice: the register-held strips of layout 0 (FP32
+// at both sizes, FP64 at N = 4096), or one plane at a time over 16-byte segments
+// (layout 32; FP64 at N = 8192 has no other)
 template <typename C>
 static hipError_t step_large_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, const StepArgs& a) {
     if (a.nbatch != 1) return hipErrorInvalidValue;
-    if (c->N == 8192) return step_large_n<8192, 32>(c, U, Xi, Vv, ZA, ZB, a);
+    if (c->N == 8192) {
+        if constexpr (sizeof(C) == sizeof(float2))
+            if (c->layout == 0) return step_large_n<8192, 0>(c, U, Xi, Vv, ZA, ZB, a);
+        return step_large_n<8192, 32>(c, U, Xi, Vv, ZA, ZB, a);
+    }
     if (c->N == 4096) {
         if (c->layout == 32) return step_large_n<4096, 32>(c, U, Xi, Vv, ZA, ZB, a);
         return step_large_n<4096, 0>(c, U, Xi, Vv, ZA, ZB, a);

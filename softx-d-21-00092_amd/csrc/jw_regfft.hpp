@@ -1,0 +1,245 @@
+// jw_regfft.hpp -- the FFT of the column passes with its data in registers.
+//
+// A length-N transform is split as N = PT * N2, N2 = PT * N3 and shared by
+// T = N / PT threads of PT points each.  Forward (decimation in frequency):
+//   1. thread j < T holds x[j + T r], r < PT, and takes the PT-point DFT over r;
+//      result k1 is multiplied by w_N^(j k1);
+//   2. exchange over the workgroup: thread (g, m) = (j / N3, j % N3) receives the
+//      sub-sequence k1 = g at n2 = m + N3 a, a < PT;
+//   3. PT-point DFT over a; result b1 is multiplied by w_N2^(m b1);
+//   4. exchange among the N3 threads of a sub-sequence: thread (g, m) receives
+//      b1 = m + N3 u, u < PT / N3, for all N3 values of the other digit;
+//   5. PT / N3 DFTs of N3 points.
+// The thread then holds the frequencies reg_freq(g, m, u, b2) =
+// g + PT (m + N3 u) + PT^2 b2 in v[u N3 + b2].  The inverse runs the steps
+// backwards and ends with the positions j + T r it started from, so that a
+// pointwise factor between the two needs no reordering.
+//
+// W sequences (columns) side by side, column fastest over the lanes.  The
+// N3 * W threads of a sub-sequence sit in one wave, so step 4 needs no workgroup
+// barrier, and it stays inside the part of LDS that the same threads read
+// in step 2.  One LDS element per point, no padding: step 4 swizzles the
+// position inside a row of N3 by exclusive or with the row.
+#pragma once
+
+#include "jw_device.hpp"
+
+namespace jw {
+
+// a * e^{DIR 2 pi i k / 16} for the constant twiddles of the 16-point DFT
+template <int DIR, typename C>
+__device__ __forceinline__ C rot16(C a, int k) {
+    typedef decltype(a.x) T;
+    const T c1 = (T)0.92387953251128675612818318939679, s1 = (T)0.38268343236508977172845998403040;
+    const T h = (T)0.70710678118654752440084436210485;
+    switch (k) {
+        case 0: return a;
+        case 4: return rot_q<DIR>(a);
+        case 2: return DIR < 0 ? C{(a.x + a.y) * h, (a.y - a.x) * h} : C{(a.x - a.y) * h, (a.y + a.x) * h};
+        case 6: return DIR < 0 ? C{(a.y - a.x) * h, -(a.x + a.y) * h} : C{-(a.x + a.y) * h, (a.x - a.y) * h};
+        default: break;
+    }
+    const T c = (k == 1) ? c1 : (k == 3) ? s1 : -c1;                       // 1, 3, 9
+    const T s = (T)(DIR < 0 ? -1 : 1) * ((k == 1) ? s1 : (k == 3) ? c1 : -s1);
+    return C{a.x * c - a.y * s, a.x * s + a.y * c};
+}
+
+// in-register DFT of R points, natural order in and out
+template <int R, int DIR, typename C>
+__device__ __forceinline__ void dft_reg(C* v) {
+    if constexpr (R <= 8) {
+        if constexpr (R > 1) dft_small<R, DIR>(v);
+    } else if constexpr (R == 16) {
+        // n = 4 n1 + n2, k = k1 + 4 k2
+        C t[4][4];
+#pragma unroll
+        for (int n2 = 0; n2 < 4; n2++) {
+#pragma unroll
+            for (int n1 = 0; n1 < 4; n1++) t[n2][n1] = v[4 * n1 + n2];
+            dft_small<4, DIR>(t[n2]);
+#pragma unroll
+            for (int k1 = 1; k1 < 4; k1++) t[n2][k1] = rot16<DIR>(t[n2][k1], n2 * k1);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < 4; k1++) {
+            C u[4] = {t[0][k1], t[1][k1], t[2][k1], t[3][k1]};
+            dft_small<4, DIR>(u);
+#pragma unroll
+            for (int k2 = 0; k2 < 4; k2++) v[k1 + 4 * k2] = u[k2];
+        }
+    } else {
+        static_assert(R == 32, "radix");
+        // n = 2 n1 + n2, k = k1 + 16 k2
+        typedef decltype(v[0].x) T;
+        const T c32[8] = {(T)1.0, (T)0.98078528040323044912618223613424, (T)0.92387953251128675612818318939679,
+                          (T)0.83146961230254523707878837761791, (T)0.70710678118654752440084436210485,
+                          (T)0.55557023301960222474283081394853, (T)0.38268343236508977172845998403040,
+                          (T)0.19509032201612826784828486847702};
+        C e[16], o[16];
+#pragma unroll
+        for (int n = 0; n < 16; n++) { e[n] = v[2 * n]; o[n] = v[2 * n + 1]; }
+        dft_reg<16, DIR>(e);
+        dft_reg<16, DIR>(o);
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            C w = o[k];
+            if (k & 7) {
+                // e^{DIR 2 pi i k / 32}: cosine and sine of the first quadrant
+                const int q = k & 7;
+                const T c = c32[q], s = (T)(DIR < 0 ? -1 : 1) * c32[8 - q];
+                w = C{w.x * c - w.y * s, w.x * s + w.y * c};
+            }
+            if (k >= 8) w = rot_q<DIR>(w);
+            v[k] = cadd(e[k], w);
+            v[k + 16] = csub(e[k], w);
+        }
+    }
+}
+
+// Points per thread.  Up to N = 512 one lattice has too few sequences to fill the chip,
+// and 8 points with one more exchange beat 16 with half the waves (loaded column
+// pass, one lattice, FP64 / FP32 us: N = 256 6.7 / 6.2 against 8.1 / 7.2; N = 512 16.0 / 9.4
+// against 20.1 / 11.1; twelve lattices at once are within 8% either way).  From 1024
+// on 16 points need one exchange less; 8192 = 32 * 32 * 8 keeps three factors.
+template <int N>
+struct RegFft {
+    static constexpr int PT = N <= 512 ? 8 : (N <= 4096 ? 16 : 32);
+    static constexpr int N2 = N / PT;
+    static constexpr int N3 = N2 / PT;       // threads of a sub-sequence
+    static constexpr int T = N / PT;         // threads of a sequence
+    static constexpr int NU = PT / N3;
+    static_assert(N3 >= 1 && N3 <= PT && PT * PT * N3 == N, "register FFT split");
+};
+
+// frequency of v[q] in thread (g, m)
+template <int N>
+__device__ __forceinline__ int reg_freq(int g, int m, int q) {
+    typedef RegFft<N> F;
+    return g + F::PT * (m + F::N3 * (q / F::N3)) + F::PT * F::PT * (q % F::N3);
+}
+
+// v[k] *= w^k (DIR > 0: conjugate), k = 1 .. PT - 1, from the table entries
+// w, w^2, w^4 (w^8, w^16): at most three (four) products deep
+template <int PT, int DIR, typename C>
+__device__ __forceinline__ void twiddle_powers(C* v, const C* __restrict__ tw, int idx) {
+    C w[8];
+    w[1] = tw[idx];
+    w[2] = tw[2 * idx];
+    w[4] = tw[4 * idx];
+    C w8, w16;
+    if constexpr (PT >= 16) w8 = tw[8 * idx];
+    if constexpr (PT >= 32) w16 = tw[16 * idx];
+    if (DIR > 0) {
+        w[1].y = -w[1].y;
+        w[2].y = -w[2].y;
+        w[4].y = -w[4].y;
+        if constexpr (PT >= 16) w8.y = -w8.y;
+        if constexpr (PT >= 32) w16.y = -w16.y;
+    }
+    w[3] = cmul(w[1], w[2]);
+    w[5] = cmul(w[1], w[4]);
+    w[6] = cmul(w[2], w[4]);
+    w[7] = cmul(w[3], w[4]);
+#pragma unroll
+    for (int k = 1; k < 8; k++) v[k] = cmul(v[k], w[k]);
+    if constexpr (PT >= 16) {
+        v[8] = cmul(v[8], w8);
+#pragma unroll
+        for (int k = 1; k < 8; k++) v[8 + k] = cmul(v[8 + k], cmul(w8, w[k]));
+    }
+    if constexpr (PT >= 32) {
+        v[16] = cmul(v[16], w16);
+        const C w24 = cmul(w8, w16);
+        v[24] = cmul(v[24], w24);
+#pragma unroll
+        for (int k = 1; k < 8; k++) {
+            v[16 + k] = cmul(v[16 + k], cmul(w16, w[k]));
+            v[24 + k] = cmul(v[24 + k], cmul(w24, w[k]));
+        }
+    }
+}
+
+// LDS order inside a wave: the compiler keeps the accesses in program order;
+// a wave's own LDS operations complete in order
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// steps 1 to 5.  c: the thread's column, j: its index in the sequence.  FIRST: no
+// access of the buffer is pending (otherwise a barrier precedes the writes).
+template <int N, int W, bool FIRST, typename C>
+__device__ __forceinline__ void reg_fft_fwd(C* v, C* lds, const C* __restrict__ tw, int tid) {
+    const int j = tid / W, c = tid % W;
+    typedef RegFft<N> F;
+    constexpr int PT = F::PT, N2 = F::N2, N3 = F::N3, NU = F::NU;
+    static_assert(N3 * W <= 64, "a sub-sequence sits in one wave");
+    dft_reg<PT, -1>(v);
+    __builtin_amdgcn_sched_barrier(0);
+    twiddle_powers<PT, -1>(v, tw, j);
+    if (!FIRST) __syncthreads();
+    {
+        C* p = lds + j * W + c;
+#pragma unroll
+        for (int k = 0; k < PT; k++) p[k * N2 * W] = v[k];
+    }
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    const int g = j / N3, m = j % N3;
+    C* sub = lds + g * N2 * W + c;
+#pragma unroll
+    for (int a = 0; a < PT; a++) v[a] = sub[(m + N3 * a) * W];
+    dft_reg<PT, -1>(v);
+    if constexpr (N3 > 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        twiddle_powers<PT, -1>(v, tw, PT * m);
+        wave_lds_fence();
+#pragma unroll
+        for (int b = 0; b < PT; b++) sub[(b * N3 + (m ^ (b % N3))) * W] = v[b];
+        wave_lds_fence();
+#pragma unroll
+        for (int u = 0; u < NU; u++) {
+#pragma unroll
+            for (int q = 0; q < N3; q++) v[u * N3 + q] = sub[((m + N3 * u) * N3 + (q ^ m)) * W];
+            dft_reg<N3, -1>(v + u * N3);
+        }
+    }
+}
+
+// the steps backwards; v from reg_freq order to positions j + T r, unscaled
+template <int N, int W, bool FIRST, typename C>
+__device__ __forceinline__ void reg_fft_inv(C* v, C* lds, const C* __restrict__ tw, int tid) {
+    const int j = tid / W, c = tid % W;
+    typedef RegFft<N> F;
+    constexpr int PT = F::PT, N2 = F::N2, N3 = F::N3, NU = F::NU;
+    static_assert(N3 * W <= 64, "a sub-sequence sits in one wave");
+    const int g = j / N3, m = j % N3;
+    C* sub = lds + g * N2 * W + c;
+    if (!FIRST) __syncthreads();
+    if constexpr (N3 > 1) {
+#pragma unroll
+        for (int u = 0; u < NU; u++) {
+            dft_reg<N3, +1>(v + u * N3);
+#pragma unroll
+            for (int q = 0; q < N3; q++) sub[((m + N3 * u) * N3 + (q ^ m)) * W] = v[u * N3 + q];
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int b = 0; b < PT; b++) v[b] = sub[(b * N3 + (m ^ (b % N3))) * W];
+        twiddle_powers<PT, +1>(v, tw, PT * m);
+        wave_lds_fence();
+    }
+    dft_reg<PT, +1>(v);
+#pragma unroll
+    for (int a = 0; a < PT; a++) sub[(m + N3 * a) * W] = v[a];
+    __syncthreads();
+    {
+        const C* p = lds + j * W + c;
+#pragma unroll
+        for (int k = 0; k < PT; k++) v[k] = p[k * N2 * W];
+    }
+    twiddle_powers<PT, +1>(v, tw, j);
+    dft_reg<PT, +1>(v);
+}
+
+}  // namespace jw
