@@ -1423,8 +1423,9 @@ static hipError_t step_fused_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     return hipSuccess;
 }
 
+// instantiated once per size and type (jw_step_n.hip)
 template <int N, typename C>
-static hipError_t step_fused_layout(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, const StepArgs& a,
+hipError_t step_fused_layout(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, const StepArgs& a,
                                     const int* kcls) {
     switch (c->layout) {
         case 0: return step_fused_n<N, 0>(c, U, Xi, Vv, ZA, ZB, a, kcls);
@@ -1436,6 +1437,14 @@ static hipError_t step_fused_layout(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB,
         default: return hipErrorInvalidValue;
     }
 }
+
+#define JW_FUSED_SIZES(M, C) M(64, C) M(128, C) M(256, C) M(512, C) M(1024, C) M(2048, C)
+#define JW_FUSED_EXTERN(n, C) \
+    extern template hipError_t step_fused_layout<n, C>(jw_ctx*, C*, C*, C*, C*, C*, const StepArgs&, const int*);
+#ifndef JW_STEP_N
+JW_FUSED_SIZES(JW_FUSED_EXTERN, cplx)
+JW_FUSED_SIZES(JW_FUSED_EXTERN, cplxf)
+#endif
 
 template <typename C>
 static hipError_t step_fused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, const StepArgs& a) {
