@@ -290,19 +290,111 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
     }
 }
 
+// Box-Muller in FP64.  The normals are bound by instructions (the noise pass runs
+// far below the memory rate), so the three functions are written for the
+// arguments that occur: u in (0, 1] and never subnormal, the angle as an integer
+// fraction of a turn.  Against the library's log, sqrt and sincospi, which
+// also take subnormals, infinities and arguments beyond one turn: about 70
+// instead of 130 FP64 instructions per pair.
+
+// log u for a normal u in (0, 1]: u = 2^e m, m in [sqrt(1/2), sqrt 2);
+// log m = 2 atanh(s), s = f / (2 + f), f = m - 1, as (f - f^2/2) + s (f^2/2 + R),
+// R = s^2 P(s^2) with P fitted (relative error 9e-18 of log m)
+__device__ __forceinline__ double log_unit(double u) {
+    uint32_t hi = (uint32_t)__double2hiint(u) + (0x3ff00000u - 0x3fe6a09eu);
+    const int e = (int)(hi >> 20) - 0x3ff;
+    hi = (hi & 0xfffffu) + 0x3fe6a09eu;
+    const double f = __hiloint2double((int)hi, __double2loint(u)) - 1.0;
+    const double d = 2.0 + f;
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(fma(-d, r, 1.0), r, r);
+    r = fma(fma(-d, r, 1.0), r, r);
+    double s = f * r;
+    s = fma(fma(-d, s, f), r, s);
+    const double z = s * s;
+    double p = 0.14617867730858242049;
+    p = fma(p, z, 0.15331597373668940049);
+    p = fma(p, z, 0.18182893205969450976);
+    p = fma(p, z, 0.22222211073019649875);
+    p = fma(p, z, 0.28571428626398112419);
+    p = fma(p, z, 0.39999999999898447552);
+    p = fma(p, z, 0.66666666666666697289);
+    const double h = 0.5 * f * f, k = (double)e;
+    const double fh = f - h, fl = (f - fh) - h;        // f - h, exactly
+    // ln 2 in two parts, the first with 20 trailing zero bits: k ln2_hi is exact
+    const double t = fma(s, fma(z, p, h), k * 7.4406171100123967161e-11);
+    return fma(k, 0x1.62e42fef00000p-1, fh + (fl + t));
+}
+
+// sqrt x, x >= 0 and not subnormal
+__device__ __forceinline__ double sqrt_pos(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    return x > 0.0 ? g : 0.0;
+}
+
+// rr (cos, sin) of (q + r) quarter turns, |r| <= 1/2: polynomials in r^2 fitted
+// to sin and cos of r pi/2 (relative errors 1.3e-17 and 1.2e-19)
+__device__ __forceinline__ void polar_quarter(double rr, uint32_t q, double r, double& z0, double& z1) {
+    const double z = r * r;
+    double ps = 5.6422280858396281912e-8;
+    ps = fma(ps, z, -3.5987029691976957449e-6);
+    ps = fma(ps, z, 0.00016044116661835320727);
+    ps = fma(ps, z, -0.0046817541342546123106);
+    ps = fma(ps, z, 0.079692626246144251951);
+    ps = fma(ps, z, -0.64596409750624617454);
+    // pi / 2 in two parts
+    const double sn = fma(r, 1.5707963267948966, r * fma(ps, z, 6.1232339957367658861e-17));
+    double pc = -6.329398172958278693e-9;
+    pc = fma(pc, z, 4.710678420640450103e-7);
+    pc = fma(pc, z, -0.000025202039028494948697);
+    pc = fma(pc, z, 0.00091926027454691019546);
+    pc = fma(pc, z, -0.020863480763340776668);
+    pc = fma(pc, z, 0.25366950790104782331);
+    // 1 + z (a + z pc), 1 + a z with its rounding error; a in two parts
+    const double a = -1.2337005501361698, ch = fma(a, z, 1.0);
+    const double cs = ch + fma(z, fma(pc, z, -7.78619e-17), fma(a, z, 1.0 - ch));
+    const double co = (q & 1u) ? sn : cs, si = (q & 1u) ? cs : sn;
+    // signs: cosine negative in quarters 1 and 2, sine in 2 and 3
+    const double rc = __hiloint2double(__double2hiint(rr) ^ (int)(((q + 1u) & 2u) << 30), __double2loint(rr));
+    const double rs = __hiloint2double(__double2hiint(rr) ^ (int)((q & 2u) << 30), __double2loint(rr));
+    z0 = rc * co;
+    z1 = rs * si;
+}
+
 __device__ __forceinline__ void box_muller_pair(uint32_t site, uint32_t step, uint32_t tag, uint32_t call,
                                                 uint32_t seed, uint32_t traj, double& z0, double& z1) {
     uint32_t c[4] = {site, step, tag, call};
     philox4x32_10(c, seed, traj);
-    const uint64_t a = ((uint64_t)c[0] << 32) | c[1];
-    const uint64_t b = ((uint64_t)c[2] << 32) | c[3];
-    const double u0 = ((double)(a >> 11) + 0.5) * 0x1.0p-53;
-    const double u1 = ((double)(b >> 11) + 0.5) * 0x1.0p-53;
-    const double rr = sqrt(-2.0 * log(u0));
-    double s, co;
-    sincospi(2.0 * u1, &s, &co);
-    z0 = rr * co;
-    z1 = rr * s;
+    // u0 = (a + 1/2) 2^-53 with a the upper 53 bits of (c0, c1), rounded once
+    const double u0 = fma((double)c[0], 0x1.0p-32, fma((double)(c[1] >> 11), 0x1.0p-53, 0x1.0p-54));
+    const double rr = sqrt_pos(-2.0 * log_unit(u0));
+    // u1 likewise from (c2, c3); in quarter turns 4 u1 = q + r, q to nearest
+    const uint32_t q = (c[2] + 0x20000000u) >> 30;
+    const double r = fma((double)(int32_t)(c[2] - (q << 30)), 0x1.0p-30,
+                         fma((double)(c[3] >> 11), 0x1.0p-51, 0x1.0p-52));
+    polar_quarter(rr, q, r, z0, z1);
+}
+
+// sqrt(-2 log u) in FP32 from w = u (lo: u < 1/2) or w = 1 - u.  One logarithm for
+// both: u < 1/2 takes log u; above, with a = 1 - w rounded (1 - a exact),
+// log1p(-w) = log(a) w / (1 - a) (Goldberg's log1p), or -w when a = 1.  Neither a
+// nor the logarithm is subnormal, zero or infinite here, so the hardware's log2 is
+// scaled by ln 2 (in two parts, as one rounding) and its reciprocal square root
+// refined once, without the library's handling of those.
+__device__ __forceinline__ float radius_f(bool lo, float w) {
+    const float a = lo ? w : 1.0f - w;
+    const float l2 = __builtin_amdgcn_logf(a);
+    const float t = l2 * 0x1.62e42ep-1f;
+    float lu = t + fmaf(l2, 0x1.efa39ep-25f, fmaf(l2, 0x1.62e42ep-1f, -t));
+    if (!lo) lu = a == 1.0f ? -w : lu * (w * __builtin_amdgcn_rcpf(1.0f - a));
+    const float x = -2.0f * lu;
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y;
+    return fmaf(fmaf(-g, g, x), 0.5f * y, g);
 }
 
 // The same pair in FP32 from the same Philox words (mixed-precision form):
@@ -315,24 +407,20 @@ __device__ __forceinline__ void box_muller_pair_f(uint32_t site, uint32_t step, 
                                                   uint32_t seed, uint32_t traj, float& z0, float& z1) {
     uint32_t c[4] = {site, step, tag, call};
     philox4x32_10(c, seed, traj);
-    const uint64_t m0 = (((uint64_t)c[0] << 32) | c[1]) >> 11;     // u0 = (m0 + 1/2) 2^-53
-    const uint64_t m1 = (((uint64_t)c[2] << 32) | c[3]) >> 11;     // u1 = (m1 + 1/2) 2^-53
-    // 53-bit integers to FP32 through FP64 (exact there, then one rounding: the
-    // same value as a direct conversion, in fewer instructions)
-    // One logarithm for both halves: u0 < 1/2 takes log u0; above, with
-    // t = 1 - u0 from the integer and a = 1 - t rounded (1 - a exact),
-    // log1p(-t) = log(a) t / (1 - a) (Goldberg's log1p), or -t when a = 1.
-    const bool lo = m0 < (1ull << 52);
-    const float t = ((float)(double)((1ull << 53) - 1 - m0) + 0.5f) * 0x1.0p-53f;
-    const float a = lo ? ((float)(double)m0 + 0.5f) * 0x1.0p-53f : 1.0f - t;
-    float lu = logf(a);
-    if (!lo) lu = a == 1.0f ? -t : lu * (t * __builtin_amdgcn_rcpf(1.0f - a));
-    const float rr = sqrtf(-2.0f * lu);
-    const int64_t d = 2 * (int64_t)m1 + 1 - (1ll << 53);            // x = d 2^-53
-    // sin and cos of pi x on the hardware's revolution-based units (x / 2
-    // revolutions, in (-1/2, 1/2)): within 1.9e-7 of FP64 sincospi on all inputs,
-    // against 1.2e-7 for the library's sincospif, in far fewer instructions
-    const float rev = (float)(double)d * 0x1.0p-54f;
+    // u0 = (m0 + 1/2) 2^-53 and u1 = (m1 + 1/2) 2^-53, m the upper 53 bits of a
+    // word pair.  53-bit integers to FP32 through FP64 (exact there, then one
+    // rounding: the same value as a direct conversion, in fewer instructions).
+    // u0 < 1/2 takes m0, u0 >= 1/2 takes 2^53 - 1 - m0 (the complement of the bits).
+    const bool lo = !(c[0] >> 31);
+    const uint32_t h0 = lo ? c[0] : ~c[0], l0 = (lo ? c[1] : ~c[1]) >> 11;
+    const float w = ((float)fma((double)h0, 0x1.0p21, (double)l0) + 0.5f) * 0x1.0p-53f;
+    const float rr = radius_f(lo, w);
+    // x / 2 revolutions in (-1/2, 1/2), x = 2 u1 - 1 = (2 m1 + 1 - 2^53) 2^-53, on
+    // the hardware's revolution-based sine and cosine units: within 1.9e-7 of FP64
+    // sincospi on all inputs, against 1.2e-7 for the library's sincospif, in
+    // far fewer instructions
+    const float rev = (float)fma((double)(int32_t)(c[2] ^ 0x80000000u), 0x1.0p22,
+                                 (double)(int32_t)((c[3] >> 11) * 2u + 1u)) * 0x1.0p-54f;
     z0 = -rr * __builtin_amdgcn_cosf(rev);
     z1 = -rr * __builtin_amdgcn_sinf(rev);
 }
@@ -349,26 +437,18 @@ __device__ __forceinline__ void box_muller_pair_f(uint32_t site, uint32_t step, 
 // and y-direction plane pairs p.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void box_muller32(uint32_t w0, uint32_t w1, double& z0, double& z1) {
-    const double u0 = ((double)w0 + 0.5) * 0x1.0p-32;
-    const double u1 = ((double)w1 + 0.5) * 0x1.0p-32;
-    const double rr = sqrt(-2.0 * log(u0));
-    double s, co;
-    sincospi(2.0 * u1, &s, &co);
-    z0 = rr * co;
-    z1 = rr * s;
+    const double rr = sqrt_pos(-2.0 * log_unit(fma((double)w0, 0x1.0p-32, 0x1.0p-33)));
+    const uint32_t q = (w1 + 0x20000000u) >> 30;
+    polar_quarter(rr, q, fma((double)(int32_t)(w1 - (q << 30)), 0x1.0p-30, 0x1.0p-31), z0, z1);
 }
 // FP32 from the same words, as box_muller_pair_f: log u0 below 1/2, above it
-// log1p(-t) with t = 1 - u0 taken from the integer; the angle pi x with
+// log1p(-w) with w = 1 - u0 taken from the integer; the angle pi x with
 // x = 2 u1 - 1 in (-1, 1)
 __device__ __forceinline__ void box_muller32(uint32_t w0, uint32_t w1, float& z0, float& z1) {
-    const bool lo = w0 < 0x80000000u;
-    const float t = (float)((double)(0xFFFFFFFFu - w0) + 0.5) * 0x1.0p-32f;
-    const float a = lo ? (float)((double)w0 + 0.5) * 0x1.0p-32f : 1.0f - t;
-    float lu = logf(a);
-    if (!lo) lu = a == 1.0f ? -t : lu * (t * __builtin_amdgcn_rcpf(1.0f - a));
-    const float rr = sqrtf(-2.0f * lu);
-    const int64_t d = 2 * (int64_t)w1 + 1 - (1ll << 32);            // x = d 2^-32
-    const float rev = (float)(double)d * 0x1.0p-33f;                 // x / 2 revolutions, as above
+    const bool lo = !(w0 >> 31);
+    const float w = (float)((double)(lo ? w0 : ~w0) + 0.5) * 0x1.0p-32f;
+    const float rr = radius_f(lo, w);
+    const float rev = (float)((double)(int32_t)(w1 ^ 0x80000000u) + 0.5) * 0x1.0p-32f;   // x / 2 revolutions
     z0 = -rr * __builtin_amdgcn_cosf(rev);
     z1 = -rr * __builtin_amdgcn_sinf(rev);
 }
