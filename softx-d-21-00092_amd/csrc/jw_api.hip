@@ -81,6 +81,16 @@ int ensure_sa16(jw_ctx* c) {
     return JW_OK;
 }
 
+// the current sa table in the column order of the row-major row spectra
+int ensure_sap(jw_ctx* c) {
+    if (!c->sap && hipMalloc(&c->sap, c->V * sizeof(double)) != hipSuccess)
+        return fail(JW_ERR_ALLOC, "coupling table allocation failed");
+    if (c->sap_gen == c->sa_gen) return JW_OK;
+    HIP_CHECK(jw::perm_columns(c, c->sap, c->sa));
+    c->sap_gen = c->sa_gen;
+    return JW_OK;
+}
+
 // noise source for the next generator call; advances the Philox step afterwards
 jw::NoiseSrc take_noise(jw_ctx* c, int per_site, uint32_t tag, bool* ok) {
     jw::NoiseSrc ns{nullptr, c->seed, c->traj, c->step, tag};
@@ -117,6 +127,22 @@ int check_field(const jw_field* f, const jw_ctx* c, int t, const char* name) {
 
 // the column passes of layouts 1, 4 and 8 read the 16-row-blocked sqrt(alpha) table
 bool uses_sa16(int layout) { return layout == 1 || layout == 4 || layout == 8 || layout >= 16; }
+// and the register-held column pass of the row-major fused step the one in its
+// column order (the matrix-core stages read the plain table)
+bool uses_sap(const jw_ctx* c, bool fused, bool mfma) { return fused && c->layout == 0 && !mfma; }
+
+// sqrt(alpha) in k for the fused or large-lattice passes of c->layout (ensure_sa done)
+int k_table(jw_ctx* c, bool fused, bool mfma, const double** sa_k) {
+    *sa_k = c->sa;
+    if (uses_sa16(c->layout)) {
+        if (int e = ensure_sa16(c)) return e;
+        *sa_k = c->sa16;
+    } else if (uses_sap(c, fused, mfma)) {
+        if (int e = ensure_sap(c)) return e;
+        *sa_k = c->sap;
+    }
+    return JW_OK;
+}
 
 // the intermediate layout when none is selected: row-major planes, whose column pass holds its strip in registers; 16-byte strips
 // one plane at a time for FP64 at N = 8192 (two planes of one column take the
@@ -152,8 +178,8 @@ int evolve_generator_basis(jw_ctx* c, jw_field* U, int nsteps, bool fused, bool 
 // The generator-basis evolution of jw_evolve for the SIN kernel on the 24
 // intermediate planes at Xi (xi 8, V 8, A 4, B 4).  tabs == nullptr: the
 // context's cached coupling tables (allocated on first use); otherwise two
-// V-double arrays into which this call builds sqrt(alpha) and, for the blocked
-// layouts, its 16-row-blocked copy (nothing allocated).
+// V-double arrays into which this call builds sqrt(alpha) and its copy in the
+// order of the layout's column pass (nothing allocated).
 int evolve_sin(jw_ctx* c, jw_field* U, int coupling, double step, const jw_alpha* a, int nsteps, cplx* Xi,
                double* tabs) {
     const size_t V = c->V;
@@ -186,20 +212,18 @@ int evolve_sin(jw_ctx* c, jw_field* U, int coupling, double step, const jw_alpha
     if (int e = check_kspace(c, coupling, fused || large)) return e;
     const int saved_layout = c->layout;
     if (c->layout < 0) c->layout = default_layout(c->N, 0, c->fft_mfma);
-    if ((fused || large) && sa_k && uses_sa16(c->layout)) {
-        if (tabs) {
-            const hipError_t he = jw::block16(c, tabs + V, tabs);
-            if (he != hipSuccess) {
-                c->layout = saved_layout;
-                return fail(JW_ERR_HIP, "coupling table: %s", hipGetErrorString(he));
-            }
+    if ((fused || large) && sa_k) {
+        int rc = JW_OK;
+        if (!tabs) {
+            rc = k_table(c, fused, false, &sa_k);
+        } else if (uses_sa16(c->layout) || uses_sap(c, fused, false)) {
+            const hipError_t he = uses_sa16(c->layout) ? jw::block16(c, tabs + V, tabs) : jw::perm_columns(c, tabs + V, tabs);
+            if (he != hipSuccess) rc = fail(JW_ERR_HIP, "coupling table: %s", hipGetErrorString(he));
             sa_k = tabs + V;
-        } else {
-            if (int e = ensure_sa16(c)) {
-                c->layout = saved_layout;
-                return e;
-            }
-            sa_k = c->sa16;
+        }
+        if (rc) {
+            c->layout = saved_layout;
+            return rc;
         }
     }
     const int rc = evolve_generator_basis(c, U, nsteps, fused, large, Xi, Vv, ZA, ZB, sa_pos, sa_k, kc, corr, s, ss);
@@ -333,12 +357,7 @@ int batch_tables(BatchGroup& g, int coupling, const jw::Alpha& al, const double*
         *sa_pos = c->sa;
     } else if (coupling == JW_SQRT_COUPLING_CONSTANT || coupling == JW_CORRELATED_NOISE_COUPLING) {
         if (int e = ensure_sa(c, 0, al)) return e;
-        if (uses_sa16(c->layout)) {
-            if (int e = ensure_sa16(c)) return e;
-            *sa_k = c->sa16;
-        } else {
-            *sa_k = c->sa;
-        }
+        if (int e = k_table(c, true, c->fft_mfma != 0, sa_k)) return e;
     }
     return JW_OK;
 }
@@ -442,8 +461,16 @@ int batch_tune_launch(jw_batch* b, int coupling, double step, const jw::Alpha& a
     b->traj0 = 0xFFFFF000u;      // scratch noise key
     float ms[2] = {1e30f, 1e30f};
     for (int mode = 0; mode < 2 && rc == JW_OK; mode++) {
-        if (mode == 1) batch_rowmajor(b);
-        bool ok = batch_step_all(b, coupling, step, al, 0, 1, 0, uc.data(), false, mode) == JW_OK;
+        bool ok = true;
+        if (mode == 1) {
+            // the row-major tables are built on the groups' streams; the one launch runs on b->stream
+            batch_rowmajor(b);
+            for (auto& g : b->g) {
+                const double *p, *k;
+                ok = ok && batch_tables(g, coupling, al, &p, &k) == JW_OK && hipStreamSynchronize(g.ctx->stream) == hipSuccess;
+            }
+        }
+        ok = ok && batch_step_all(b, coupling, step, al, 0, 1, 0, uc.data(), false, mode) == JW_OK;
         ok = ok && hipEventRecord(e0, b->stream) == hipSuccess;
         for (int it = 0; it < 3 && ok; it++) ok = batch_step_all(b, coupling, step, al, 0, 1, 0, uc.data(), false, mode) == JW_OK;
         ok = ok && hipEventRecord(e1, b->stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
@@ -604,6 +631,7 @@ void jw_destroy(jw_ctx* c) {
     if (c->sb) hipFree(c->sb);
     if (c->sa) hipFree(c->sa);
     if (c->sa16) hipFree(c->sa16);
+    if (c->sap) hipFree(c->sap);
     if (c->inj) hipFree(c->inj);
     if (c->ws) hipFree(c->ws);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -1068,10 +1096,7 @@ int jw_evolve_mixed(jw_ctx* c, jw_field* U, int coupling, int kernel, double ste
     const int saved_layout = c->layout;
     if (c->layout < 0) c->layout = default_layout(c->N, 1, c->fft_mfma);
     int rc = JW_OK;
-    if ((fused || large) && sa_k && uses_sa16(c->layout)) {
-        rc = ensure_sa16(c);
-        sa_k = c->sa16;
-    }
+    if ((fused || large) && sa_k) rc = k_table(c, fused, c->fft_mfma != 0, &sa_k);
     // the fused and large-lattice passes hold rows 0 and 1 of U (row 2 rebuilt),
     // the unfused sequence all nine entries
     const int uplanes = fused || large ? 6 : 9;

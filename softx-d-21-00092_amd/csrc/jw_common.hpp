@@ -156,6 +156,7 @@ __device__ __forceinline__ void store9(cplx* __restrict__ f, size_t V, size_t i,
 // form), or m3f with S = float (the mixed form's products).
 template <typename M, typename S>
 __device__ __forceinline__ void uxiu_gen(const M& u, const S h[8], S out[8]) {
+#pragma clang fp contract(off)
     typedef decltype(u.m[0]) CR;
     typedef typename std::remove_const<typename std::remove_reference<CR>::type>::type Cx;
     const S d8 = h[7] * (S)JW_INV_SQRT3;
@@ -167,14 +168,14 @@ __device__ __forceinline__ void uxiu_gen(const M& u, const S h[8], S out[8]) {
     for (int r = 0; r < 3; r++) {
         const Cx a = u.m[3 * r], b = u.m[3 * r + 1], c = u.m[3 * r + 2];
         // row r of U X, X Hermitian: X10 = conj(x01), X20 = conj(x02), X21 = conj(x12)
-        const Cx w0 = cadd(cadd(cscale(a, x00), cmulc(b, x01)), cmulc(c, x02));
-        const Cx w1 = cadd(cadd(cmul(a, x01), cscale(b, x11)), cmulc(c, x12));
-        const Cx w2 = cadd(cadd(cmul(a, x02), cmul(b, x12)), cscale(c, x22));
+        const Cx w0 = cmadc(cmadc(cscale(a, x00), b, x01), c, x02);
+        const Cx w1 = cmadc(cmads(cmul(a, x01), b, x11), c, x12);
+        const Cx w2 = cmads(cmad(cmul(a, x02), b, x12), c, x22);
 #pragma unroll
         for (int cc = r; cc < 3; cc++) {
             Cx s = cmulc(w0, u.m[3 * cc]);
-            s = cadd(s, cmulc(w1, u.m[3 * cc + 1]));
-            s = cadd(s, cmulc(w2, u.m[3 * cc + 2]));
+            s = cmadc(s, w1, u.m[3 * cc + 1]);
+            s = cmadc(s, w2, u.m[3 * cc + 2]);
             if (cc == r) d[r] = s.x;
             else up[r + cc - 1] = s;
         }

@@ -14,11 +14,20 @@ namespace jw {
 // ---------------------------------------------------------------------------
 typedef double2 cplx;
 
+// Products are written with their fused multiply-adds spelled out, and the functions
+// made of them form no others: a kernel body gives the same bits whichever kernel
+// inlines it (a batch's trajectories against a single lattice's).
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return fma(a, b, c); }
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ cplx mk(double r, double i) { return make_double2(r, i); }
 __device__ __forceinline__ cplx cadd(cplx a, cplx b) { return mk(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ cplx csub(cplx a, cplx b) { return mk(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ cplx cmul(cplx a, cplx b) { return mk(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
-__device__ __forceinline__ cplx cmulc(cplx a, cplx b) { return mk(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y); }  // a*conj(b)
+__device__ __forceinline__ cplx cmul(cplx a, cplx b) {
+    return mk(fma_t(a.x, b.x, -(a.y * b.y)), fma_t(a.x, b.y, a.y * b.x));
+}
+__device__ __forceinline__ cplx cmulc(cplx a, cplx b) {      // a*conj(b)
+    return mk(fma_t(a.x, b.x, a.y * b.y), fma_t(a.y, b.x, -(a.x * b.y)));
+}
 __device__ __forceinline__ cplx conjg(cplx a) { return mk(a.x, -a.y); }
 __device__ __forceinline__ cplx cscale(cplx a, double s) { return mk(a.x * s, a.y * s); }
 __device__ __forceinline__ cplx cmuli(cplx a) { return mk(-a.y, a.x); }       // i*a
@@ -33,11 +42,28 @@ typedef float2 cplxf;
 __device__ __forceinline__ cplxf mkf(float r, float i) { return make_float2(r, i); }
 __device__ __forceinline__ cplxf cadd(cplxf a, cplxf b) { return mkf(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ cplxf csub(cplxf a, cplxf b) { return mkf(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ cplxf cmul(cplxf a, cplxf b) { return mkf(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+__device__ __forceinline__ cplxf cmul(cplxf a, cplxf b) {
+    return mkf(fma_t(a.x, b.x, -(a.y * b.y)), fma_t(a.x, b.y, a.y * b.x));
+}
+__device__ __forceinline__ cplxf cmulc(cplxf a, cplxf b) {
+    return mkf(fma_t(a.x, b.x, a.y * b.y), fma_t(a.y, b.x, -(a.x * b.y)));
+}
 __device__ __forceinline__ cplxf cscale(cplxf a, float s) { return mkf(a.x * s, a.y * s); }
 __device__ __forceinline__ cplxf cmuli(cplxf a) { return mkf(-a.y, a.x); }
 __device__ __forceinline__ cplxf cmulmi(cplxf a) { return mkf(a.y, -a.x); }
-__device__ __forceinline__ cplxf cmulc(cplxf a, cplxf b) { return mkf(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y); }
+// s + a b, s + a conj(b), s + a r (r real)
+template <typename C>
+__device__ __forceinline__ C cmad(C s, C a, C b) {
+    return C{fma_t(a.x, b.x, fma_t(-a.y, b.y, s.x)), fma_t(a.x, b.y, fma_t(a.y, b.x, s.y))};
+}
+template <typename C>
+__device__ __forceinline__ C cmadc(C s, C a, C b) {
+    return C{fma_t(a.x, b.x, fma_t(a.y, b.y, s.x)), fma_t(a.y, b.x, fma_t(-a.x, b.y, s.y))};
+}
+template <typename C, typename T>
+__device__ __forceinline__ C cmads(C s, C a, T r) {
+    return C{fma_t(a.x, r, s.x), fma_t(a.y, r, s.y)};
+}
 __device__ __forceinline__ cplxf conjg(cplxf a) { return mkf(a.x, -a.y); }
 
 // complex value of type C (double2 or float2) from two doubles, and back
@@ -61,8 +87,8 @@ __device__ __forceinline__ m3 mmul(const m3& a, const m3& b) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             cplx s = cmul(a.m[3 * i], b.m[j]);
-            s = cadd(s, cmul(a.m[3 * i + 1], b.m[3 + j]));
-            s = cadd(s, cmul(a.m[3 * i + 2], b.m[6 + j]));
+            s = cmad(s, a.m[3 * i + 1], b.m[3 + j]);
+            s = cmad(s, a.m[3 * i + 2], b.m[6 + j]);
             c.m[3 * i + j] = s;
         }
     return c;
@@ -79,8 +105,8 @@ __device__ __forceinline__ m3f mmul(const m3f& a, const m3f& b) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             cplxf s = cmul(a.m[3 * i], b.m[j]);
-            s = cadd(s, cmul(a.m[3 * i + 1], b.m[3 + j]));
-            s = cadd(s, cmul(a.m[3 * i + 2], b.m[6 + j]));
+            s = cmad(s, a.m[3 * i + 1], b.m[3 + j]);
+            s = cmad(s, a.m[3 * i + 2], b.m[6 + j]);
             c.m[3 * i + j] = s;
         }
     return c;
@@ -109,6 +135,7 @@ __device__ __forceinline__ m3 to_d(const m3f& a) {
 
 // Hermitian traceless matrix s*H(h)
 __device__ __forceinline__ m3 herm_from_gen(const double h[8], double s) {
+#pragma clang fp contract(off)
     m3 X;
     const double d8 = h[7] * JW_INV_SQRT3;
     X.m[0] = mk(s * (h[2] + d8), 0.0);
@@ -153,9 +180,10 @@ __device__ __forceinline__ void gen_from_upper(const m3& M, double h[8]) {
 __device__ __forceinline__ m3 su3_project(const m3& M);
 
 __device__ __forceinline__ m3 exp_i_gen(const double h[8], double s) {
+#pragma clang fp contract(off)
     double c1 = 0.0;
 #pragma unroll
-    for (int a = 0; a < 8; a++) c1 += h[a] * h[a];
+    for (int a = 0; a < 8; a++) c1 = fma(h[a], h[a], c1);
     c1 *= s * s;
     m3 E;
     if (!(c1 > 0.0)) {   // X == 0 (or NaN input: propagate it)
@@ -172,16 +200,18 @@ __device__ __forceinline__ m3 exp_i_gen(const double h[8], double s) {
     const double d0 = X.m[0].x, d1 = X.m[4].x, d2 = X.m[8].x;
     const cplx x = X.m[1], y = X.m[2], z = X.m[5];
     const cplx xz = cmul(x, z);
-    const double c0 = d0 * d1 * d2 + 2.0 * (xz.x * y.x + xz.y * y.y)
-                      - d0 * (z.x * z.x + z.y * z.y) - d1 * (y.x * y.x + y.y * y.y)
-                      - d2 * (x.x * x.x + x.y * x.y);
+    const double ax = fma(x.x, x.x, x.y * x.y), ay = fma(y.x, y.x, y.y * y.y), az = fma(z.x, z.x, z.y * z.y);
+    double c0 = fma(d0 * d1, d2, 2.0 * fma(xz.x, y.x, xz.y * y.y));
+    c0 = fma(-d0, az, c0);
+    c0 = fma(-d1, ay, c0);
+    c0 = fma(-d2, ax, c0);
     // scaled coefficients A = a_n/n!, B = b_n/n!, D = d_n/n!; n = 0
     double A = 1.0, B = 0.0, D = 0.0;
     double f0r = 1.0, f0i = 0.0, f1r = 0.0, f1i = 0.0, f2r = 0.0, f2i = 0.0;
 #pragma unroll
     for (int n = 1; n <= JW_EXP_SERIES_TERMS; n++) {
         const double inv = 1.0 / n;
-        const double An = c0 * D * inv, Bn = (A + c1 * D) * inv, Dn = B * inv;
+        const double An = c0 * D * inv, Bn = fma(c1, D, A) * inv, Dn = B * inv;
         A = An; B = Bn; D = Dn;
         // i^n: n%4 = 0 -> +1, 1 -> +i, 2 -> -1, 3 -> -i
         if ((n & 3) == 0) { f0r += A; f1r += B; f2r += D; }
@@ -195,7 +225,7 @@ __device__ __forceinline__ m3 exp_i_gen(const double h[8], double s) {
     const cplx f0 = mk(f0r, f0i), f1 = mk(f1r, f1i), f2 = mk(f2r, f2i);
     const m3 X2 = mmul(X, X);
 #pragma unroll
-    for (int q = 0; q < 9; q++) E.m[q] = cadd(cmul(f1, X.m[q]), cmul(f2, X2.m[q]));
+    for (int q = 0; q < 9; q++) E.m[q] = cmad(cmul(f1, X.m[q]), f2, X2.m[q]);
     E.m[0] = cadd(E.m[0], f0);
     E.m[4] = cadd(E.m[4], f0);
     E.m[8] = cadd(E.m[8], f0);
@@ -213,9 +243,10 @@ __device__ __forceinline__ m3 exp_i_gen(const double h[8], double s) {
 // Fewer live registers than the FP64 matrices of exp_i_gen.
 template <typename H>
 __device__ __forceinline__ m3f exp_i_gen_f(const H h[8], double s) {
+#pragma clang fp contract(off)
     double c1 = 0.0;
 #pragma unroll
-    for (int a = 0; a < 8; a++) c1 += (double)h[a] * (double)h[a];
+    for (int a = 0; a < 8; a++) c1 = fma((double)h[a], (double)h[a], c1);
     c1 *= s * s;
     m3f E;
     if (!(c1 > 0.0)) {
@@ -232,15 +263,18 @@ __device__ __forceinline__ m3f exp_i_gen_f(const H h[8], double s) {
     const double d0 = sk * ((double)h[2] + d8), d1 = sk * (-(double)h[2] + d8), d2 = sk * (-2.0 * d8);
     const cplx x = mk(sk * (double)h[0], sk * (double)h[1]), y = mk(sk * (double)h[3], sk * (double)h[4]),
                z = mk(sk * (double)h[5], sk * (double)h[6]);
-    const double ax = x.x * x.x + x.y * x.y, ay = y.x * y.x + y.y * y.y, az = z.x * z.x + z.y * z.y;
+    const double ax = fma(x.x, x.x, x.y * x.y), ay = fma(y.x, y.x, y.y * y.y), az = fma(z.x, z.x, z.y * z.y);
     const cplx xz = cmul(x, z);
-    const double c0 = d0 * d1 * d2 + 2.0 * (xz.x * y.x + xz.y * y.y) - d0 * az - d1 * ay - d2 * ax;
+    double c0 = fma(d0 * d1, d2, 2.0 * fma(xz.x, y.x, xz.y * y.y));
+    c0 = fma(-d0, az, c0);
+    c0 = fma(-d1, ay, c0);
+    c0 = fma(-d2, ax, c0);
     double A = 1.0, B = 0.0, D = 0.0;
     double f0r = 1.0, f0i = 0.0, f1r = 0.0, f1i = 0.0, f2r = 0.0, f2i = 0.0;
 #pragma unroll
     for (int n = 1; n <= JW_EXP_SERIES_TERMS; n++) {
         const double inv = 1.0 / n;
-        const double An = c0 * D * inv, Bn = (A + c1 * D) * inv, Dn = B * inv;
+        const double An = c0 * D * inv, Bn = fma(c1, D, A) * inv, Dn = B * inv;
         A = An; B = Bn; D = Dn;
         if ((n & 3) == 0) { f0r += A; f1r += B; f2r += D; }
         else if ((n & 3) == 1) { f0i += A; f1i += B; f2i += D; }
@@ -251,17 +285,17 @@ __device__ __forceinline__ m3f exp_i_gen_f(const H h[8], double s) {
     }
     const cplx f1 = mk(f1r, f1i), f2 = mk(f2r, f2i);
     // X^2: real diagonal and upper triangle
-    const double q0 = d0 * d0 + ax + ay, q1 = ax + d1 * d1 + az, q2 = ay + az + d2 * d2;
-    const cplx q01 = cadd(cscale(x, d0 + d1), cmulc(y, z));      // x (d0 + d1) + y z*
-    const cplx q02 = cadd(cscale(y, d0 + d2), xz);               // y (d0 + d2) + x z
-    const cplx q12 = cadd(cmulc(y, x), cscale(z, d1 + d2));      // x* y + z (d1 + d2)
+    const double q0 = fma(d0, d0, ax) + ay, q1 = fma(d1, d1, ax) + az, q2 = fma(d2, d2, ay + az);
+    const cplx q01 = cmads(cmulc(y, z), x, d0 + d1);             // x (d0 + d1) + y z*
+    const cplx q02 = cmads(xz, y, d0 + d2);                      // y (d0 + d2) + x z
+    const cplx q12 = cmads(cmulc(y, x), z, d1 + d2);             // x* y + z (d1 + d2)
     // E = f0 + f1 X + f2 X^2; the lower triangle from conj(X), conj(X^2)
-    E.m[0] = mkf((float)(f0r + f1r * d0 + f2r * q0), (float)(f0i + f1i * d0 + f2i * q0));
-    E.m[4] = mkf((float)(f0r + f1r * d1 + f2r * q1), (float)(f0i + f1i * d1 + f2i * q1));
-    E.m[8] = mkf((float)(f0r + f1r * d2 + f2r * q2), (float)(f0i + f1i * d2 + f2i * q2));
+    E.m[0] = mkf((float)fma(f2r, q0, fma(f1r, d0, f0r)), (float)fma(f2i, q0, fma(f1i, d0, f0i)));
+    E.m[4] = mkf((float)fma(f2r, q1, fma(f1r, d1, f0r)), (float)fma(f2i, q1, fma(f1i, d1, f0i)));
+    E.m[8] = mkf((float)fma(f2r, q2, fma(f1r, d2, f0r)), (float)fma(f2i, q2, fma(f1i, d2, f0i)));
     auto off = [&](cplx a, cplx b, cplxf& up, cplxf& lo) {
-        const cplx u = cadd(cmul(f1, a), cmul(f2, b));
-        const cplx l = cadd(cmul(f1, conjg(a)), cmul(f2, conjg(b)));
+        const cplx u = cmad(cmul(f1, a), f2, b);
+        const cplx l = cmadc(cmulc(f1, a), f2, b);
         up = mkf((float)u.x, (float)u.y);
         lo = mkf((float)l.x, (float)l.y);
     };
@@ -295,12 +329,14 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
 // arguments that occur: u in (0, 1] and never subnormal, the angle as an integer
 // fraction of a turn.  Against the library's log, sqrt and sincospi, which
 // also take subnormals, infinities and arguments beyond one turn: about 70
-// instead of 130 FP64 instructions per pair.
+// instead of 130 FP64 instructions per pair.  The fused multiply-adds are written out
+// and no others are formed: every kernel gives the same bits.
 
 // log u for a normal u in (0, 1]: u = 2^e m, m in [sqrt(1/2), sqrt 2);
 // log m = 2 atanh(s), s = f / (2 + f), f = m - 1, as (f - f^2/2) + s (f^2/2 + R),
 // R = s^2 P(s^2) with P fitted (relative error 9e-18 of log m)
 __device__ __forceinline__ double log_unit(double u) {
+#pragma clang fp contract(off)
     uint32_t hi = (uint32_t)__double2hiint(u) + (0x3ff00000u - 0x3fe6a09eu);
     const int e = (int)(hi >> 20) - 0x3ff;
     hi = (hi & 0xfffffu) + 0x3fe6a09eu;
@@ -328,6 +364,7 @@ __device__ __forceinline__ double log_unit(double u) {
 
 // sqrt x, x >= 0 and not subnormal
 __device__ __forceinline__ double sqrt_pos(double x) {
+#pragma clang fp contract(off)
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     const double r = fma(-h, g, 0.5);
@@ -340,6 +377,7 @@ __device__ __forceinline__ double sqrt_pos(double x) {
 // rr (cos, sin) of (q + r) quarter turns, |r| <= 1/2: polynomials in r^2 fitted
 // to sin and cos of r pi/2 (relative errors 1.3e-17 and 1.2e-19)
 __device__ __forceinline__ void polar_quarter(double rr, uint32_t q, double r, double& z0, double& z1) {
+#pragma clang fp contract(off)
     const double z = r * r;
     double ps = 5.6422280858396281912e-8;
     ps = fma(ps, z, -3.5987029691976957449e-6);
@@ -387,6 +425,7 @@ __device__ __forceinline__ void box_muller_pair(uint32_t site, uint32_t step, ui
 // scaled by ln 2 (in two parts, as one rounding) and its reciprocal square root
 // refined once, without the library's handling of those.
 __device__ __forceinline__ float radius_f(bool lo, float w) {
+#pragma clang fp contract(off)
     const float a = lo ? w : 1.0f - w;
     const float l2 = __builtin_amdgcn_logf(a);
     const float t = l2 * 0x1.62e42ep-1f;
@@ -461,32 +500,40 @@ __device__ __forceinline__ void kspace_normals4(uint32_t k, uint32_t step, uint3
     box_muller32(c[2], c[3], z[2], z[3]);
 }
 
+// row 2 of an SU(3) matrix from rows 0 and 1: conj(row 0 x row 1)
+template <typename C>
+__device__ __forceinline__ void row2_of(C* m) {
+    auto minor = [](C a, C b, C c, C d) { return conjg(cmad(cmul(a, b), C{-c.x, -c.y}, d)); };      // conj(a b - c d)
+    m[6] = minor(m[1], m[5], m[2], m[4]);
+    m[7] = minor(m[2], m[3], m[0], m[5]);
+    m[8] = minor(m[0], m[4], m[1], m[3]);
+}
+
 // Projection of a near-unitary 3x3 matrix onto SU(3): Gram-Schmidt on rows 0
 // and 1, row 2 = conj(row0 x row1) (unit determinant).  The periodic
 // reunitarisation of the mixed-precision form.
 __device__ __forceinline__ m3 su3_project(const m3& M) {
+#pragma clang fp contract(off)
     m3 R;
     double n0 = 0.0;
 #pragma unroll
-    for (int k = 0; k < 3; k++) n0 += M.m[k].x * M.m[k].x + M.m[k].y * M.m[k].y;
+    for (int k = 0; k < 3; k++) n0 = fma(M.m[k].x, M.m[k].x, fma(M.m[k].y, M.m[k].y, n0));
     n0 = 1.0 / sqrt(n0);
 #pragma unroll
     for (int k = 0; k < 3; k++) R.m[k] = cscale(M.m[k], n0);
     cplx p = mk(0.0, 0.0);     // <row0, row1>
 #pragma unroll
-    for (int k = 0; k < 3; k++) p = cadd(p, cmulc(M.m[3 + k], R.m[k]));
+    for (int k = 0; k < 3; k++) p = cmadc(p, M.m[3 + k], R.m[k]);
     double n1 = 0.0;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        R.m[3 + k] = csub(M.m[3 + k], cmul(p, R.m[k]));
-        n1 += R.m[3 + k].x * R.m[3 + k].x + R.m[3 + k].y * R.m[3 + k].y;
+        R.m[3 + k] = cmad(M.m[3 + k], mk(-p.x, -p.y), R.m[k]);
+        n1 = fma(R.m[3 + k].x, R.m[3 + k].x, fma(R.m[3 + k].y, R.m[3 + k].y, n1));
     }
     n1 = 1.0 / sqrt(n1);
 #pragma unroll
     for (int k = 0; k < 3; k++) R.m[3 + k] = cscale(R.m[3 + k], n1);
-    R.m[6] = conjg(csub(cmul(R.m[1], R.m[5]), cmul(R.m[2], R.m[4])));
-    R.m[7] = conjg(csub(cmul(R.m[2], R.m[3]), cmul(R.m[0], R.m[5])));
-    R.m[8] = conjg(csub(cmul(R.m[0], R.m[4]), cmul(R.m[1], R.m[3])));
+    row2_of(R.m);
     return R;
 }
 

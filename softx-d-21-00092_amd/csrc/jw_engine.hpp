@@ -36,15 +36,25 @@
 
 namespace jw {
 
-// Row passes: N / DIV threads (64..1024), SPT sites per thread.  At N = 2048
-// the four padded rows in LDS (139 KB) allow one workgroup per CU; 512 threads
-// (DIV = 4) measured faster than 1024 for these passes.
-template <int N, int DIV = 4>
+// Row passes: one lattice row and four planes a workgroup, T = N / PT threads a plane
+// (jw_regfft.hpp).  A plane of the row sits in LDS in the order of the transform's
+// own exchange, so that the thread that transforms reads and writes its own
+// slots; site y is at slot (y / T) SUB + y mod T.
+template <int N>
 struct RowE {
-    static constexpr int NT = (N / DIV < 64) ? 64 : ((N / DIV > 1024) ? 1024 : N / DIV);
+    static constexpr int T = RegFft<N>::T, PT = RegFft<N>::PT;
+    static constexpr int NT = 4 * T;
     static constexpr int SPT = N / NT;                  // sites per thread
-    static_assert(SPT >= 1 && SPT * NT == N, "row pass needs N a multiple of its thread count");
+    static_assert(SPT >= 1 && SPT * NT == N && NT >= 64, "row pass");
 };
+template <int N, typename C>
+struct RowT {
+    static constexpr int SUB = RegLds<N, 1, C>::SUB, PL = RegLds<N, 1, C>::ELEMS;      // PL: elements of a plane
+};
+template <int N, typename C>
+__device__ __forceinline__ int row_slot_of(int y) {
+    return (y / RowE<N>::T) * RowT<N, C>::SUB + y % RowE<N>::T;
+}
 // Row-major column passes hold the X and Y tiles of one W-column strip together
 // in LDS (2 W N complex values plus one padding row in eight, 144 KB at most in
 // FP64): W = min(16, 4096 / N) for both forms (wider FP32 strips measured
@@ -60,11 +70,10 @@ struct ColE {
     static_assert(W >= 1 && W <= N && N % W == 0 && PER * NT == ELEMS && PAIRS * NT == W * N, "column tiling");
 };
 
-// minimum waves per SIMD requested of the row passes: the FP32 rows (4 padded
-// rows, 70 KB of LDS at N = 2048) fit two 512-thread workgroups per CU when
-// they stay within 128 VGPRs
+// minimum waves per SIMD requested of the row passes: two 512-thread workgroups per CU
+// in FP32 (128 registers; 70 KB of LDS at N = 2048), one in FP64
 template <typename C>
-struct RowWaves { static constexpr int value = sizeof(C) == sizeof(double2) ? 1 : 4; };
+struct RowWaves { static constexpr int value = sizeof(C) == sizeof(double2) ? 2 : 4; };
 
 // strip index for block b so that the strips on one XCD (blocks b, b+8, ...) are adjacent
 __device__ __forceinline__ int xcd_strip(int b, int nstrips) {
@@ -73,10 +82,11 @@ __device__ __forceinline__ int xcd_strip(int b, int nstrips) {
 }
 
 // offset of site (x, y) in an intermediate plane of layout BF (0 and 2
-// row-major, 1 row-major for the 64-byte-strip column pass, 4 and 8 row blocks)
+// row-major, 1 row-major for the 64-byte-strip column pass, 3 row-major in frequency
+// order: the matrix-core column stages and the large lattices, 4 and 8 row blocks)
 template <int N, int BF>
 __device__ __forceinline__ size_t lay(int x, int y) {
-    if constexpr (BF <= 2 || BF >= 16) return (size_t)x * N + y;
+    if constexpr (BF <= 3 || BF >= 16) return (size_t)x * N + y;
     else return ((size_t)(x / BF) * N + y) * BF + (x % BF);
 }
 
@@ -91,12 +101,33 @@ __device__ __forceinline__ size_t pat(int q, int x, int y, size_t V) {
     else return (size_t)q * V + lay<N, BF>(x, y);
 }
 
+// Row spectra on row-major planes (BF = 0) are stored in the order in which the
+// row transform ends: position s = q T + j holds the frequency of v[q] in thread j,
+// so that a wave writes and reads whole contiguous runs (in frequency order its
+// 64 elements are eight runs of 8; FP32 U xi~ U^dagger at N = 2048 242 against 195 us).  The column
+// pass takes columns independently and needs only their frequency.
+template <int N, int BF>
+__device__ __forceinline__ int freq_of_pos(int s) {
+    typedef RegFft<N> F;
+    if constexpr (BF != 0) return s;
+    else return reg_freq<N>(s % F::T / F::N3, s % F::N3, 0) + reg_freq_q<N>(s / F::T);
+}
+// position of v[q] in thread j: pos0(j) + posq(q)
+template <int N, int BF>
+__device__ __forceinline__ int pos0(int j) {
+    return BF == 0 ? j : reg_freq<N>(j / RegFft<N>::N3, j % RegFft<N>::N3, 0);
+}
+template <int N, int BF>
+__device__ __forceinline__ constexpr int posq(int q) {
+    return BF == 0 ? q * RegFft<N>::T : reg_freq_q<N>(q);
+}
+
 // lattice row of row-pass block b.  Blocks are dealt round-robin to the 8 XCDs;
 // with a blocked layout the BF rows sharing segments go to one XCD in
 // consecutive turns (a bijection on [0, N) for N a multiple of 8 BF).
 template <int N, int BF>
 __device__ __forceinline__ int row_of_block(int b) {
-    if constexpr (BF <= 2 || BF >= 16) return b;
+    if constexpr (BF <= 3 || BF >= 16) return b;
     else {
         static_assert(N % (8 * BF) == 0, "blocked layout needs N a multiple of 8 BF");
         const int t = b >> 3, xcd = b & 7;
@@ -152,9 +183,7 @@ __device__ __forceinline__ void load_u(M& u, const C* __restrict__ U, size_t V, 
 #pragma unroll
     for (int k = 0; k < UPlanes<C>::value; k++) u.m[k] = U[k * V + i];
     if constexpr (UPlanes<C>::value == 6) {
-        u.m[6] = conjg(csub(cmul(u.m[1], u.m[5]), cmul(u.m[2], u.m[4])));
-        u.m[7] = conjg(csub(cmul(u.m[2], u.m[3]), cmul(u.m[0], u.m[5])));
-        u.m[8] = conjg(csub(cmul(u.m[0], u.m[4]), cmul(u.m[1], u.m[3])));
+        row2_of(u.m);
     }
 }
 template <typename C, typename M>
@@ -187,12 +216,40 @@ __device__ __forceinline__ int opaque_v(int v) {
     return v;
 }
 
-// inverse row FFT of 4 planes in LDS; in FP32 through opaque twiddles and
-// thread index (fewer live registers around the site algebra)
-template <int N, int NT, int PN, typename C, typename TW>
-__device__ __forceinline__ void row_ifft4(C* lds, TW tw, int tid) {
-    if constexpr (sizeof(C) == sizeof(float2) || N <= 1024) lds_fft<N, 4, 1, PN, NT, +1, 4>(lds, tw_fft(tw), opaque_v(tid));
-    else lds_fft<N, 4, 1, PN, NT, +1, 4>(lds, tw, tid);
+// the points of a thread (plane tid / T) of a row spectrum: src(plane, position)
+template <int N, int BF, typename C, typename F>
+__device__ __forceinline__ void row_load(C* v, int tid, F&& src) {
+    const int t = opaque_v(tid), p = t / RowE<N>::T, j = t % RowE<N>::T;
+    const int k0 = pos0<N, BF>(j);
+#pragma unroll
+    for (int q = 0; q < RowE<N>::PT; q++) v[q] = src(p, k0 + posq<N, BF>(q));
+}
+// inverse transform of the loaded points into the plane's slots (site order).
+// FIRST: no access of the slots by other threads is pending.
+template <int N, bool FIRST, typename C>
+__device__ __forceinline__ void row_inv(C* v, C* lds, const C* __restrict__ tw, int tid) {
+    const int t = opaque_v(tid), p = t / RowE<N>::T, j = t % RowE<N>::T;
+    C* pl = lds + p * RowT<N, C>::PL;
+    reg_fft_inv<N, 1, FIRST>(v, pl, tw_fft(tw), j);
+    const int j2 = opaque_v(tid) % RowE<N>::T;
+#pragma unroll
+    for (int r = 0; r < RowE<N>::PT; r++) pl[r * RowT<N, C>::SUB + j2] = v[r];
+}
+// forward transform of the plane's slots, stored by dst(plane, position, value)
+template <int N, int BF, typename C, typename F>
+__device__ __forceinline__ void row_fwd(C* lds, const C* __restrict__ tw, int tid, F&& dst) {
+    C v[RowE<N>::PT];
+    {
+        const int t = opaque_v(tid), p = t / RowE<N>::T, j = t % RowE<N>::T;
+        C* pl = lds + p * RowT<N, C>::PL;
+#pragma unroll
+        for (int r = 0; r < RowE<N>::PT; r++) v[r] = pl[r * RowT<N, C>::SUB + j];
+        reg_fft_fwd<N, 1, true>(v, pl, tw_fft(tw), j);
+    }
+    const int t = opaque_v(tid), p = t / RowE<N>::T, j = t % RowE<N>::T;
+    const int k0 = pos0<N, BF>(j);
+#pragma unroll
+    for (int q = 0; q < RowE<N>::PT; q++) dst(p, k0 + posq<N, BF>(q), v[q]);
 }
 
 // a thread's site index in a row pass's site loop, opaque, so that the compiler
@@ -210,108 +267,100 @@ __device__ __forceinline__ int site_of(int y) {
 // for the next step after its own sites (the noise is compute-bound, the
 // update memory-bound).  lds: 4 padded rows.
 // ---------------------------------------------------------------------------
-template <int N, int BF, typename C, typename TW>
+template <int N, int BF, typename C>
 __device__ __forceinline__ void row_noise_body(C* lds, C* __restrict__ Xi, size_t V, const NoiseSrc& ns,
-                                               const double* __restrict__ sa_pos, TW tw, int x, int tid) {
+                                               const double* __restrict__ sa_pos, const C* __restrict__ tw, int x, int tid) {
     typedef typename scalar_of<C>::type T;
-    constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT;
-    constexpr int PN = padded<N, 4>::value;     // padded row length in LDS
+    constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT, PL = RowT<N, C>::PL;
     const size_t row0 = (size_t)x * N;
     T m[SPT][8];
 #pragma unroll
     for (int q = 0; q < SPT; q++) {
-        // FP32: sites one after another (no spills at two workgroups per CU)
-        const int y = sizeof(C) == sizeof(float2) ? site_of<C>(tid + q * NT) : tid + q * NT;
+        const int y = tid + q * NT;
         T z[16];
         normals16_t(ns, row0 + y, z);
         const T s = sa_pos ? (T)sa_pos[row0 + y] : (T)1;      // in the element type: no FP64 in FP32
 #pragma unroll
-        for (int p = 0; p < 4; p++) lds[lpos<1, PN, 4>(y, p)] = C{z[4 * p] * s, z[4 * p + 2] * s};
+        for (int p = 0; p < 4; p++) lds[p * PL + row_slot_of<N, C>(y)] = C{z[4 * p] * s, z[4 * p + 2] * s};
 #pragma unroll
         for (int k = 0; k < 8; k++) m[q][k] = z[2 * k + 1] * s;
     }
     __syncthreads();
-    lds_fft<N, 4, 1, PN, NT, -1, 4>(lds, tw, tid);
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < SPT; q++) Xi[pat<N, BF>(p, x, tid + q * NT, V)] = lds[lpos<1, PN, 4>(tid + q * NT, p)];
+    row_fwd<N, BF>(lds, tw, tid, [&](int p, int k, C v) { Xi[pat<N, BF>(p, x, k, V)] = v; });
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < SPT; q++)
 #pragma unroll
-        for (int p = 0; p < 4; p++) lds[lpos<1, PN, 4>(tid + q * NT, p)] = mkc<C>(m[q][2 * p], m[q][2 * p + 1]);
+        for (int p = 0; p < 4; p++)
+            lds[p * PL + row_slot_of<N, C>(tid + q * NT)] = mkc<C>(m[q][2 * p], m[q][2 * p + 1]);
     __syncthreads();
-    lds_fft<N, 4, 1, PN, NT, -1, 4>(lds, tw, tid);
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < SPT; q++) Xi[pat<N, BF>(4 + p, x, tid + q * NT, V)] = lds[lpos<1, PN, 4>(tid + q * NT, p)];
+    row_fwd<N, BF>(lds, tw, tid, [&](int p, int k, C v) { Xi[pat<N, BF>(4 + p, x, k, V)] = v; });
 }
 
-// The noise pass proper: one plane pair at a time.  Plane p of xi_x holds
-// (n_2p, n_2p+1) and plane p of xi_y (m_2p, m_2p+1), the normals of Philox
-// calls 2p and 2p+1 (draw order n0, m0, n1, m1, ...: call q gives n_q, m_q),
-// so each pair is generated, transformed and stored on its own and nothing is
-// held across pairs: two padded rows in LDS (70 KB in FP64 at N = 2048) fit
-// two workgroups per CU (FP32: 35 KB, four); the waves-per-SIMD bound asks
-// the compiler for the registers of that many.
-template <int N, typename C>
-struct NoiseWaves { static constexpr int value = sizeof(C) == sizeof(double2) ? 4 : 8; };
+// The noise pass proper: one plane pair of a row by T threads.  Plane p of xi_x holds
+// (n_2p, n_2p+1) and plane p of xi_y (m_2p, m_2p+1), the normals of Philox calls 2p
+// and 2p+1 (draw order n0, m0, n1, m1, ...: call q gives n_q, m_q), so a thread draws
+// the PT sites of both planes that it transforms, in registers.
+template <int N>
+struct RowN {
+    static constexpr int T = RegFft<N>::T;
+    static constexpr int NT = T < 128 ? 128 : T;        // threads: NT / T rows side by side
+    static constexpr int RPW = NT / T;
+};
 
+// row x, plane pair bi.by, thread j of the row's T; lds: one plane of the row
 template <int N, int BF, typename C>
 __device__ __forceinline__ void row_noise_fwd_body(C* lds, BlockIx bi, C* __restrict__ Xi, size_t V, NoiseSrc ns,
-                                                              const double* __restrict__ sa_pos,
-                                                              const C* __restrict__ tw) {
+                                                   const double* __restrict__ sa_pos, const C* __restrict__ tw) {
     typedef typename scalar_of<C>::type T;
-    constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT;
-    constexpr int PN = padded<N, 4>::value;
-    const auto twl = tw_source<N, true>(tw);
+    constexpr int PT = RegFft<N>::PT, TR = RegFft<N>::T;
     Xi += zofs_z(bi.bz, 8, V);
     ns = batch_noise_z(ns, V, bi.bz);
-    const int x = row_of_block<N, BF>(bi.bx);
-    const size_t row0 = (size_t)x * N;
-    const int tid = bi.tid;
-#pragma unroll 1
-    for (int p = 0; p < 4; p++) {
+    const int x = row_of_block<N, BF>(bi.bx), p = bi.by;
+    const unsigned row0 = (unsigned)x * N;
+    C a[PT], b[PT];
+    const int j = opaque_v(bi.tid);
 #pragma unroll
-        for (int q = 0; q < SPT; q++) {
-            const int y = site_of<C>(tid + q * NT);
-            const size_t i = row0 + y;
-            T z[4];
-            if (ns.inj) {
-                const double* zi = ns.inj + 16 * i + 4 * p;
+    for (int r = 0; r < PT; r++) {
+        const unsigned i = row0 + j + r * TR;
+        T z[4];
+        if (ns.inj) {
+            const double* zi = ns.inj + 16 * (size_t)i + 4 * p;
 #pragma unroll
-                for (int k = 0; k < 4; k++) z[k] = (T)zi[k];
-            } else if constexpr (sizeof(T) == sizeof(double)) {
-                box_muller_pair((uint32_t)i, ns.step, ns.tag, (uint32_t)(2 * p), ns.seed, ns.traj, z[0], z[1]);
-                box_muller_pair((uint32_t)i, ns.step, ns.tag, (uint32_t)(2 * p + 1), ns.seed, ns.traj, z[2], z[3]);
-            } else {
-                box_muller_pair_f((uint32_t)i, ns.step, ns.tag, (uint32_t)(2 * p), ns.seed, ns.traj, z[0], z[1]);
-                box_muller_pair_f((uint32_t)i, ns.step, ns.tag, (uint32_t)(2 * p + 1), ns.seed, ns.traj, z[2], z[3]);
-            }
-            const T s = sa_pos ? (T)sa_pos[i] : (T)1;
-            lds[lpos<1, PN, 4>(y, 0)] = C{z[0] * s, z[2] * s};      // xi_x plane p: (n_2p, n_2p+1)
-            lds[lpos<1, PN, 4>(y, 1)] = C{z[1] * s, z[3] * s};      // xi_y plane p: (m_2p, m_2p+1)
+            for (int k = 0; k < 4; k++) z[k] = (T)zi[k];
+        } else if constexpr (sizeof(T) == sizeof(double)) {
+            box_muller_pair(i, ns.step, ns.tag, (uint32_t)(2 * p), ns.seed, ns.traj, z[0], z[1]);
+            box_muller_pair(i, ns.step, ns.tag, (uint32_t)(2 * p + 1), ns.seed, ns.traj, z[2], z[3]);
+        } else {
+            box_muller_pair_f(i, ns.step, ns.tag, (uint32_t)(2 * p), ns.seed, ns.traj, z[0], z[1]);
+            box_muller_pair_f(i, ns.step, ns.tag, (uint32_t)(2 * p + 1), ns.seed, ns.traj, z[2], z[3]);
         }
-        __syncthreads();
-        lds_fft<N, 2, 1, PN, NT, -1, 4>(lds, tw_fft(twl), opaque_v(tid));
-#pragma unroll
-        for (int q = 0; q < SPT; q++) {
-            const int y = tid + q * NT;
-            Xi[pat<N, BF>(p, x, y, V)] = lds[lpos<1, PN, 4>(y, 0)];
-            Xi[pat<N, BF>(4 + p, x, y, V)] = lds[lpos<1, PN, 4>(y, 1)];
-        }
-        __syncthreads();
+        const T s = sa_pos ? (T)sa_pos[i] : (T)1;
+        a[r] = C{z[0] * s, z[2] * s};
+        b[r] = C{z[1] * s, z[3] * s};
+        fence(a[r]);
+        fence(b[r]);
     }
+    auto store = [&](const C* v, int pl) {
+        const int t = opaque_v(bi.tid);
+        const int k0 = pos0<N, BF>(t);
+#pragma unroll
+        for (int q = 0; q < PT; q++) Xi[pat<N, BF>(pl, x, k0 + posq<N, BF>(q), V)] = v[q];
+    };
+    reg_fft_fwd<N, 1, true>(a, lds, tw_fft(tw), opaque_v(bi.tid));
+    store(a, p);
+    reg_fft_fwd<N, 1, false>(b, lds, tw_fft(tw), opaque_v(bi.tid));
+    store(b, 4 + p);
 }
 
 template <int N, int BF, typename C>
-__global__ __launch_bounds__(RowE<N>::NT, (NoiseWaves<N, C>::value)) void k_row_noise_fwd(C* __restrict__ Xi, size_t V, NoiseSrc ns,
+__global__ __launch_bounds__(RowN<N>::NT, RowWaves<C>::value) void k_row_noise_fwd(C* __restrict__ Xi, size_t V, NoiseSrc ns,
                                                               const double* __restrict__ sa_pos,
                                                               const C* __restrict__ tw) {
-    __shared__ C lds[2 * padded<N, 4>::value];
-    row_noise_fwd_body<N, BF, C>(lds, own_block(), Xi, V, ns, sa_pos, tw);
+    __shared__ C lds[RowN<N>::RPW * RowT<N, C>::PL];
+    const int s = threadIdx.x / RowN<N>::T;
+    const BlockIx bi{(int)blockIdx.x * RowN<N>::RPW + s, (int)blockIdx.y, (int)blockIdx.z, (int)threadIdx.x % RowN<N>::T};
+    row_noise_fwd_body<N, BF, C>(lds + s * RowT<N, C>::PL, bi, Xi, V, ns, sa_pos, tw);
 }
 
 // ---------------------------------------------------------------------------
@@ -324,9 +373,8 @@ __device__ __forceinline__ void row_uxiu_fwd_body(C* lds, BlockIx bi, C* __restr
                                                              const C* __restrict__ tw) {
     typedef typename scalar_of<C>::type T;
     constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT;
-    constexpr int PN = padded<N, 4>::value;     // padded row length in LDS
+    constexpr int PL = RowT<N, C>::PL;
     const int tid = bi.tid;
-    const auto twl = tw_source<N, true>(tw);
     Vv += zofs_z(bi.bz, 8, V);
     U += zofs_z(bi.bz, UPlanes<C>::value, V);
     ns = batch_noise_z(ns, V, bi.bz);
@@ -355,33 +403,25 @@ __device__ __forceinline__ void row_uxiu_fwd_body(C* lds, BlockIx bi, C* __restr
             fence(vy[q][k]);
         }
 #pragma unroll
-        for (int p = 0; p < 4; p++) lds[lpos<1, PN, 4>(y, p)] = mkc<C>(vx[2 * p], vx[2 * p + 1]);
+        for (int p = 0; p < 4; p++) lds[p * PL + row_slot_of<N, C>(y)] = mkc<C>(vx[2 * p], vx[2 * p + 1]);
     }
     __syncthreads();
-    lds_fft<N, 4, 1, PN, NT, -1, 4>(lds, twl, tid);
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < SPT; q++) Vv[pat<N, BF>(p, x, tid + q * NT, V)] = lds[lpos<1, PN, 4>(tid + q * NT, p)];
+    row_fwd<N, BF>(lds, tw, tid, [&](int p, int k, C v) { Vv[pat<N, BF>(p, x, k, V)] = v; });
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < SPT; q++)
 #pragma unroll
-        for (int p = 0; p < 4; p++) lds[lpos<1, PN, 4>(tid + q * NT, p)] = mkc<C>(vy[q][2 * p], vy[q][2 * p + 1]);
+        for (int p = 0; p < 4; p++)
+            lds[p * PL + row_slot_of<N, C>(tid + q * NT)] = mkc<C>(vy[q][2 * p], vy[q][2 * p + 1]);
     __syncthreads();
-    lds_fft<N, 4, 1, PN, NT, -1, 4>(lds, twl, tid);
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < SPT; q++)
-            Vv[pat<N, BF>(4 + p, x, tid + q * NT, V)] = lds[lpos<1, PN, 4>(tid + q * NT, p)];
+    row_fwd<N, BF>(lds, tw, tid, [&](int p, int k, C v) { Vv[pat<N, BF>(4 + p, x, k, V)] = v; });
 }
 
 template <int N, int BF, typename C>
 __global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_uxiu_fwd(C* __restrict__ Vv, const C* __restrict__ U,
                                                              size_t V, NoiseSrc ns, const double* __restrict__ sa_pos,
                                                              const C* __restrict__ tw) {
-    __shared__ C lds[4 * padded<N, 4>::value];
+    __shared__ C lds[4 * RowT<N, C>::PL];
     row_uxiu_fwd_body<N, BF, C>(lds, own_block(), Vv, U, V, ns, sa_pos, tw);
 }
 
@@ -398,51 +438,43 @@ __device__ __forceinline__ void row_uxiu_corr_body(C* lds, BlockIx bi, C* __rest
                                                               const C* __restrict__ Xs, size_t V,
                                                               const C* __restrict__ tw) {
     typedef typename scalar_of<C>::type T;
-    constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT;
-    constexpr int PN = padded<N, 4>::value;
+    constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT, PL = RowT<N, C>::PL;
     const int tid = bi.tid;
-    const auto twl = tw_source<N, false>(tw);
     Vv += zofs_z(bi.bz, 8, V);
     U += zofs_z(bi.bz, UPlanes<C>::value, V);
     Xs += zofs_z(bi.bz, 8, V);
     const int x = row_of_block<N, BF>(bi.bx);
     const size_t row0 = (size_t)x * N;
-#pragma unroll 1
+    C h[RowE<N>::PT];
+    row_load<N, BF>(h, tid, [&](int p, int k) { return Xs[pat<N, BF>(p, x, k, V)]; });
+#pragma unroll
     for (int half = 0; half < 2; half++) {
-#pragma unroll
-        for (int p = 0; p < 4; p++)
-#pragma unroll
-            for (int q = 0; q < SPT; q++)
-                lds[lpos<1, PN, 4>(tid + q * NT, p)] = Xs[pat<N, BF>(4 * half + p, x, tid + q * NT, V)];
+        row_inv<N, true>(h, lds, tw, tid);
+        // the y direction's spectra are in flight during the x direction's site algebra
+        if (half == 0) row_load<N, BF>(h, tid, [&](int p, int k) { return Xs[pat<N, BF>(4 + p, x, k, V)]; });
         __syncthreads();
-        lds_fft<N, 4, 1, PN, NT, +1, 4>(lds, twl, tid);
         // one site at a time: keeps a single U (9 complex, row 2 rebuilt) live
 #pragma unroll 1
         for (int q = 0; q < SPT; q++) {
             const int y = tid + q * NT;
             const size_t i = row0 + y;
-            T h[8];
+            C* const slot = lds + row_slot_of<N, C>(y);
+            T g[8];
 #pragma unroll
             for (int p = 0; p < 4; p++) {
-                const C a = lds[lpos<1, PN, 4>(y, p)];
-                h[2 * p] = a.x;
-                h[2 * p + 1] = a.y;
+                const C a = slot[p * PL];
+                g[2 * p] = a.x;
+                g[2 * p + 1] = a.y;
             }
             typename site_mat<C>::type u;
             load_u(u, U, V, i);
             T v[8];
-            uxiu_gen(u, h, v);
+            uxiu_gen(u, g, v);
 #pragma unroll
-            for (int p = 0; p < 4; p++) lds[lpos<1, PN, 4>(y, p)] = mkc<C>(v[2 * p], v[2 * p + 1]);
+            for (int p = 0; p < 4; p++) slot[p * PL] = mkc<C>(v[2 * p], v[2 * p + 1]);
         }
         __syncthreads();
-        lds_fft<N, 4, 1, PN, NT, -1, 4>(lds, twl, tid);
-#pragma unroll
-        for (int p = 0; p < 4; p++)
-#pragma unroll
-            for (int q = 0; q < SPT; q++)
-                Vv[pat<N, BF>(4 * half + p, x, tid + q * NT, V)] = lds[lpos<1, PN, 4>(tid + q * NT, p)];
-        __syncthreads();
+        row_fwd<N, BF>(lds, tw, tid, [&](int p, int k, C v) { Vv[pat<N, BF>(4 * half + p, x, k, V)] = v; });
     }
 }
 
@@ -450,7 +482,7 @@ template <int N, int BF, typename C>
 __global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_uxiu_corr(C* __restrict__ Vv, const C* __restrict__ U,
                                                               const C* __restrict__ Xs, size_t V,
                                                               const C* __restrict__ tw) {
-    __shared__ C lds[4 * padded<N, 4>::value];
+    __shared__ C lds[4 * RowT<N, C>::PL];
     row_uxiu_corr_body<N, BF, C>(lds, own_block(), Vv, U, Xs, V, tw);
 }
 
@@ -464,7 +496,8 @@ __global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_uxiu_co
 //   (kspace_normals4, plane pair p = bi.by, noise key from ns); X and Y then
 //   receive the row spectra of the position-space noise.
 // X, Y: row spectra of plane p; one workgroup per strip of W columns and plane
-// pair.  A thread holds PT points of one column of X and of Y; LDS holds one
+// pair.  BF = 0: columns in the order of freq_of_pos, and sa's likewise; otherwise
+// (the large lattices) column c is frequency c.  A thread holds PT points of one column of X and of Y; LDS holds one
 // plane of the strip for the exchanges, and the (4 sin^2, sin) table of kx.
 //
 // What bounds it: the loaded pass moves 12 planes at 3.1-3.2 TB/s (FP64 and FP32
@@ -486,7 +519,7 @@ struct ColR {
     static constexpr int WMAX = (F64 ? 8192 : 16384) / N;
     static constexpr int W = WMAX < WSEG ? WMAX : (N / RegFft<N>::PT * WSEG < 64 ? 64 / (N / RegFft<N>::PT) : WSEG);
     static constexpr int NT = N / RegFft<N>::PT * W;
-    static constexpr int ELEMS = N * W;                                  // of C in LDS
+    static constexpr int ELEMS = RegLds<N, W, C>::ELEMS;                 // of C in LDS
     static constexpr bool TAB = ELEMS * (int)sizeof(C) + N * 16 <= 160 * 1024;
     static constexpr int LDS = ELEMS + (TAB ? N * 16 / (int)sizeof(C) : 0);
     // registers: 256 (FP64; 32 points a thread) or 128 a thread
@@ -502,8 +535,8 @@ __device__ __forceinline__ int after(int v, T d) {
     return v;
 }
 
-// lds: N W elements; kt: N (q4, sb) pairs (TAB), filled here by the whole workgroup
-template <int N, int CORR, int GEN, int MODE, typename C>
+// lds: ColR::ELEMS elements; kt: N (q4, sb) pairs (TAB), filled here by the whole workgroup
+template <int N, int CORR, int GEN, int MODE, int BF, typename C>
 __device__ __forceinline__ void col_reg_body(C* lds, double2* kt, BlockIx bi, C* __restrict__ Z, C* __restrict__ X,
                                              C* __restrict__ Y, size_t V, const double* __restrict__ q4,
                                              const double* __restrict__ sb, const double* __restrict__ sa,
@@ -542,9 +575,9 @@ __device__ __forceinline__ void col_reg_body(C* lds, double2* kt, BlockIx bi, C*
     }
     const NoiseSrc nk = batch_noise_z(ns, V, bi.bz);
     const double invV = 1.0 / ((double)N * (double)N);
-    const int j = tk / W, ky = col0 + tk % W;
+    const int j = tk / W, cy = col0 + tk % W, ky = freq_of_pos<N, BF>(cy);
     const int kx0 = reg_freq<N>(j / F::N3, j % F::N3, 0);
-    const unsigned k0 = (unsigned)(kx0 * N + ky);
+    const unsigned k0 = (unsigned)(kx0 * N + ky), s0 = (unsigned)(kx0 * N + cy);     // sa is stored by position
     const double q4y = q4[ky];
     const T sby = (T)sb[ky];
 #pragma unroll
@@ -561,16 +594,16 @@ __device__ __forceinline__ void col_reg_body(C* lds, double2* kt, BlockIx bi, C*
         else kq = make_double2((q4 + dk)[kx0], (sb + dk)[kx0]);
         // kernel factors in the element type: one FP64 division per pair in FP64,
         // one FP32 division in the mixed form (whose spectra are FP32)
-        const double cc = MODE == 1 ? (sa + (size_t)dk * N)[k0] : 1.0;
+        const double cc = MODE == 1 ? (sa + (size_t)dk * N)[s0] : 1.0;
         T f = (T)(-2.0 * M_PI * invV * cc) / (T)(kq.x + q4y);
         if (q == 0 && k0 == 0) f = 0;
         const T fx = f * (T)kq.y, fy = f * sby;
         if constexpr (MODE == 2) {
-            const T s = (T)(sa + (size_t)dk * N)[k0];
+            const T s = (T)(sa + (size_t)dk * N)[s0];
             x[q] = cscale(x[q], s);
             y[q] = cscale(y[q], s);
         }
-        const C zq = mkc<C>(-(fx * x[q].y + fy * y[q].y), fx * x[q].x + fy * y[q].x);   // i (fx x + fy y)
+        const C zq = C{-fma_t(fx, x[q].y, fy * y[q].y), fma_t(fx, x[q].x, fy * y[q].x)};   // i (fx x + fy y)
         // the fences end each element before the next (an interleaved order spills)
         if constexpr (CORR) {
             z[q] = zq;
@@ -602,12 +635,12 @@ __device__ __forceinline__ void col_reg_body(C* lds, double2* kt, BlockIx bi, C*
     }
 }
 
-template <int N, int CORR, int GEN, int MODE, typename C>
+template <int N, int CORR, int GEN, int MODE, int BF, typename C>
 __global__ __launch_bounds__((ColR<N, C>::NT), (ColR<N, C>::WAVES)) void k_col_reg(
     C* __restrict__ Z, C* __restrict__ X, C* __restrict__ Y, size_t V, const double* __restrict__ q4,
     const double* __restrict__ sb, const double* __restrict__ sa, const C* __restrict__ tw, NoiseSrc ns) {
     __shared__ __align__(16) C lds[ColR<N, C>::LDS];
-    col_reg_body<N, CORR, GEN, MODE, C>(lds, reinterpret_cast<double2*>(lds + ColR<N, C>::ELEMS), own_block(), Z, X, Y,
+    col_reg_body<N, CORR, GEN, MODE, BF, C>(lds, reinterpret_cast<double2*>(lds + ColR<N, C>::ELEMS), own_block(), Z, X, Y,
                                         V, q4, sb, sa, tw, ns);
 }
 
@@ -932,39 +965,30 @@ __device__ __forceinline__ void row_update_body(C* lds, BlockIx bi, C* __restric
                                                               int reunit, const C* __restrict__ tw, int next_noise,
                                                               C* __restrict__ Xi, NoiseSrc ns,
                                                               const double* __restrict__ sa_pos) {
-    static_assert(RowE<N, 4>::NT == RowE<N>::NT, "the update and noise bodies share the thread count");
     typedef typename scalar_of<C>::type T;
-    constexpr int NT = RowE<N, 4>::NT, SPT = RowE<N, 4>::SPT;
-    constexpr int PN = padded<N, 4>::value;     // padded row length in LDS
+    constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT, PL = RowT<N, C>::PL;
     const int tid = bi.tid;
-    const auto twl = tw_source<N, sizeof(C) == sizeof(float2)>(tw);
     U += zofs_z(bi.bz, UPlanes<C>::value, V);
     ZA += zofs_z(bi.bz, 4, V);
     ZB += zofs_z(bi.bz, 4, V);
     const int x = row_of_block<N, BF>(bi.bx);
     const size_t row0 = (size_t)x * N;
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < SPT; q++) lds[lpos<1, PN, 4>(tid + q * NT, p)] = ZA[p * V + lay<N, BF>(x, tid + q * NT)];
+    C za[RowE<N>::PT], zb[RowE<N>::PT];
+    row_load<N, BF>(za, tid, [&](int p, int k) { return ZA[p * V + lay<N, BF>(x, k)]; });
+    row_load<N, BF>(zb, tid, [&](int p, int k) { return ZB[p * V + lay<N, BF>(x, k)]; });
+    row_inv<N, true>(za, lds, tw, tid);
     __syncthreads();
-    row_ifft4<N, NT, PN>(lds, twl, tid);
     T ha[SPT][8];
 #pragma unroll
     for (int q = 0; q < SPT; q++)
 #pragma unroll
         for (int p = 0; p < 4; p++) {
-            const C a = lds[lpos<1, PN, 4>(tid + q * NT, p)];
+            const C a = lds[p * PL + row_slot_of<N, C>(tid + q * NT)];
             ha[q][2 * p] = a.x;
             ha[q][2 * p + 1] = a.y;
         }
+    row_inv<N, false>(zb, lds, tw, tid);
     __syncthreads();
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < SPT; q++) lds[lpos<1, PN, 4>(tid + q * NT, p)] = ZB[p * V + lay<N, BF>(x, tid + q * NT)];
-    __syncthreads();
-    row_ifft4<N, NT, PN>(lds, twl, tid);
 #pragma unroll
     for (int q = 0; q < SPT; q++) {
         const int y = site_of<C>(tid + q * NT);
@@ -972,7 +996,7 @@ __device__ __forceinline__ void row_update_body(C* lds, BlockIx bi, C* __restric
         T hb[8];
 #pragma unroll
         for (int p = 0; p < 4; p++) {
-            const C b = lds[lpos<1, PN, 4>(y, p)];
+            const C b = lds[p * PL + row_slot_of<N, C>(y)];
             hb[2 * p] = b.x;
             hb[2 * p + 1] = b.y;
         }
@@ -1015,17 +1039,17 @@ __device__ __forceinline__ void row_update_body(C* lds, BlockIx bi, C* __restric
         __syncthreads();
         NoiseSrc nn = batch_noise_z(ns, V, bi.bz);
         nn.step += 1;
-        row_noise_body<N, BF, C>(lds, Xi + zofs_z(bi.bz, 8, V), V, nn, sa_pos, tw_fft(twl), x, bi.tid);
+        row_noise_body<N, BF, C>(lds, Xi + zofs_z(bi.bz, 8, V), V, nn, sa_pos, tw, x, bi.tid);
     }
 }
 
 template <int N, int BF, typename C>
-__global__ __launch_bounds__((RowE<N, 4>::NT), RowWaves<C>::value) void k_row_update(C* __restrict__ U, const C* __restrict__ ZA,
+__global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_update(C* __restrict__ U, const C* __restrict__ ZA,
                                                               const C* __restrict__ ZB, size_t V, double ss,
                                                               int reunit, const C* __restrict__ tw, int next_noise,
                                                               C* __restrict__ Xi, NoiseSrc ns,
                                                               const double* __restrict__ sa_pos) {
-    __shared__ C lds[4 * padded<N, 4>::value];
+    __shared__ C lds[4 * RowT<N, C>::PL];
     row_update_body<N, BF, C>(lds, own_block(), U, ZA, ZB, V, ss, reunit, tw, next_noise, Xi, ns, sa_pos);
 }
 
@@ -1094,7 +1118,9 @@ struct ColMultiT { static constexpr int value = sizeof(C) == sizeof(double2) ? 5
 template <int T, int planes, typename C>
 struct RowMultiLds {
     template <int N>
-    static constexpr int need() { return RowE<N>::NT <= T ? (T / RowE<N>::NT) * planes * padded<N, 4>::value : 0; }
+    static constexpr int NT() { return planes == 1 ? RegFft<N>::T : RowE<N>::NT; }
+    template <int N>
+    static constexpr int need() { return NT<N>() <= T ? (T / NT<N>()) * planes * RowT<N, C>::PL : 0; }
     static constexpr int a = need<64>() > need<128>() ? need<64>() : need<128>();
     static constexpr int b = need<256>() > need<512>() ? need<256>() : need<512>();
     static constexpr int c = need<1024>() > need<2048>() ? need<1024>() : need<2048>();
@@ -1126,13 +1152,17 @@ __device__ __forceinline__ BlockIx row_slot(int b) {
 template <int N, int T>
 __device__ __forceinline__ int row_sub() { return threadIdx.x / RowE<N>::NT; }
 
+// noise: T / (threads of a row) rows of one plane pair in a block; plane pairs, then trajectories
+template <int N> struct RowNoiseNT { static constexpr int value = RegFft<N>::T; };
 template <typename C, int T>
-__global__ __launch_bounds__(T, (NoiseWaves<64, C>::value)) void k_row_noise_fwd_multi(MultiRun<C> m) {
-    __shared__ C lds[RowMultiLds<T, 2, C>::value];
-    dispatch_group<T, RowNT>(m, [&](auto n, const GroupRun<C>& g, int b) {
+__global__ __launch_bounds__(T, RowWaves<C>::value) void k_row_noise_fwd_multi(MultiRun<C> m) {
+    __shared__ C lds[RowMultiLds<T, 1, C>::value];
+    dispatch_group<T, RowNoiseNT>(m, [&](auto n, const GroupRun<C>& g, int b) {
         constexpr int N = decltype(n)::value;
-        row_noise_fwd_body<N, 0, C>(lds + row_sub<N, T>() * 2 * padded<N, 4>::value, row_slot<N, T>(b), g.Xi, g.V,
-                                    g.ns, g.sa_pos, g.tw);
+        constexpr int TR = RegFft<N>::T, RPB = T / TR, NRB = N / RPB;
+        const int s = threadIdx.x / TR;
+        const BlockIx bi{(b % NRB) * RPB + s, (b / NRB) % 4, b / (NRB * 4), (int)threadIdx.x % TR};
+        row_noise_fwd_body<N, 0, C>(lds + s * RowT<N, C>::PL, bi, g.Xi, g.V, g.ns, g.sa_pos, g.tw);
     });
 }
 template <typename C, int T>
@@ -1140,7 +1170,7 @@ __global__ __launch_bounds__(T, RowWaves<C>::value) void k_row_uxiu_fwd_multi(Mu
     __shared__ C lds[RowMultiLds<T, 4, C>::value];
     dispatch_group<T, RowNT>(m, [&](auto n, const GroupRun<C>& g, int b) {
         constexpr int N = decltype(n)::value;
-        row_uxiu_fwd_body<N, 0, C>(lds + row_sub<N, T>() * 4 * padded<N, 4>::value, row_slot<N, T>(b), g.Vv, g.U, g.V,
+        row_uxiu_fwd_body<N, 0, C>(lds + row_sub<N, T>() * 4 * RowT<N, C>::PL, row_slot<N, T>(b), g.Vv, g.U, g.V,
                                    g.ns, g.sa_pos, g.tw);
     });
 }
@@ -1149,7 +1179,7 @@ __global__ __launch_bounds__(T, RowWaves<C>::value) void k_row_uxiu_corr_multi(M
     __shared__ C lds[RowMultiLds<T, 4, C>::value];
     dispatch_group<T, RowNT>(m, [&](auto n, const GroupRun<C>& g, int b) {
         constexpr int N = decltype(n)::value;
-        row_uxiu_corr_body<N, 0, C>(lds + row_sub<N, T>() * 4 * padded<N, 4>::value, row_slot<N, T>(b), g.Vv, g.U, g.Xi,
+        row_uxiu_corr_body<N, 0, C>(lds + row_sub<N, T>() * 4 * RowT<N, C>::PL, row_slot<N, T>(b), g.Vv, g.U, g.Xi,
                                     g.V, g.tw);
     });
 }
@@ -1158,7 +1188,7 @@ __global__ __launch_bounds__(T, RowWaves<C>::value) void k_row_update_multi(Mult
     __shared__ C lds[RowMultiLds<T, 4, C>::value];
     dispatch_group<T, RowNT>(m, [&](auto n, const GroupRun<C>& g, int b) {
         constexpr int N = decltype(n)::value;
-        row_update_body<N, 0, C>(lds + row_sub<N, T>() * 4 * padded<N, 4>::value, row_slot<N, T>(b), g.U, g.ZA, g.ZB,
+        row_update_body<N, 0, C>(lds + row_sub<N, T>() * 4 * RowT<N, C>::PL, row_slot<N, T>(b), g.U, g.ZA, g.ZB,
                                  g.V, ss, reunit, g.tw, 0, g.Xi, g.ns, g.sa_pos);
     });
 }
@@ -1175,34 +1205,40 @@ __global__ __launch_bounds__((ColMultiT<C>::value), (ColR<2048, C>::WAVES)) void
         const int s = threadIdx.x / CR::NT, u = (b % NB) * SPB + s;
         const BlockIx bi{u % NS, u / NS, b / NB, (int)threadIdx.x % CR::NT};
         C* X = use_v ? g.Vv : g.Xi;
-        col_reg_body<N, CORR, GEN, MODE, C>(lds + s * CR::ELEMS, reinterpret_cast<double2*>(lds + SPB * CR::ELEMS), bi,
+        col_reg_body<N, CORR, GEN, MODE, 0, C>(lds + s * CR::ELEMS, reinterpret_cast<double2*>(lds + SPB * CR::ELEMS), bi,
                                             use_v ? g.ZB : g.ZA, X, X + 4 * g.V, g.V, g.q4, g.sb, g.sa_k, g.tw, g.ns);
     });
 }
 
-// blocks of group g in a row launch of T threads / in a column launch
-template <typename C>
+// f(int_c<N>) for a batch size
+template <typename F>
+inline int for_size(int N, F&& f) {
+    switch (N) {
+        case 64: return f(int_c<64>{});
+        case 128: return f(int_c<128>{});
+        case 256: return f(int_c<256>{});
+        case 512: return f(int_c<512>{});
+        case 1024: return f(int_c<1024>{});
+        default: return f(int_c<2048>{});
+    }
+}
+// blocks of group g in a row launch of T threads, in the noise launch and in a
+// column launch
 inline int row_blocks(int N, int count, int T) {
-    const int nt = N / 4 < 64 ? 64 : (N / 4 > 1024 ? 1024 : N / 4);      // RowE<N>::NT
-    return count * N / (T / nt);
+    return for_size(N, [&](auto n) { constexpr int M = decltype(n)::value; return count * M / (T / RowE<M>::NT); });
+}
+inline int noise_blocks(int N, int count, int T) {
+    return for_size(N, [&](auto n) { constexpr int M = decltype(n)::value; return count * 4 * (M / (T / RegFft<M>::T)); });
 }
 template <typename C>
 inline int col_blocks(int N, int count) {
-    auto blocks = [&](auto n) {
+    return for_size(N, [&](auto n) {
         constexpr int M = decltype(n)::value;
         constexpr int SPB = ColMultiT<C>::value / ColR<M, C>::NT;
         constexpr int units = 4 * (M / ColR<M, C>::W);      // strips of the four plane pairs
         static_assert(SPB >= 1 && units % SPB == 0, "strips of a block");
         return count * (units / SPB);
-    };
-    switch (N) {
-        case 64: return blocks(int_c<64>{});
-        case 128: return blocks(int_c<128>{});
-        case 256: return blocks(int_c<256>{});
-        case 512: return blocks(int_c<512>{});
-        case 1024: return blocks(int_c<1024>{});
-        default: return blocks(int_c<2048>{});
-    }
+    });
 }
 
 // one step of every group of a batch, one launch per kernel class (row-major
@@ -1211,22 +1247,23 @@ template <typename C>
 static hipError_t step_multi_t(hipStream_t st, MultiRun<C> m, const int* counts, int maxN, const StepArgs& a) {
     if (m.ng < 1 || m.ng > JW_MAX_GROUPS) return hipErrorInvalidValue;
     const int T = maxN > 1024 ? 512 : 256;
-    int nrow = 0, ncol = 0;
+    int nrow = 0, ncol = 0, nnoise = 0;
     for (int g = 0; g < m.ng; g++) {
         if (m.g[g].N < 64 || m.g[g].N > 2048) return hipErrorInvalidValue;
-        nrow += row_blocks<C>(m.g[g].N, counts[g], T);
+        nrow += row_blocks(m.g[g].N, counts[g], T);
+        nnoise += noise_blocks(m.g[g].N, counts[g], T);
         ncol += col_blocks<C>(m.g[g].N, counts[g]);
     }
     auto set_blocks = [&](bool col) {
         for (int g = 0; g < m.ng; g++)
-            m.g[g].nblk = col ? col_blocks<C>(m.g[g].N, counts[g]) : row_blocks<C>(m.g[g].N, counts[g], T);
+            m.g[g].nblk = col ? col_blocks<C>(m.g[g].N, counts[g]) : row_blocks(m.g[g].N, counts[g], T);
     };
     const int wb = a.corr || a.kspace;
     hipError_t e;
     if (!a.kspace) {
-        set_blocks(false);
-        if (T == 256) hipLaunchKernelGGL((k_row_noise_fwd_multi<C, 256>), dim3(nrow), dim3(256), 0, st, m);
-        else hipLaunchKernelGGL((k_row_noise_fwd_multi<C, 512>), dim3(nrow), dim3(512), 0, st, m);
+        for (int g = 0; g < m.ng; g++) m.g[g].nblk = noise_blocks(m.g[g].N, counts[g], T);
+        if (T == 256) hipLaunchKernelGGL((k_row_noise_fwd_multi<C, 256>), dim3(nnoise), dim3(256), 0, st, m);
+        else hipLaunchKernelGGL((k_row_noise_fwd_multi<C, 512>), dim3(nnoise), dim3(512), 0, st, m);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     set_blocks(true);
@@ -1302,27 +1339,20 @@ static hipError_t col_pass(jw_ctx* c, C* Z, C* X, C* Y, const double* sa_k, int 
     const size_t V = c->V;
     const C* tw = twiddles<C>(c);
 #define JW_COL_ARGS Z, X, Y, V, sqrt_coupling, c->q4, c->sb, sa_k, tw, ns, noise_scale
-    if constexpr (BF == 0) {
+    if constexpr (BF == 3 && N <= 2048) {
         // split-BF16 matrix-core radix-16 stages (FP32 storage)
-        if constexpr (sizeof(C) == sizeof(float2) && N <= 2048) {
-            if (c->fft_mfma) {
-                const dim3 grid(N / ColE<N, C>::W, 4, nbatch);
-                if (gen)
-                    hipLaunchKernelGGL((k_col_kmult<N, 1, C, 0, 1, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream,
-                                       JW_COL_ARGS);
-                else if (corr)
-                    hipLaunchKernelGGL((k_col_kmult<N, 1, C, 0, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream,
-                                       JW_COL_ARGS);
-                else
-                    hipLaunchKernelGGL((k_col_kmult<N, 0, C, 0, 1>), grid, dim3(ColE<N, C, 0>::NT), 0, c->stream,
-                                       JW_COL_ARGS);
-                return hipGetLastError();
-            }
-        }
+        const dim3 grid(N / ColE<N, C>::W, 4, nbatch);
+        if (gen)
+            hipLaunchKernelGGL((k_col_kmult<N, 1, C, 0, 1, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream, JW_COL_ARGS);
+        else if (corr)
+            hipLaunchKernelGGL((k_col_kmult<N, 1, C, 0, 1>), grid, dim3(ColE<N, C, 1>::NT), 0, c->stream, JW_COL_ARGS);
+        else
+            hipLaunchKernelGGL((k_col_kmult<N, 0, C, 0, 1>), grid, dim3(ColE<N, C, 0>::NT), 0, c->stream, JW_COL_ARGS);
+    } else if constexpr (BF == 0 || BF == 3) {
         typedef ColR<N, C> CR;
         const dim3 grid(N / CR::W, 4, nbatch);
 #define JW_COL_REG(corr_, gen_, mode_)                                                                               \
-    hipLaunchKernelGGL((k_col_reg<N, corr_, gen_, mode_, C>), grid, dim3(CR::NT), 0, c->stream, Z, X, Y, V, c->q4, \
+    hipLaunchKernelGGL((k_col_reg<N, corr_, gen_, mode_, BF, C>), grid, dim3(CR::NT), 0, c->stream, Z, X, Y, V, c->q4, \
                        c->sb, sa_k, tw, ns)
         if (gen) {
             if (noise_scale) JW_COL_REG(1, 1, 2);
@@ -1389,7 +1419,7 @@ static hipError_t step_fused_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     const int next_noise = a.kspace ? 0 : fuse_noise ? a.next_noise : 0;
     if (first_noise) {
         KTimer t(c, kcls[0]);
-        hipLaunchKernelGGL((k_row_noise_fwd<N, BF, C>), dim3(N, 1, a.nbatch), dim3(RowE<N>::NT), 0, c->stream, Xi, V, a.ns,
+        hipLaunchKernelGGL((k_row_noise_fwd<N, BF, C>), dim3(N / RowN<N>::RPW, 4, a.nbatch), dim3(RowN<N>::NT), 0, c->stream, Xi, V, a.ns,
                            a.sa_pos, tw);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
@@ -1416,7 +1446,7 @@ static hipError_t step_fused_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     }
     {
         KTimer t(c, kcls[3]);
-        hipLaunchKernelGGL((k_row_update<N, BF, C>), dim3(N, 1, a.nbatch), dim3(RowE<N, 4>::NT), 0, c->stream, U, ZA, ZB, V,
+        hipLaunchKernelGGL((k_row_update<N, BF, C>), dim3(N, 1, a.nbatch), dim3(RowE<N>::NT), 0, c->stream, U, ZA, ZB, V,
                            a.sqrt_step, a.reunit, tw, next_noise, Xi, a.ns, a.sa_pos);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
@@ -1428,7 +1458,10 @@ template <int N, typename C>
 hipError_t step_fused_layout(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, const StepArgs& a,
                                     const int* kcls) {
     switch (c->layout) {
-        case 0: return step_fused_n<N, 0>(c, U, Xi, Vv, ZA, ZB, a, kcls);
+        case 0:
+            if constexpr (sizeof(C) == sizeof(float2))
+                if (c->fft_mfma) return step_fused_n<N, 3>(c, U, Xi, Vv, ZA, ZB, a, kcls);
+            return step_fused_n<N, 0>(c, U, Xi, Vv, ZA, ZB, a, kcls);
         case 1: return step_fused_n<N, 1>(c, U, Xi, Vv, ZA, ZB, a, kcls);
         case 2: return step_fused_n<N, 2>(c, U, Xi, Vv, ZA, ZB, a, kcls);
         case 4: return step_fused_n<N, 4>(c, U, Xi, Vv, ZA, ZB, a, kcls);

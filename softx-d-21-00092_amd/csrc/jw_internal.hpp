@@ -60,6 +60,10 @@ struct jw_ctx {
     // sa16[((kx / 16) N + ky) 16 + kx mod 16] = sa[kx N + ky]
     double* sa16;
     unsigned sa16_gen;     // sa_gen it was built from (0: never)
+    // k-space sqrt(alpha) with ky in the order of the fused step's row-major row
+    // spectra: sap[kx N + s] = sa[kx N + frequency of position s]
+    double* sap;
+    unsigned sap_gen;      // sa_gen it was built from (0: never)
     // injected normals (AoS, up to 16 per site), valid for one generator call
     double* inj;
     int inj_per_site;      // 0 when no injection is pending
@@ -132,7 +136,7 @@ bool fused_supported(int N);
 struct StepArgs {
     NoiseSrc ns;
     const double* sa_pos;    // sqrt(alpha) at positions (NOISE coupling) or nullptr
-    const double* sa_k;      // sqrt(alpha) in k: row-major for layout 0, sa16 otherwise; or nullptr
+    const double* sa_k;      // sqrt(alpha) in k as the layout's column pass reads it (sa, sap, sa16), or nullptr
     int sqrt_coupling;       // kernel factor carries sqrt(alpha) (SQRT coupling)
     int corr;                // per-mode correlated noise
     double sqrt_step;        // sqrt(Delta s)
@@ -169,6 +173,7 @@ hipError_t u_convert(jw_ctx* c, cplxf* u32, cplx* u64, int to_f32, int planes);
 hipError_t u_rebuild(jw_ctx* c, cplx* U, hipStream_t s);
 hipError_t step_inc(hipStream_t s, uint32_t* step);
 hipError_t block16(jw_ctx* c, double* out, const double* in);
+hipError_t perm_columns(jw_ctx* c, double* out, const double* in);
 
 // observables
 hipError_t corr_from_Uk(jw_ctx* c, const cplx* Uk, double* corr);

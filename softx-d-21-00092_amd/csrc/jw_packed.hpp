@@ -191,9 +191,7 @@ __device__ __forceinline__ void load_u_d(m3& u, const C* __restrict__ U, size_t 
 #pragma unroll
     for (int k = 0; k < (U6 ? 6 : 9); k++) u.m[k] = to_d(U[k * V + i]);
     if constexpr (U6 != 0) {
-        u.m[6] = conjg(csub(cmul(u.m[1], u.m[5]), cmul(u.m[2], u.m[4])));
-        u.m[7] = conjg(csub(cmul(u.m[2], u.m[3]), cmul(u.m[0], u.m[5])));
-        u.m[8] = conjg(csub(cmul(u.m[0], u.m[4]), cmul(u.m[1], u.m[3])));
+        row2_of(u.m);
     }
 }
 
@@ -460,12 +458,12 @@ static hipError_t step_large_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     if (a.nbatch != 1) return hipErrorInvalidValue;
     if (c->N == 8192) {
         if constexpr (sizeof(C) == sizeof(float2))
-            if (c->layout == 0) return step_large_n<8192, 0>(c, U, Xi, Vv, ZA, ZB, a);
+            if (c->layout == 0) return step_large_n<8192, 3>(c, U, Xi, Vv, ZA, ZB, a);
         return step_large_n<8192, 32>(c, U, Xi, Vv, ZA, ZB, a);
     }
     if (c->N == 4096) {
         if (c->layout == 32) return step_large_n<4096, 32>(c, U, Xi, Vv, ZA, ZB, a);
-        return step_large_n<4096, 0>(c, U, Xi, Vv, ZA, ZB, a);
+        return step_large_n<4096, 3>(c, U, Xi, Vv, ZA, ZB, a);
     }
     return hipErrorInvalidValue;
 }

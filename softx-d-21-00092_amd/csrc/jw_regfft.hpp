@@ -18,17 +18,21 @@
 // W sequences (columns) side by side, column fastest over the lanes.  The
 // N3 * W threads of a sub-sequence sit in one wave, so step 4 needs no workgroup
 // barrier, and it stays inside the part of LDS that the same threads read
-// in step 2.  One LDS element per point, no padding: step 4 swizzles the
-// position inside a row of N3 by exclusive or with the row.
+// in step 2.  One LDS element per point: step 4 swizzles the
+// position inside a row of N3 by exclusive or with the row; step 2 pads short runs (RegLds).
 #pragma once
 
 #include "jw_device.hpp"
 
 namespace jw {
 
+// In what follows no multiplication is fused with an addition except where it is
+// written out (the same bits wherever a transform is inlined).
+
 // a * e^{DIR 2 pi i k / 16} for the constant twiddles of the 16-point DFT
 template <int DIR, typename C>
 __device__ __forceinline__ C rot16(C a, int k) {
+#pragma clang fp contract(off)
     typedef decltype(a.x) T;
     const T c1 = (T)0.92387953251128675612818318939679, s1 = (T)0.38268343236508977172845998403040;
     const T h = (T)0.70710678118654752440084436210485;
@@ -41,13 +45,40 @@ __device__ __forceinline__ C rot16(C a, int k) {
     }
     const T c = (k == 1) ? c1 : (k == 3) ? s1 : -c1;                       // 1, 3, 9
     const T s = (T)(DIR < 0 ? -1 : 1) * ((k == 1) ? s1 : (k == 3) ? c1 : -s1);
-    return C{a.x * c - a.y * s, a.x * s + a.y * c};
+    return cmul(a, C{c, s});
+}
+
+// 8 points: two 4-point halves; the odd outputs' 1 / sqrt 2 rides on the last additions
+template <int DIR, typename C>
+__device__ __forceinline__ void dft8_reg(C* v) {
+#pragma clang fp contract(off)
+    typedef decltype(v[0].x) T;
+    C e[4] = {v[0], v[2], v[4], v[6]};
+    C o[4] = {v[1], v[3], v[5], v[7]};
+    dft_small<4, DIR>(e);
+    dft_small<4, DIR>(o);
+    const T h = (T)0.70710678118654752440084436210485;
+    // o1 (1 + DIR i), o3 (-1 + DIR i), each to be scaled by h; o2 DIR i
+    const C o1 = DIR < 0 ? C{o[1].x + o[1].y, o[1].y - o[1].x} : C{o[1].x - o[1].y, o[1].y + o[1].x};
+    const C o3 = DIR < 0 ? C{o[3].y - o[3].x, -o[3].y - o[3].x} : C{-o[3].x - o[3].y, o[3].x - o[3].y};
+    const C o2 = rot_q<DIR>(o[2]);
+    v[0] = cadd(e[0], o[0]);
+    v[4] = csub(e[0], o[0]);
+    v[1] = C{fma_t(h, o1.x, e[1].x), fma_t(h, o1.y, e[1].y)};
+    v[5] = C{fma_t(-h, o1.x, e[1].x), fma_t(-h, o1.y, e[1].y)};
+    v[2] = cadd(e[2], o2);
+    v[6] = csub(e[2], o2);
+    v[3] = C{fma_t(h, o3.x, e[3].x), fma_t(h, o3.y, e[3].y)};
+    v[7] = C{fma_t(-h, o3.x, e[3].x), fma_t(-h, o3.y, e[3].y)};
 }
 
 // in-register DFT of R points, natural order in and out
 template <int R, int DIR, typename C>
 __device__ __forceinline__ void dft_reg(C* v) {
-    if constexpr (R <= 8) {
+#pragma clang fp contract(off)
+    if constexpr (R == 8) {
+        dft8_reg<DIR>(v);
+    } else if constexpr (R < 8) {
         if constexpr (R > 1) dft_small<R, DIR>(v);
     } else if constexpr (R == 16) {
         // n = 4 n1 + n2, k = k1 + 4 k2
@@ -87,7 +118,7 @@ __device__ __forceinline__ void dft_reg(C* v) {
                 // e^{DIR 2 pi i k / 32}: cosine and sine of the first quadrant
                 const int q = k & 7;
                 const T c = c32[q], s = (T)(DIR < 0 ? -1 : 1) * c32[8 - q];
-                w = C{w.x * c - w.y * s, w.x * s + w.y * c};
+                w = cmul(w, C{c, s});
             }
             if (k >= 8) w = rot_q<DIR>(w);
             v[k] = cadd(e[k], w);
@@ -100,10 +131,11 @@ __device__ __forceinline__ void dft_reg(C* v) {
 // and 8 points with one more exchange beat 16 with half the waves (loaded column
 // pass, one lattice, FP64 / FP32 us: N = 256 6.7 / 6.2 against 8.1 / 7.2; N = 512 16.0 / 9.4
 // against 20.1 / 11.1; twelve lattices at once are within 8% either way).  From 1024
-// on 16 points need one exchange less; 8192 = 32 * 32 * 8 keeps three factors.
+// on 16 points need one exchange less; 8192 = 32 * 32 * 8 keeps three factors; 64 = 4 * 4 * 4
+// gives the row passes a whole wave per row.
 template <int N>
 struct RegFft {
-    static constexpr int PT = N <= 512 ? 8 : (N <= 4096 ? 16 : 32);
+    static constexpr int PT = N == 64 ? 4 : (N <= 512 ? 8 : (N <= 4096 ? 16 : 32));
     static constexpr int N2 = N / PT;
     static constexpr int N3 = N2 / PT;       // threads of a sub-sequence
     static constexpr int T = N / PT;         // threads of a sequence
@@ -111,51 +143,35 @@ struct RegFft {
     static_assert(N3 >= 1 && N3 <= PT && PT * PT * N3 == N, "register FFT split");
 };
 
-// frequency of v[q] in thread (g, m)
+// frequency of v[q] in thread (g, m): the thread's part and the point's
 template <int N>
-__device__ __forceinline__ int reg_freq(int g, int m, int q) {
+__device__ __forceinline__ constexpr int reg_freq_q(int q) {
     typedef RegFft<N> F;
-    return g + F::PT * (m + F::N3 * (q / F::N3)) + F::PT * F::PT * (q % F::N3);
+    return F::PT * F::N3 * (q / F::N3) + F::PT * F::PT * (q % F::N3);
+}
+template <int N>
+__device__ __forceinline__ constexpr int reg_freq(int g, int m, int q) {
+    return g + RegFft<N>::PT * m + reg_freq_q<N>(q);
 }
 
-// v[k] *= w^k (DIR > 0: conjugate), k = 1 .. PT - 1, from the table entries
-// w, w^2, w^4 (w^8, w^16): at most three (four) products deep
+// v[k] *= w^k (DIR > 0: conjugate), k = 1 .. PT - 1, w = tw[idx]: w^(4 a + b) as the
+// product of two table entries (one rounding more than the table's own)
 template <int PT, int DIR, typename C>
 __device__ __forceinline__ void twiddle_powers(C* v, const C* __restrict__ tw, int idx) {
-    C w[8];
-    w[1] = tw[idx];
-    w[2] = tw[2 * idx];
-    w[4] = tw[4 * idx];
-    C w8, w16;
-    if constexpr (PT >= 16) w8 = tw[8 * idx];
-    if constexpr (PT >= 32) w16 = tw[16 * idx];
-    if (DIR > 0) {
-        w[1].y = -w[1].y;
-        w[2].y = -w[2].y;
-        w[4].y = -w[4].y;
-        if constexpr (PT >= 16) w8.y = -w8.y;
-        if constexpr (PT >= 32) w16.y = -w16.y;
+    C w[4];
+#pragma unroll
+    for (int b = 1; b < 4; b++) {
+        w[b] = tw[b * idx];
+        if (DIR > 0) w[b].y = -w[b].y;
+        v[b] = cmul(v[b], w[b]);
     }
-    w[3] = cmul(w[1], w[2]);
-    w[5] = cmul(w[1], w[4]);
-    w[6] = cmul(w[2], w[4]);
-    w[7] = cmul(w[3], w[4]);
 #pragma unroll
-    for (int k = 1; k < 8; k++) v[k] = cmul(v[k], w[k]);
-    if constexpr (PT >= 16) {
-        v[8] = cmul(v[8], w8);
+    for (int a = 4; a < PT; a += 4) {
+        C wa = tw[a * idx];
+        if (DIR > 0) wa.y = -wa.y;
+        v[a] = cmul(v[a], wa);
 #pragma unroll
-        for (int k = 1; k < 8; k++) v[8 + k] = cmul(v[8 + k], cmul(w8, w[k]));
-    }
-    if constexpr (PT >= 32) {
-        v[16] = cmul(v[16], w16);
-        const C w24 = cmul(w8, w16);
-        v[24] = cmul(v[24], w24);
-#pragma unroll
-        for (int k = 1; k < 8; k++) {
-            v[16 + k] = cmul(v[16 + k], cmul(w16, w[k]));
-            v[24 + k] = cmul(v[24 + k], cmul(w24, w[k]));
-        }
+        for (int b = 1; b < 4; b++) v[a + b] = cmul(v[a + b], cmul(wa, w[b]));
     }
 }
 
@@ -166,13 +182,24 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// steps 1 to 5.  c: the thread's column, j: its index in the sequence.  FIRST: no
-// access of the buffer is pending (otherwise a barrier precedes the writes).
+// elements from one sub-sequence to the next in LDS: where the N3 * W elements that
+// neighbouring lanes read together are less than 128 bytes, one such run of padding
+// moves the next sub-sequence's run to other banks
+template <int N, int W, typename C>
+struct RegLds {
+    static constexpr int RUN = RegFft<N>::N3 * W;
+    static constexpr int SUB = RegFft<N>::N2 * W + (RUN * (int)sizeof(C) < 128 ? RUN : 0);
+    static constexpr int ELEMS = RegFft<N>::PT * SUB;
+};
+
+// steps 1 to 5.  tid = j W + c: the thread's index in its sequence and its column.
+// FIRST: no other wave's access of the buffer is pending (otherwise a barrier
+// precedes the writes).
 template <int N, int W, bool FIRST, typename C>
 __device__ __forceinline__ void reg_fft_fwd(C* v, C* lds, const C* __restrict__ tw, int tid) {
     const int j = tid / W, c = tid % W;
     typedef RegFft<N> F;
-    constexpr int PT = F::PT, N2 = F::N2, N3 = F::N3, NU = F::NU;
+    constexpr int PT = F::PT, N3 = F::N3, NU = F::NU, SUB = RegLds<N, W, C>::SUB;
     static_assert(N3 * W <= 64, "a sub-sequence sits in one wave");
     dft_reg<PT, -1>(v);
     __builtin_amdgcn_sched_barrier(0);
@@ -181,12 +208,12 @@ __device__ __forceinline__ void reg_fft_fwd(C* v, C* lds, const C* __restrict__ 
     {
         C* p = lds + j * W + c;
 #pragma unroll
-        for (int k = 0; k < PT; k++) p[k * N2 * W] = v[k];
+        for (int k = 0; k < PT; k++) p[k * SUB] = v[k];
     }
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     const int g = j / N3, m = j % N3;
-    C* sub = lds + g * N2 * W + c;
+    C* sub = lds + g * SUB + c;
 #pragma unroll
     for (int a = 0; a < PT; a++) v[a] = sub[(m + N3 * a) * W];
     dft_reg<PT, -1>(v);
@@ -211,10 +238,10 @@ template <int N, int W, bool FIRST, typename C>
 __device__ __forceinline__ void reg_fft_inv(C* v, C* lds, const C* __restrict__ tw, int tid) {
     const int j = tid / W, c = tid % W;
     typedef RegFft<N> F;
-    constexpr int PT = F::PT, N2 = F::N2, N3 = F::N3, NU = F::NU;
+    constexpr int PT = F::PT, N3 = F::N3, NU = F::NU, SUB = RegLds<N, W, C>::SUB;
     static_assert(N3 * W <= 64, "a sub-sequence sits in one wave");
     const int g = j / N3, m = j % N3;
-    C* sub = lds + g * N2 * W + c;
+    C* sub = lds + g * SUB + c;
     if (!FIRST) __syncthreads();
     if constexpr (N3 > 1) {
 #pragma unroll
@@ -236,7 +263,7 @@ __device__ __forceinline__ void reg_fft_inv(C* v, C* lds, const C* __restrict__ 
     {
         const C* p = lds + j * W + c;
 #pragma unroll
-        for (int k = 0; k < PT; k++) v[k] = p[k * N2 * W];
+        for (int k = 0; k < PT; k++) v[k] = p[k * SUB];
     }
     twiddle_powers<PT, +1>(v, tw, j);
     dft_reg<PT, +1>(v);

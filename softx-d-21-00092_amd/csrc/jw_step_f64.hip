@@ -26,6 +26,23 @@ hipError_t block16(jw_ctx* c, double* out, const double* in) {
     return hipGetLastError();
 }
 
+// sqrt(alpha) with its columns in the order of the row-major row spectra
+template <int N>
+__global__ __launch_bounds__(256) void k_perm_columns(double* __restrict__ out, const double* __restrict__ in) {
+    GRID_STRIDE(i, (size_t)N * N) out[i] = in[i / N * N + freq_of_pos<N, 0>((int)(i % N))];
+}
+
+hipError_t perm_columns(jw_ctx* c, double* out, const double* in) {
+#define JW_PERM(n, C) \
+    case n: hipLaunchKernelGGL(k_perm_columns<n>, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, out, in); break;
+    switch (c->N) {
+        JW_FUSED_SIZES(JW_PERM, cplx)
+        default: return hipErrorInvalidValue;
+    }
+#undef JW_PERM
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // U between the FP64 field (9 planes) and the FP32 state of the mixed-precision
 // form: 9 planes, or rows 0 and 1 (6 planes, the fused and large-lattice passes) with row 2
@@ -39,15 +56,12 @@ __global__ __launch_bounds__(256) void k_u_to_f64(cplx* __restrict__ out, const 
 }
 __global__ __launch_bounds__(256) void k_u2_to_f64(cplx* __restrict__ out, const cplxf* __restrict__ in, size_t V) {
     GRID_STRIDE(i, V) {
-        cplx m[6];
+        cplx m[9];
 #pragma unroll
-        for (int k = 0; k < 6; k++) {
-            m[k] = to_d(in[k * V + i]);
-            out[k * V + i] = m[k];
-        }
-        out[6 * V + i] = conjg(csub(cmul(m[1], m[5]), cmul(m[2], m[4])));
-        out[7 * V + i] = conjg(csub(cmul(m[2], m[3]), cmul(m[0], m[5])));
-        out[8 * V + i] = conjg(csub(cmul(m[0], m[4]), cmul(m[1], m[3])));
+        for (int k = 0; k < 6; k++) m[k] = to_d(in[k * V + i]);
+        row2_of(m);
+#pragma unroll
+        for (int k = 0; k < 9; k++) out[k * V + i] = m[k];
     }
 }
 
@@ -55,12 +69,12 @@ __global__ __launch_bounds__(256) void k_u2_to_f64(cplx* __restrict__ out, const
 // which keep only those rows current)
 __global__ __launch_bounds__(256) void k_u_rebuild(cplx* __restrict__ U, size_t V) {
     GRID_STRIDE(i, V) {
-        cplx m[6];
+        cplx m[9];
 #pragma unroll
         for (int k = 0; k < 6; k++) m[k] = U[k * V + i];
-        U[6 * V + i] = conjg(csub(cmul(m[1], m[5]), cmul(m[2], m[4])));
-        U[7 * V + i] = conjg(csub(cmul(m[2], m[3]), cmul(m[0], m[5])));
-        U[8 * V + i] = conjg(csub(cmul(m[0], m[4]), cmul(m[1], m[3])));
+        row2_of(m);
+#pragma unroll
+        for (int k = 6; k < 9; k++) U[k * V + i] = m[k];
     }
 }
 
