@@ -1130,7 +1130,6 @@ int jw_mv_init(jw_ctx* c, jw_field* U, int Ny, double g, double mu, double mass,
     if (Ny < 1) return fail(JW_ERR_ARG, "Ny must be >= 1");
     if (int e = ensure_ws(c, 24)) return e;
     cplx* R = c->ws;
-    HIP_CHECK(jw::set_unit(c, U->d));
     const double sigma = g * mu / sqrt((double)Ny);
     const double m = mass * pow(g, 2.0) * mu;
     for (int s = 0; s < Ny; s++) {
@@ -1140,11 +1139,7 @@ int jw_mv_init(jw_ctx* c, jw_field* U, int Ny, double g, double mu, double mass,
             ns.inj = c->inj;
             c->inj_per_site = 0;
         }
-        HIP_CHECK(jw::mv_noise_packed(c, R, ns, sigma));
-        HIP_CHECK(jw::fft2d(c, R, 4, 1, 1.0 / c->N));
-        HIP_CHECK(jw::poisson_packed(c, R, m, g));
-        HIP_CHECK(jw::fft2d(c, R, 4, 0, 1.0 / c->N));
-        HIP_CHECK(jw::mul_exp_packed(c, U->d, R));
+        HIP_CHECK(jw::mv_sheet(c, U->d, R, ns, sigma, m, g, s == 0, s == Ny - 1));
     }
     return JW_OK;
 }

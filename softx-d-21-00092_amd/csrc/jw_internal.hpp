@@ -127,9 +127,8 @@ hipError_t step_unfused(jw_ctx* c, cplx* U, cplx* Xi, cplx* Vv, cplx* ZA, cplx* 
                         const double* sa_pos, const double* sa_k, int kc, int corr, double ss);
 hipError_t step_unfused_f32(jw_ctx* c, cplxf* U, cplxf* Xi, cplxf* Vv, cplxf* ZA, cplxf* ZB, const NoiseSrc& ns,
                             const double* sa_pos, const double* sa_k, int kc, int corr, double ss, int reunit);
-hipError_t mv_noise_packed(jw_ctx* c, cplx* R, const NoiseSrc& ns, double sigma);
-hipError_t poisson_packed(jw_ctx* c, cplx* R, double mass, double g);
-hipError_t mul_exp_packed(jw_ctx* c, cplx* U, const cplx* R);
+// one MV sheet: U <- U exp(i A_s), from U = 1 on the first; U is whole after the last
+hipError_t mv_sheet(jw_ctx* c, cplx* U, cplx* R, const NoiseSrc& ns, double sigma, double mass, double g, int first, int last);
 
 // fused generator-basis step (64 <= N <= 2048), FP64 or FP32 storage
 bool fused_supported(int N);

@@ -459,13 +459,13 @@ __global__ __launch_bounds__(256) void k_mv_noise_packed(cplx* __restrict__ R, s
     }
 }
 
-hipError_t mv_noise_packed(jw_ctx* c, cplx* R, const NoiseSrc& ns, double sigma) {
+static hipError_t mv_noise_packed(jw_ctx* c, cplx* R, const NoiseSrc& ns, double sigma) {
     KTimer t(c, K_MV);
     hipLaunchKernelGGL(k_mv_noise_packed, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, R, c->V, ns, sigma);
     return hipGetLastError();
 }
 
-hipError_t poisson_packed(jw_ctx* c, cplx* R, double mass, double g) { return solve_poisson(c, R, 4, mass, g); }
+static hipError_t poisson_packed(jw_ctx* c, cplx* R, double mass, double g) { return solve_poisson(c, R, 4, mass, g); }
 
 __global__ __launch_bounds__(256) void k_mul_exp_packed(cplx* __restrict__ U, const cplx* __restrict__ R, size_t V) {
     GRID_STRIDE(i, V) {
@@ -476,10 +476,146 @@ __global__ __launch_bounds__(256) void k_mul_exp_packed(cplx* __restrict__ U, co
     }
 }
 
-hipError_t mul_exp_packed(jw_ctx* c, cplx* U, const cplx* R) {
+static hipError_t mul_exp_packed(jw_ctx* c, cplx* U, const cplx* R) {
     KTimer t(c, K_MV);
     hipLaunchKernelGGL(k_mul_exp_packed, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, U, R, c->V);
     return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// MV sheets, 64 <= N <= 2048, in three passes of the fused step's make (jw_engine.hpp,
+// jw_regfft.hpp) instead of noise, row and column transforms, Poisson, two transforms
+// back and the exponential (28 complex planes moved a sheet instead of 70):
+//   k_mv_noise_row : charges drawn in registers, forward row FFT              W 4
+//   k_mv_col       : column FFT, -g / (-phat2 + m^2), inverse column FFT       R 4 W 4
+//   k_mv_row_exp   : inverse row FFT, U <- U exp(i A)                           R 10 W 6
+// (U as rows 0 and 1; the first sheet reads no U, the last writes all nine
+// entries.)  Bound by memory but for the charges, whose logarithms and sines are.
+// N = 1024: 222 -> 125 us a sheet.
+// ---------------------------------------------------------------------------
+template <int N>
+__global__ __launch_bounds__(RowN<N>::NT, 2) void k_mv_noise_row(cplx* __restrict__ R, size_t V, NoiseSrc ns, double sigma,
+                                                                const cplx* __restrict__ tw) {
+    constexpr int PT = RegFft<N>::PT, T = RegFft<N>::T;
+    __shared__ cplx lds[RowN<N>::RPW * RowT<N, cplx>::PL];
+    const int x = blockIdx.x * RowN<N>::RPW + threadIdx.x / T, p = blockIdx.y;
+    const int j = opaque_v((int)threadIdx.x % T);
+    const unsigned row0 = (unsigned)x * N;
+    cplx a[PT];
+#pragma unroll
+    for (int r = 0; r < PT; r++) {
+        const unsigned i = row0 + j + r * T;
+        if (ns.inj) {
+            a[r] = reinterpret_cast<const double2*>(ns.inj + 8 * (size_t)i)[p];
+        } else {
+            box_muller_pair(i, ns.step, ns.tag, (uint32_t)p, ns.seed, ns.traj, a[r].x, a[r].y);
+        }
+        a[r] = cscale(a[r], sigma);
+        fence(a[r]);
+    }
+    reg_fft_fwd<N, 1, true>(a, lds + (threadIdx.x / T) * RowT<N, cplx>::PL, tw_fft(tw), opaque_v((int)threadIdx.x % T));
+    const int k0 = pos0<N, 0>(opaque_v((int)threadIdx.x % T));
+#pragma unroll
+    for (int q = 0; q < PT; q++) R[pat<N, 0>(p, x, k0 + posq<N, 0>(q), V)] = a[q];
+}
+
+template <int N>
+__global__ __launch_bounds__((ColR<N, cplx>::NT), (ColR<N, cplx>::WAVES)) void k_mv_col(cplx* __restrict__ R, size_t V,
+                                                                                       const double* __restrict__ q4,
+                                                                                       double mass, double g, int zero_mode,
+                                                                                       const cplx* __restrict__ tw) {
+    typedef RegFft<N> F;
+    constexpr int PT = F::PT, W = ColR<N, cplx>::W;
+    constexpr size_t RS = (size_t)F::T * N;
+    __shared__ cplx lds[ColR<N, cplx>::ELEMS];
+    const int col0 = xcd_strip(blockIdx.x, N / W) * W;
+    R += (size_t)blockIdx.y * V;
+    const unsigned o = (unsigned)((int)(threadIdx.x / W) * N + col0 + (int)threadIdx.x % W);
+    cplx v[PT];
+#pragma unroll
+    for (int r = 0; r < PT; r++) v[r] = (R + r * RS)[o];
+    reg_fft_fwd<N, W, true>(v, lds, tw_fft(tw), opaque_v((int)threadIdx.x));
+    const int t = after((int)threadIdx.x, v[PT - 1].x);
+    const int j = t / W, ky = freq_of_pos<N, 0>(col0 + t % W);
+    const int kx0 = reg_freq<N>(j / F::N3, j % F::N3, 0);
+    const double q4y = q4[ky], num = -1.0 * g * (1.0 / ((double)N * (double)N));
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+        const double f = num / (-((q4 + reg_freq_q<N>(q))[kx0] + q4y) + mass * mass);
+        v[q] = zero_mode && q == 0 && kx0 == 0 && ky == 0 ? mk(0.0, 0.0) : cscale(v[q], f);
+    }
+    reg_fft_inv<N, W, true>(v, lds, tw_fft(tw), opaque_v((int)threadIdx.x));
+#pragma unroll
+    for (int r = 0; r < PT; r++) (R + r * RS)[o] = v[r];
+}
+
+template <int N>
+__global__ __launch_bounds__(RowE<N>::NT, 2) void k_mv_row_exp(cplx* __restrict__ U, const cplx* __restrict__ R, size_t V,
+                                                              int first, int last, const cplx* __restrict__ tw) {
+    constexpr int NT = RowE<N>::NT, SPT = RowE<N>::SPT, PL = RowT<N, cplx>::PL;
+    __shared__ cplx lds[4 * PL];
+    const int tid = threadIdx.x, x = blockIdx.x;
+    const size_t row0 = (size_t)x * N;
+    cplx a[RowE<N>::PT];
+    row_load<N, 0>(a, tid, [&](int p, int k) { return R[pat<N, 0>(p, x, k, V)]; });
+    row_inv<N, true>(a, lds, tw, tid);
+    __syncthreads();
+#pragma unroll 1
+    for (int q = 0; q < SPT; q++) {
+        const int y = tid + q * NT;
+        const size_t i = row0 + y;
+        double h[8];
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const cplx b = lds[p * PL + row_slot_of<N, cplx>(y)];
+            h[2 * p] = b.x;
+            h[2 * p + 1] = b.y;
+        }
+        m3 e = exp_i_gen(h, 1.0);
+        if (!first) {
+            m3 u;
+            load_u(u, U, V, i);
+            e = mmul(u, e);
+        }
+        if (last) store9(U, V, i, e);
+        else store_u(U, V, i, e);
+    }
+}
+
+template <int N>
+static hipError_t mv_sheet_n(jw_ctx* c, cplx* U, cplx* R, const NoiseSrc& ns, double sigma, double mass, double g, int first,
+                             int last) {
+    KTimer t(c, K_MV);
+    const size_t V = c->V;
+    hipError_t e;
+    hipLaunchKernelGGL(k_mv_noise_row<N>, dim3(N / RowN<N>::RPW, 4), dim3(RowN<N>::NT), 0, c->stream, R, V, ns, sigma, c->tw);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_mv_col<N>, dim3(N / ColR<N, cplx>::W, 4), dim3(ColR<N, cplx>::NT), 0, c->stream, R, V, c->q4, mass, g,
+                       c->mv_zero_mode, c->tw);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_mv_row_exp<N>, dim3(N), dim3(RowE<N>::NT), 0, c->stream, U, R, V, first, last, c->tw);
+    return hipGetLastError();
+}
+
+// one sheet on the planes R (four): the fused passes for 64 <= N <= 2048, else the
+// separate ones (the first sheet starts from U = 1)
+hipError_t mv_sheet(jw_ctx* c, cplx* U, cplx* R, const NoiseSrc& ns, double sigma, double mass, double g, int first, int last) {
+#define JW_MV(n, C) case n: return mv_sheet_n<n>(c, U, R, ns, sigma, mass, g, first, last);
+    switch (c->N) {
+        JW_FUSED_SIZES(JW_MV, cplx)
+        default: break;
+    }
+#undef JW_MV
+    hipError_t e;
+#define JW_TRY(x) if ((e = (x)) != hipSuccess) return e
+    if (first) JW_TRY(set_unit(c, U));
+    JW_TRY(mv_noise_packed(c, R, ns, sigma));
+    JW_TRY(fft2d(c, R, 4, 1, 1.0 / c->N));
+    JW_TRY(poisson_packed(c, R, mass, g));
+    JW_TRY(fft2d(c, R, 4, 0, 1.0 / c->N));
+    JW_TRY(mul_exp_packed(c, U, R));
+#undef JW_TRY
+    return hipSuccess;
 }
 
 // ===========================================================================
