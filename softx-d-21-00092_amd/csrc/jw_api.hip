@@ -1,4 +1,5 @@
 // jw_api.hip -- the C ABI declared in include/jimwlk.h.
+#include "jw_host.hpp"
 #include "jw_internal.hpp"
 
 #include <math.h>
@@ -633,6 +634,7 @@ void jw_destroy(jw_ctx* c) {
     if (c->sa16) hipFree(c->sa16);
     if (c->sap) hipFree(c->sap);
     if (c->inj) hipFree(c->inj);
+    jw::lanes_free(c);
     if (c->ws) hipFree(c->ws);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
@@ -670,27 +672,21 @@ void jw_field_destroy(jw_field* f) {
 int jw_field_upload(jw_field* f, const double* h) {
     if (!f || !h) return fail(JW_ERR_ARG, "null argument");
     jw_ctx* c = f->ctx;
-    const size_t V = c->V;
-    std::vector<cplx> soa(f->t * V);
-    for (size_t i = 0; i < V; i++)
-        for (int k = 0; k < f->t; k++) soa[k * V + i] = make_double2(h[2 * (i * f->t + k)], h[2 * (i * f->t + k) + 1]);
-    HIP_CHECK(hipMemcpyAsync(f->d, soa.data(), soa.size() * sizeof(cplx), hipMemcpyHostToDevice, c->stream));
-    HIP_CHECK(hipStreamSynchronize(c->stream));
+    const hipError_t e = jw::host_transfer(c, const_cast<double*>(h), c->V, f->t * sizeof(cplx), false,
+                                           [&](void* pin, size_t s0, size_t n) {
+                                               return jw::aos_to_planes(c, f->d, static_cast<cplx*>(pin), f->t, s0, n);
+                                           });
+    HIP_CHECK(e);
     return JW_OK;
 }
 
 int jw_field_download(const jw_field* f, double* h) {
     if (!f || !h) return fail(JW_ERR_ARG, "null argument");
     jw_ctx* c = f->ctx;
-    const size_t V = c->V;
-    std::vector<cplx> soa(f->t * V);
-    HIP_CHECK(hipMemcpyAsync(soa.data(), f->d, soa.size() * sizeof(cplx), hipMemcpyDeviceToHost, c->stream));
-    HIP_CHECK(hipStreamSynchronize(c->stream));
-    for (size_t i = 0; i < V; i++)
-        for (int k = 0; k < f->t; k++) {
-            h[2 * (i * f->t + k)] = soa[k * V + i].x;
-            h[2 * (i * f->t + k) + 1] = soa[k * V + i].y;
-        }
+    const hipError_t e = jw::host_transfer(c, h, c->V, f->t * sizeof(cplx), true, [&](void* pin, size_t s0, size_t n) {
+        return jw::planes_to_aos(c, static_cast<cplx*>(pin), f->d, f->t, s0, n);
+    });
+    HIP_CHECK(e);
     return JW_OK;
 }
 

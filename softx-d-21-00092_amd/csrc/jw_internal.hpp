@@ -17,6 +17,9 @@
 #define JW_TAG_MV 0x4D565348u         // 'MVSH'
 #define JW_TAG_KSPACE 0x4B535043u     // 'KSPC': momentum-space Langevin noise
 
+// host transfers: staging buffers (and host threads) a context uses at once
+#define JW_LANES 4
+
 namespace jw {
 
 typedef double2 cplx;
@@ -69,6 +72,11 @@ struct jw_ctx {
     int inj_per_site;      // 0 when no injection is pending
     // Philox stream state for the generators
     uint32_t seed, traj, step;
+    // pinned staging of the host transfers (jw_host.hpp): up to JW_LANES buffers of
+    // lane_cap bytes, allocated on first use, freed with the context
+    void* lane_pin[JW_LANES];
+    hipEvent_t lane_ev[JW_LANES];
+    size_t lane_cap;
     // workspace: generator-basis planes (packed) and scratch complex planes
     jw::cplx* ws;
     size_t ws_planes;
@@ -177,6 +185,11 @@ hipError_t perm_columns(jw_ctx* c, double* out, const double* in);
 // observables
 hipError_t corr_from_Uk(jw_ctx* c, const cplx* Uk, double* corr);
 hipError_t accumulate_real(jw_ctx* c, const double* corr, double* sum, double* err);
+
+// sites s0 .. s0 + n - 1 of a field of t planes to / from the reference's AoS order
+// (aos: element (s - s0) t + k, device-visible host memory)
+hipError_t planes_to_aos(jw_ctx* c, cplx* aos, const cplx* planes, int t, size_t s0, size_t n);
+hipError_t aos_to_planes(jw_ctx* c, cplx* planes, const cplx* aos, int t, size_t s0, size_t n);
 
 // instrumentation and unit-test hooks
 hipError_t calibration_copy(jw_ctx* c, const cplx* a, cplx* b, size_t n);

@@ -33,6 +33,38 @@ hipError_t fft2d(jw_ctx* c, cplx* planes, int nplanes, int dir, double scale) {
 }
 
 // ===========================================================================
+// host transfers: field planes <-> the reference's AoS order, on pinned host memory
+// (consecutive lanes touch consecutive 16-byte words of it: whole bus transactions; bound
+// by the bus)
+// ===========================================================================
+template <int T>
+__global__ __launch_bounds__(256) void k_planes_to_aos(cplx* __restrict__ aos, const cplx* __restrict__ f, size_t V, size_t s0,
+                                                       size_t n) {
+    GRID_STRIDE(e, n * T) aos[e] = f[(e % T) * V + s0 + e / T];
+}
+template <int T>
+__global__ __launch_bounds__(256) void k_aos_to_planes(cplx* __restrict__ f, const cplx* __restrict__ aos, size_t V, size_t s0,
+                                                       size_t n) {
+    GRID_STRIDE(e, n * T) f[(e % T) * V + s0 + e / T] = aos[e];
+}
+
+hipError_t planes_to_aos(jw_ctx* c, cplx* aos, const cplx* f, int t, size_t s0, size_t n) {
+    const dim3 g(grid_for(n * t, 256)), b(256);
+    if (t == 9) hipLaunchKernelGGL(k_planes_to_aos<9>, g, b, 0, c->stream, aos, f, c->V, s0, n);
+    else if (t == 1) hipLaunchKernelGGL(k_planes_to_aos<1>, g, b, 0, c->stream, aos, f, c->V, s0, n);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t aos_to_planes(jw_ctx* c, cplx* f, const cplx* aos, int t, size_t s0, size_t n) {
+    const dim3 g(grid_for(n * t, 256)), b(256);
+    if (t == 9) hipLaunchKernelGGL(k_aos_to_planes<9>, g, b, 0, c->stream, f, aos, c->V, s0, n);
+    else if (t == 1) hipLaunchKernelGGL(k_aos_to_planes<1>, g, b, 0, c->stream, f, aos, c->V, s0, n);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// ===========================================================================
 // tables
 // ===========================================================================
 // variant 0: sqrt(alpha) with prepare_A_local's operation order (field.h:2045-2046)

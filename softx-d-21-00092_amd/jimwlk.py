@@ -141,7 +141,7 @@ class Field:
         return self
 
     def download(self):
-        a = np.zeros((self.ctx.V, self.t), np.complex128)
+        a = np.empty((self.ctx.V, self.t), np.complex128)      # written whole by the library
         _check(lib().jw_field_download(self.h, _p(a)))
         return a
 
