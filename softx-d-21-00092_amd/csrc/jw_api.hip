@@ -1145,33 +1145,31 @@ int jw_measure_corr(jw_ctx* c, const jw_field* U, double* host_corr) {
     if (int e = check_field(U, c, 9, "U")) return e;
     if (!host_corr) return fail(JW_ERR_ARG, "null output");
     if (int e = ensure_ws(c, 24)) return e;
-    const size_t V = c->V;
-    cplx* Uk = c->ws;
-    cplx* tr = Uk + 9 * V;
-    cplx* sym = tr + V;
-    HIP_CHECK(hipMemcpyAsync(Uk, U->d, 9 * V * sizeof(cplx), hipMemcpyDeviceToDevice, c->stream));
-    HIP_CHECK(jw::fft2d(c, Uk, 9, 1, 1.0 / c->N));
-    HIP_CHECK(jw::trace(c, Uk, tr));
-    HIP_CHECK(jw::average_and_symmetrize(c, tr, sym));
-    std::vector<cplx> h(V);
-    HIP_CHECK(hipMemcpyAsync(h.data(), sym, V * sizeof(cplx), hipMemcpyDeviceToHost, c->stream));
-    HIP_CHECK(hipStreamSynchronize(c->stream));
-    for (size_t i = 0; i < V; i++) host_corr[i] = h[i].x;
+    cplx* planes = c->ws;
+    double* corr = reinterpret_cast<double*>(planes + 9 * c->V);
+    HIP_CHECK(jw::correlator(c, U->d, planes, corr));
+    // symmetrised on the way into the caller's memory
+    const hipError_t e = jw::host_transfer(c, host_corr, c->V, sizeof(double), true, [&](void* pin, size_t s0, size_t n) {
+        return jw::symmetrize_real(c, corr, static_cast<double*>(pin), s0, n);
+    });
+    HIP_CHECK(e);
     return JW_OK;
 }
 
 int jw_dipole_from_corr(jw_ctx* c, const double* host_corr, double* host_S) {
     if (!c || !host_corr || !host_S) return fail(JW_ERR_ARG, "null argument");
     if (int e = ensure_ws(c, 24)) return e;
-    const size_t V = c->V;
-    std::vector<cplx> h(V);
-    for (size_t i = 0; i < V; i++) h[i] = make_double2(host_corr[i], 0.0);
-    HIP_CHECK(hipMemcpyAsync(c->ws, h.data(), V * sizeof(cplx), hipMemcpyHostToDevice, c->stream));
+    hipError_t e = jw::host_transfer(c, const_cast<double*>(host_corr), c->V, sizeof(double), false,
+                                     [&](void* pin, size_t s0, size_t n) {
+                                         return jw::plane_from_real(c, c->ws + s0, static_cast<double*>(pin), n);
+                                     });
+    HIP_CHECK(e);
     HIP_CHECK(jw::fft2d(c, c->ws, 1, 0, 1.0));
-    HIP_CHECK(hipMemcpyAsync(h.data(), c->ws, V * sizeof(cplx), hipMemcpyDeviceToHost, c->stream));
-    HIP_CHECK(hipStreamSynchronize(c->stream));
-    const double f = (double)V / 3.0;
-    for (size_t i = 0; i < V; i++) host_S[i] = f * h[i].x;
+    const double f = (double)c->V / 3.0;
+    e = jw::host_transfer(c, host_S, c->V, sizeof(double), true, [&](void* pin, size_t s0, size_t n) {
+        return jw::real_from_plane(c, static_cast<double*>(pin), c->ws + s0, n, f);
+    });
+    HIP_CHECK(e);
     return JW_OK;
 }
 

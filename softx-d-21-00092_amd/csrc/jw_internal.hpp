@@ -183,7 +183,11 @@ hipError_t block16(jw_ctx* c, double* out, const double* in);
 hipError_t perm_columns(jw_ctx* c, double* out, const double* in);
 
 // observables
-hipError_t corr_from_Uk(jw_ctx* c, const cplx* Uk, double* corr);
+// corr (V reals) = tr[(F U / V)(F U / V)^dagger], planes: nine of workspace
+hipError_t correlator(jw_ctx* c, const cplx* U, cplx* planes, double* corr);
+hipError_t symmetrize_real(jw_ctx* c, const double* in, double* out, size_t s0, size_t n);
+hipError_t plane_from_real(jw_ctx* c, cplx* f, const double* in, size_t n);
+hipError_t real_from_plane(jw_ctx* c, double* out, const cplx* f, size_t n, double s);
 hipError_t accumulate_real(jw_ctx* c, const double* corr, double* sum, double* err);
 
 // sites s0 .. s0 + n - 1 of a field of t planes to / from the reference's AoS order

@@ -314,14 +314,140 @@ hipError_t trace(jw_ctx* c, const cplx* U, cplx* corr) {
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// tr[(F U / V)(F U / V)^dagger] over the lattice as reals: forward row transforms of
+// the nine planes of U out of place (R 9 W 9), then the nine column transforms of a
+// strip with the trace summed in registers (R 9 W 1/2), in trace_site's order of sums.
+// Against the copy of U, two in-place transforms and the trace as passes of their own
+// (R 36 W 28): N = 1024 60 + 65 us against 53 + 63 + 24 and the copy.  64 <= N <= 2048; others
+// take those passes.
+// ---------------------------------------------------------------------------
+template <int N>
+__global__ __launch_bounds__(RowN<N>::NT, 2) void k_corr_rows(cplx* __restrict__ out, const cplx* __restrict__ U, size_t V,
+                                                             const cplx* __restrict__ tw) {
+    constexpr int PT = RegFft<N>::PT, T = RegFft<N>::T;
+    __shared__ cplx lds[RowN<N>::RPW * RowT<N, cplx>::PL];
+    const int x = blockIdx.x * RowN<N>::RPW + threadIdx.x / T, j = threadIdx.x % T;
+    const size_t row = (size_t)blockIdx.y * V + (size_t)x * N;
+    cplx v[PT];
+#pragma unroll
+    for (int r = 0; r < PT; r++) v[r] = U[row + j + r * T];
+    reg_fft_fwd<N, 1, true>(v, lds + (threadIdx.x / T) * RowT<N, cplx>::PL, tw_fft(tw), opaque_v(j));
+    const int k0 = pos0<N, 0>(opaque_v(j));
+#pragma unroll
+    for (int q = 0; q < PT; q++) out[row + k0 + posq<N, 0>(q)] = v[q];
+}
+
+template <int N>
+__global__ __launch_bounds__((ColR<N, cplx>::NT), (ColR<N, cplx>::WAVES)) void k_corr_cols(double* __restrict__ corr,
+                                                                                          const cplx* __restrict__ R, size_t V,
+                                                                                          const cplx* __restrict__ tw) {
+#pragma clang fp contract(off)
+    typedef RegFft<N> F;
+    constexpr int PT = F::PT, W = ColR<N, cplx>::W;
+    constexpr size_t RS = (size_t)F::T * N;
+    __shared__ cplx lds[ColR<N, cplx>::ELEMS];
+    const int col0 = xcd_strip(blockIdx.x, N / W) * W;
+    const unsigned o = (unsigned)((int)(threadIdx.x / W) * N + col0 + (int)threadIdx.x % W);
+    double sum[PT], diag[PT];
+    // 1 / (N V): the unitary transform and the trace's division by V, a power of two
+    const double s = 1.0 / ((double)N * (double)N * (double)N);
+    // the next plane in flight under a transform where the registers allow it (small
+    // lattices: few workgroups, latency)
+    constexpr bool AHEAD = PT <= 8;
+    cplx v[PT], w[AHEAD ? PT : 1];
+    auto load = [&](cplx* d, int k) {
+#pragma unroll
+        for (int r = 0; r < PT; r++) d[r] = (R + k * V + r * RS)[o];
+    };
+    if constexpr (AHEAD) load(w, 0);
+#pragma unroll 1
+    for (int k = 0; k < 9; k++) {
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int r = 0; r < PT; r++) v[r] = w[r];
+            if (k < 8) load(w, k + 1);
+        } else {
+            load(v, k);
+        }
+        reg_fft_fwd<N, W, false>(v, lds, tw_fft(tw), opaque_v((int)threadIdx.x));
+#pragma unroll
+        for (int q = 0; q < PT; q++) {
+            const double ax = v[q].x * s, ay = v[q].y * s, e = ax * ax + ay * ay;
+            diag[q] = k % 3 == 0 ? e : diag[q] + e;
+            if (k == 2) sum[q] = diag[q];
+            if (k == 5 || k == 8) sum[q] = sum[q] + diag[q];
+        }
+    }
+    const int j = threadIdx.x / W, ky = freq_of_pos<N, 0>(col0 + (int)threadIdx.x % W);
+    const int kx0 = reg_freq<N>(j / F::N3, j % F::N3, 0);
+#pragma unroll
+    for (int q = 0; q < PT; q++) corr[(size_t)(kx0 + reg_freq_q<N>(q)) * N + ky] = sum[q];
+}
+
+template <int N>
+static hipError_t corr_n(jw_ctx* c, const cplx* U, cplx* planes, double* corr) {
+    KTimer t(c, K_OBS);
+    hipLaunchKernelGGL(k_corr_rows<N>, dim3(N / RowN<N>::RPW, 9), dim3(RowN<N>::NT), 0, c->stream, planes, U, c->V, c->tw);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_corr_cols<N>, dim3(N / ColR<N, cplx>::W), dim3(ColR<N, cplx>::NT), 0, c->stream, corr, planes, c->V,
+                       c->tw);
+    return hipGetLastError();
+}
+
 __global__ __launch_bounds__(256) void k_corr_from_Uk(const cplx* __restrict__ U, double* __restrict__ corr, size_t V, double vol) {
     GRID_STRIDE(i, V) corr[i] = trace_site(U, V, i, vol);
 }
 
-hipError_t corr_from_Uk(jw_ctx* c, const cplx* Uk, double* corr) {
+hipError_t correlator(jw_ctx* c, const cplx* U, cplx* planes, double* corr) {
+#define JW_CORR(n, C) case n: return corr_n<n>(c, U, planes, corr);
+    switch (c->N) {
+        JW_FUSED_SIZES(JW_CORR, cplx)
+        default: break;
+    }
+#undef JW_CORR
+    hipError_t e = hipMemcpyAsync(planes, U, 9 * c->V * sizeof(cplx), hipMemcpyDeviceToDevice, c->stream);
+    if (e != hipSuccess) return e;
+    if ((e = fft2d(c, planes, 9, 1, 1.0 / c->N)) != hipSuccess) return e;
     KTimer t(c, K_OBS);
-    hipLaunchKernelGGL(k_corr_from_Uk, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, Uk, corr, c->V,
-                       1.0 * c->N * c->N);
+    hipLaunchKernelGGL(k_corr_from_Uk, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, planes, corr, c->V, 1.0 * c->N * c->N);
+    return hipGetLastError();
+}
+
+// average_and_symmetrize on reals, sites s0 .. s0 + n - 1 into host memory (same operations)
+__global__ __launch_bounds__(256) void k_symmetrize_real(const double* __restrict__ in, double* __restrict__ out, int N, size_t s0,
+                                                         size_t n) {
+#pragma clang fp contract(off)
+    GRID_STRIDE(e, n) {
+        const size_t idx = s0 + e;
+        const int i = (int)(idx / N), j = (int)(idx % N);
+        const int a = (N - i) % N, b = (N - j) % N;
+        auto tmp = [&](int x, int y) { return 0.5 * (in[(size_t)x * N + y] + in[(size_t)y * N + x]); };
+        const double t1 = tmp(i, j), t2 = tmp(a, j), t3 = tmp(i, b), t4 = tmp(a, b);
+        out[e] = 0.25 * (((t1 + t2) + t3) + t4);
+    }
+}
+
+hipError_t symmetrize_real(jw_ctx* c, const double* in, double* out, size_t s0, size_t n) {
+    KTimer t(c, K_OBS);
+    hipLaunchKernelGGL(k_symmetrize_real, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, in, out, c->N, s0, n);
+    return hipGetLastError();
+}
+
+// reals to a complex plane, and the real part of one, scaled, back
+__global__ __launch_bounds__(256) void k_plane_from_real(cplx* __restrict__ f, const double* __restrict__ in, size_t n) {
+    GRID_STRIDE(i, n) f[i] = mk(in[i], 0.0);
+}
+__global__ __launch_bounds__(256) void k_real_from_plane(double* __restrict__ out, const cplx* __restrict__ f, size_t n, double s) {
+    GRID_STRIDE(i, n) out[i] = s * f[i].x;
+}
+hipError_t plane_from_real(jw_ctx* c, cplx* f, const double* in, size_t n) {
+    hipLaunchKernelGGL(k_plane_from_real, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, f, in, n);
+    return hipGetLastError();
+}
+hipError_t real_from_plane(jw_ctx* c, double* out, const cplx* f, size_t n, double s) {
+    hipLaunchKernelGGL(k_real_from_plane, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, out, f, n, s);
     return hipGetLastError();
 }
 

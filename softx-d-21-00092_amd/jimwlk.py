@@ -292,13 +292,13 @@ class Context:
 
     # observables
     def measure_corr(self, U):
-        c = np.zeros(self.V)
+        c = np.empty(self.V)
         _check(lib().jw_measure_corr(self.h, U.h, _p(c)))
         return c
 
     def dipole_from_corr(self, corr):
         corr = np.ascontiguousarray(corr, dtype=np.float64)
-        S = np.zeros(self.V)
+        S = np.empty(self.V)
         _check(lib().jw_dipole_from_corr(self.h, _p(corr), _p(S)))
         return S
 
