@@ -163,15 +163,14 @@ int evolve_generator_basis(jw_ctx* c, jw_field* U, int nsteps, bool fused, bool 
         jw::NoiseSrc ns = take_noise(c, 16, c->noise_kspace ? JW_TAG_KSPACE : JW_TAG_LANGEVIN, &ok);
         if (!ok) return fail(JW_ERR_STATE, "pending injection has %d normals per site, need 16", c->inj_per_site);
         if (fused || large) {
-            const jw::StepArgs sa{ns, sa_pos, sa_k, kc == 0, corr, ss, 0, 1, it == 0, it < nsteps - 1, c->noise_kspace};
+            const jw::StepArgs sa{ns, sa_pos, sa_k, kc == 0, corr, ss, 0, 1, it == 0, it < nsteps - 1, c->noise_kspace,
+                                  it == nsteps - 1};
             if (fused) HIP_CHECK(jw::step_fused(c, U->d, Xi, Vv, ZA, ZB, sa));
             else HIP_CHECK(jw::step_large(c, U->d, Xi, Vv, ZA, ZB, sa));
             continue;
         }
         HIP_CHECK(jw::step_unfused(c, U->d, Xi, Vv, ZA, ZB, ns, sa_pos, sa_k, kc, corr, ss));
     }
-    // the fused and large-lattice passes keep rows 0 and 1 of U current
-    if ((fused || large) && nsteps > 0) HIP_CHECK(jw::u_rebuild(c, U->d, c->stream));
     return JW_OK;
 }
 
@@ -370,7 +369,7 @@ hipError_t batch_group_step(jw_batch* b, BatchGroup& g, int coupling, double ste
                     b->d_step};
     const jw::StepArgs a{ns,      sa_pos,      sa_k,  coupling == JW_SQRT_COUPLING_CONSTANT,
                          coupling == JW_CORRELATED_NOISE_COUPLING, sqrt(step), reunit, count, first_noise, next_noise,
-                         b->kspace};
+                         b->kspace, 0};
     if (b->fp32)
         return jw::step_fused_f32(g.ctx, (jw::cplxf*)U, (jw::cplxf*)g.Xi, (jw::cplxf*)g.Vv, (jw::cplxf*)g.ZA,
                                   (jw::cplxf*)g.ZB, a);
@@ -404,7 +403,7 @@ int batch_step_all(jw_batch* b, int coupling, double step, const jw::Alpha& al, 
                                    b->fp32 ? (const void*)g.ctx->twf : (const void*)g.ctx->tw};
         }
         const jw::StepArgs a{ga[0].ns, nullptr, nullptr, coupling == JW_SQRT_COUPLING_CONSTANT,
-                             coupling == JW_CORRELATED_NOISE_COUPLING, sqrt(step), reunit, 1, 1, 0, b->kspace};
+                             coupling == JW_CORRELATED_NOISE_COUPLING, sqrt(step), reunit, 1, 1, 0, b->kspace, 0};
         HIP_CHECK(b->fp32 ? jw::step_multi_f32(b->stream, ga, ng, a) : jw::step_multi(b->stream, ga, ng, a));
     } else {
         HIP_CHECK(hipEventRecord(b->fork, b->stream));
@@ -1108,7 +1107,7 @@ int jw_evolve_mixed(jw_ctx* c, jw_field* U, int coupling, int kernel, double ste
         const int reunit = reunit_every > 0 && ((it + 1) % reunit_every == 0 || it == nsteps - 1);
         const jw::StepArgs sa{ns,      sa_pos,        sa_k,           coupling == JW_SQRT_COUPLING_CONSTANT,
                               corr,    sqrt(step),    reunit,         1,
-                              it == 0, it < nsteps - 1, c->noise_kspace};
+                              it == 0, it < nsteps - 1, c->noise_kspace, 0};
         const hipError_t he = fused ? jw::step_fused_f32(c, U32, Xi, Vv, ZA, ZB, sa)
                               : large ? jw::step_large_f32(c, U32, Xi, Vv, ZA, ZB, sa)
                                     : jw::step_unfused_f32(c, U32, Xi, Vv, ZA, ZB, ns, sa_pos, sa_k,

@@ -174,8 +174,8 @@ struct site_mat<float2> { typedef m3f type; };
 // 2 rebuilt on load as conj(row 0 x row 1) -- U is in SU(3) to the rounding of
 // its form (and the mixed form projects it every few steps, rebuilding row 2
 // the same way) -- so that the row passes move a third less U.  The FP64 field
-// keeps its nine planes; row 2 is rebuilt into it after the fused steps
-// (u_rebuild).
+// keeps its nine planes; the last step of a call writes row 2 too (a pass of its own,
+// R 6 W 3, took 118 us at N = 2048 and a tenth of a call of one step at N = 64).
 template <typename C>
 struct UPlanes { static constexpr int value = 6; };
 template <typename C, typename M>
@@ -962,7 +962,7 @@ __global__ __launch_bounds__((ColB<N, BF, C>::NT), (ColB<N, BF, C>::WAVES)) void
 template <int N, int BF, typename C>
 __device__ __forceinline__ void row_update_body(C* lds, BlockIx bi, C* __restrict__ U, const C* __restrict__ ZA,
                                                               const C* __restrict__ ZB, size_t V, double ss,
-                                                              int reunit, const C* __restrict__ tw, int next_noise,
+                                                              int reunit, int whole, const C* __restrict__ tw, int next_noise,
                                                               C* __restrict__ Xi, NoiseSrc ns,
                                                               const double* __restrict__ sa_pos) {
     typedef typename scalar_of<C>::type T;
@@ -1015,6 +1015,11 @@ __device__ __forceinline__ void row_update_body(C* lds, BlockIx bi, C* __restric
             m3 r = mmul(w, exp_i_gen(hd, -ss));
             if (reunit) r = su3_project(r);
             store_u(U, V, i, r);
+            if (whole) {        // a call's last step leaves all nine entries
+                row2_of(r.m);
+#pragma unroll
+                for (int k = 6; k < 9; k++) U[k * V + i] = r.m[k];
+            }
         } else {
             // FP64 exponentials, FP32 products; the projection in FP64.  The
             // fences keep the two exponentials apart (fewer live registers).
@@ -1046,11 +1051,11 @@ __device__ __forceinline__ void row_update_body(C* lds, BlockIx bi, C* __restric
 template <int N, int BF, typename C>
 __global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_update(C* __restrict__ U, const C* __restrict__ ZA,
                                                               const C* __restrict__ ZB, size_t V, double ss,
-                                                              int reunit, const C* __restrict__ tw, int next_noise,
+                                                              int reunit, int whole, const C* __restrict__ tw, int next_noise,
                                                               C* __restrict__ Xi, NoiseSrc ns,
                                                               const double* __restrict__ sa_pos) {
     __shared__ C lds[4 * RowT<N, C>::PL];
-    row_update_body<N, BF, C>(lds, own_block(), U, ZA, ZB, V, ss, reunit, tw, next_noise, Xi, ns, sa_pos);
+    row_update_body<N, BF, C>(lds, own_block(), U, ZA, ZB, V, ss, reunit, whole, tw, next_noise, Xi, ns, sa_pos);
 }
 
 // ---------------------------------------------------------------------------
@@ -1189,7 +1194,7 @@ __global__ __launch_bounds__(T, RowWaves<C>::value) void k_row_update_multi(Mult
     dispatch_group<T, RowNT>(m, [&](auto n, const GroupRun<C>& g, int b) {
         constexpr int N = decltype(n)::value;
         row_update_body<N, 0, C>(lds + row_sub<N, T>() * 4 * RowT<N, C>::PL, row_slot<N, T>(b), g.U, g.ZA, g.ZB,
-                                 g.V, ss, reunit, g.tw, 0, g.Xi, g.ns, g.sa_pos);
+                                 g.V, ss, reunit, 0, g.tw, 0, g.Xi, g.ns, g.sa_pos);
     });
 }
 // column passes: the strips of a group in the order strip, plane pair, trajectory
@@ -1447,7 +1452,7 @@ static hipError_t step_fused_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     {
         KTimer t(c, kcls[3]);
         hipLaunchKernelGGL((k_row_update<N, BF, C>), dim3(N, 1, a.nbatch), dim3(RowE<N>::NT), 0, c->stream, U, ZA, ZB, V,
-                           a.sqrt_step, a.reunit, tw, next_noise, Xi, a.ns, a.sa_pos);
+                           a.sqrt_step, a.reunit, a.whole, tw, next_noise, Xi, a.ns, a.sa_pos);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return hipSuccess;

@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256) void k_uxiu_packed(C* __restrict__ Vv, const C
 
 template <typename C, int U6 = 0>
 __global__ __launch_bounds__(256) void k_update_packed(C* __restrict__ U, const C* __restrict__ ZA,
-                                                       const C* __restrict__ ZB, size_t V, double ss, int reunit) {
+                                                       const C* __restrict__ ZB, size_t V, double ss, int reunit, int whole) {
     GRID_STRIDE(i, V) {
         double ha[8], hb[8];
 #pragma unroll
@@ -248,6 +248,11 @@ __global__ __launch_bounds__(256) void k_update_packed(C* __restrict__ U, const 
         if (reunit) r = su3_project(r);
 #pragma unroll
         for (int k = 0; k < (U6 ? 6 : 9); k++) U[k * V + i] = mkc<C>(r.m[k].x, r.m[k].y);
+        if (U6 && whole) {      // a call's last step leaves all nine entries
+            row2_of(r.m);
+#pragma unroll
+            for (int k = 6; k < 9; k++) U[k * V + i] = mkc<C>(r.m[k].x, r.m[k].y);
+        }
     }
 }
 
@@ -291,7 +296,7 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
     JW_TRY(fft2d_t(c, ZB, 4, 0, s));
     {
         KTimer t(c, K_UPDATE);
-        hipLaunchKernelGGL(k_update_packed<C>, dim3(g), dim3(256), 0, c->stream, U, ZA, ZB, V, ss, reunit);
+        hipLaunchKernelGGL(k_update_packed<C>, dim3(g), dim3(256), 0, c->stream, U, ZA, ZB, V, ss, reunit, 0);
         JW_TRY(hipGetLastError());
     }
 #undef JW_TRY
@@ -443,7 +448,7 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     {
         KTimer t(c, K_UPDATE);
         hipLaunchKernelGGL((k_update_packed<C, 1>), dim3(g), dim3(256), 0, c->stream, U, ZA, ZB, V, a.sqrt_step,
-                           a.reunit);
+                           a.reunit, a.whole);
         JW_TRY(hipGetLastError());
     }
 #undef JW_TRY
