@@ -67,23 +67,89 @@ __global__ __launch_bounds__((ColCfg<N, C>::NT)) void k_fft_cols(C* __restrict__
         base[(size_t)(i / G::W) * N + (i % G::W)] = cscale(lds[lpos<G::W, 1, 3>(i / G::W, i % G::W)], (T)scale);
 }
 
+// From N = 64 on the transforms run in registers (jw_regfft.hpp), T threads a row or a
+// column, and LDS is touched by one exchange over the workgroup and one inside a wave
+// instead of by every radix-8 stage; a column strip is a 64-byte segment wide.  Bound by
+// memory: nine planes of FP64 at N = 512 (2 x 38 MB), rows 17.0 -> 16.8 us, columns 22.0 ->
+// 14.5; four at N = 8192 8.9 -> 6.6 ms (columns).
+template <int N, int DIR, typename C>
+__global__ __launch_bounds__(RowN<N>::NT) void k_fft_rows_reg(C* __restrict__ data, size_t plane_stride,
+                                                              const C* __restrict__ tw, double scale) {
+    typedef typename scalar_of<C>::type T;
+    typedef RegFft<N> F;
+    __shared__ C lds[RowN<N>::RPW * RowT<N, C>::PL];
+    C* row = data + blockIdx.y * plane_stride + ((size_t)blockIdx.x * RowN<N>::RPW + threadIdx.x / F::T) * N;
+    C* buf = lds + (threadIdx.x / F::T) * RowT<N, C>::PL;
+    const int j = threadIdx.x % F::T;
+    C v[F::PT];
+    auto site = [&](int r) { return opaque_v(j) + r * F::T; };
+    auto freq = [&](int q) {
+        const int i = opaque_v(j);
+        return reg_freq<N>(i / F::N3, i % F::N3, 0) + reg_freq_q<N>(q);
+    };
+#pragma unroll
+    for (int r = 0; r < F::PT; r++) v[r] = row[DIR < 0 ? site(r) : freq(r)];
+    if constexpr (DIR < 0) reg_fft_fwd<N, 1, true>(v, buf, tw_fft(tw), opaque_v(j));
+    else reg_fft_inv<N, 1, true>(v, buf, tw_fft(tw), opaque_v(j));
+#pragma unroll
+    for (int r = 0; r < F::PT; r++) row[DIR < 0 ? freq(r) : site(r)] = cscale(v[r], (T)scale);
+}
+
+template <int N, int DIR, typename C>
+__global__ __launch_bounds__((ColR<N, C>::NT)) void k_fft_cols_reg(C* __restrict__ data, size_t plane_stride,
+                                                                   const C* __restrict__ tw, double scale) {
+    typedef typename scalar_of<C>::type T;
+    typedef RegFft<N> F;
+    constexpr int W = ColR<N, C>::W;
+    __shared__ C lds[ColR<N, C>::ELEMS];
+    data += blockIdx.y * plane_stride + (size_t)xcd_strip(blockIdx.x, N / W) * W;
+    auto site = [&]() { const int t = opaque_v((int)threadIdx.x); return (unsigned)(t / W * N + t % W); };
+    auto freq = [&]() {
+        const int t = opaque_v((int)threadIdx.x), j = t / W;
+        return (unsigned)(reg_freq<N>(j / F::N3, j % F::N3, 0) * N + t % W);
+    };
+    constexpr size_t RS = (size_t)F::T * N;
+    auto rq = [](int q) { return (size_t)reg_freq_q<N>(q) * N; };
+    C v[F::PT];
+    const unsigned o = DIR < 0 ? site() : freq();
+#pragma unroll
+    for (int r = 0; r < F::PT; r++) v[r] = (data + (DIR < 0 ? r * RS : rq(r)))[o];
+    if constexpr (DIR < 0) reg_fft_fwd<N, W, true>(v, lds, tw_fft(tw), opaque_v((int)threadIdx.x));
+    else reg_fft_inv<N, W, true>(v, lds, tw_fft(tw), opaque_v((int)threadIdx.x));
+    const unsigned e = DIR < 0 ? freq() : site();
+#pragma unroll
+    for (int r = 0; r < F::PT; r++) (data + (DIR < 0 ? rq(r) : r * RS))[e] = cscale(v[r], (T)scale);
+}
+
 template <int N, typename C>
 static hipError_t launch_rows(jw_ctx* c, C* p, int np, int dir, double scale, const C* tw) {
-    using G = RowCfg<N, C>;
-    dim3 grid(N / G::RPW, np);
     KTimer t(c, K_FFT_ROWS);
-    if (dir) hipLaunchKernelGGL((k_fft_rows<N, -1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
-    else hipLaunchKernelGGL((k_fft_rows<N, +1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
+    if constexpr (N >= 64) {
+        dim3 grid(N / RowN<N>::RPW, np), block(RowN<N>::NT);
+        if (dir) hipLaunchKernelGGL((k_fft_rows_reg<N, -1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
+        else hipLaunchKernelGGL((k_fft_rows_reg<N, +1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
+    } else {
+        using G = RowCfg<N, C>;
+        dim3 grid(N / G::RPW, np);
+        if (dir) hipLaunchKernelGGL((k_fft_rows<N, -1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
+        else hipLaunchKernelGGL((k_fft_rows<N, +1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
+    }
     return hipGetLastError();
 }
 
 template <int N, typename C>
 static hipError_t launch_cols(jw_ctx* c, C* p, int np, int dir, double scale, const C* tw) {
-    using G = ColCfg<N, C>;
-    dim3 grid(N / G::W, np);
     KTimer t(c, K_FFT_COLS);
-    if (dir) hipLaunchKernelGGL((k_fft_cols<N, -1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
-    else hipLaunchKernelGGL((k_fft_cols<N, +1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
+    if constexpr (N >= 64) {
+        dim3 grid(N / ColR<N, C>::W, np), block(ColR<N, C>::NT);
+        if (dir) hipLaunchKernelGGL((k_fft_cols_reg<N, -1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
+        else hipLaunchKernelGGL((k_fft_cols_reg<N, +1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
+    } else {
+        using G = ColCfg<N, C>;
+        dim3 grid(N / G::W, np);
+        if (dir) hipLaunchKernelGGL((k_fft_cols<N, -1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
+        else hipLaunchKernelGGL((k_fft_cols<N, +1, C>), grid, dim3(G::NT), 0, c->stream, p, c->V, tw, scale);
+    }
     return hipGetLastError();
 }
 
