@@ -372,7 +372,7 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
 
 // ===========================================================================
 // Large lattices (N = 4096, 8192): the fused column passes of jw_engine.hpp
-// (forward column FFT, kernel multiply, inverse column FFT in LDS per strip;
+// (forward column FFT, kernel multiply, inverse column FFT per strip;
 // the momentum-space noise drawn there) with the row transforms and the site
 // algebra as separate passes, since one lattice row of four planes no longer
 // fits LDS (FP64 at N = 4096 needs 256 KB).  U is held as rows 0 and 1 (row 2
@@ -380,7 +380,7 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
 //   [position-space noise: noise W 8, forward row FFT R 8 W 8]
 //   column A                     R 8 (0 drawn) W 4 (+8 correlated or drawn)
 //   inverse row FFT of A         R 4 W 4
-//   correlated or drawn noise, k_row_uxiu_1p (FP32 at N = 8192):
+//   correlated or drawn noise, k_row_uxiu_1p (not in FP64 at N = 8192):
 //     inverse row FFT of xi~, U xi~ U^dagger, forward row FFT of V  R 20 W 8
 //   otherwise: [inverse row FFT of xi~ R 8 W 8]
 //     U xi U^dagger              R 6 (+8) W 8
@@ -388,80 +388,145 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
 //   column B                     R 8 W 4
 //   inverse row FFT of B         R 4 W 4
 //   update                       R 14 W 6
-// 88 planes with the noise drawn per mode in FP32 at N = 8192 (114 otherwise),
-// against 66 for the fused step of N <= 2048.  Column strips: BF = 32 (16-byte
-// row segments) at N = 8192, BF = 0 or 32 at N = 4096 (the intermediate planes
-// stay row-major).
+// 88 planes with the noise drawn per mode (114 in FP64 at N = 8192),
+// against 66 for the fused step of N <= 2048.  Column strips: k_col_reg on planes in
+// natural order (layout 3 of its parameter), 16-byte row segments in FP32 at N = 8192, 32 at
+// N = 4096; one plane at a time over 16-byte segments (BF = 32) in FP64 at N = 8192.
 // ===========================================================================
-// U xi~ U^dagger of the large-lattice step as one pass over a lattice row (FP32
-// at N = 8192; FP32 at 4096 and FP64 spill registers), where four planes of a row do not fit
-// LDS: each plane of xi~ is inverse-transformed alone in LDS and its values at
-// the thread's SPT sites are kept in registers; with the four planes of a
-// direction held, V = U xi~ U^dagger per site (U as rows 0 and 1, read once per
-// direction), and the four planes of V go through LDS one at a time for the
-// forward row transform.  In place of the inverse row FFT of xi~ (R 8 W 8), the
-// site pass (R 14 W 8) and the forward row FFT of V (R 8 W 8): R 20 W 8.
+// U xi~ U^dagger of the large-lattice step as one pass over a lattice row, where
+// four planes of a row do not fit LDS: the four planes of a direction are in the
+// registers of T threads each (jw_regfft.hpp), and every exchange goes through LDS
+// for the real parts and then for the imaginary parts (4 N elements of 4 bytes:
+// 132 KB at N = 8192).  The transformed planes are exchanged once more so that each
+// thread holds the four of its own sites for V = U xi~ U^dagger (U as rows 0 and 1,
+// read once per direction), and back.  In place of the inverse row FFT of xi~ (R 8 W 8),
+// the site pass (R 14 W 8) and the forward row FFT of V (R 8 W 8): R 20 W 8.
+// Bound by memory and by its own exchanges in turn (one workgroup a CU): FP32 at N = 8192
+// 4.6 ms (10.7 GB), where a plane at a time through LDS stages took 7.7 ms.  Against the
+// three passes, two steps at N = 4096 with drawn correlated noise: FP64 18.3 -> 15.5 ms, FP32
+// 10.8 -> 10.0.  FP64 at N = 8192 fits neither LDS nor registers and keeps the three passes.
 template <int N, typename C>
 struct Row1P {
-    static constexpr int NT = 1024, SPT = N / NT;
-    static constexpr bool ok = N == 8192 && sizeof(C) == sizeof(float2);
-};
-template <int N, typename C>
-__global__ __launch_bounds__(1024, 1) void k_row_uxiu_1p(C* __restrict__ Vv, const C* __restrict__ U,
-                                                          const C* __restrict__ Xs, size_t V,
-                                                          const C* __restrict__ tw) {
+    typedef RegFft<N> F;
     typedef typename scalar_of<C>::type T;
-    constexpr int NT = Row1P<N, C>::NT, SPT = Row1P<N, C>::SPT;
-    constexpr int PN = padded<N, 4>::value;
-    static_assert(SPT * NT == N, "row tiling");
-    __shared__ C lds[PN];
-    const int tid = threadIdx.x;
+    static constexpr int NT = 4 * F::T, SPT = N / NT;
+    static constexpr int SUB = RegLds<N, 1, T>::SUB, PL = RegLds<N, 1, T>::ELEMS;
+    static constexpr bool ok = sizeof(C) == sizeof(float2) || N == 4096;
+};
+// v[k] -> LDS at to(k), v[k] <- LDS from from(k), the real parts and then the imaginary
+// parts; WG: over the workgroup (otherwise inside each wave).  Ends with its reads.
+template <int PT, bool WG, typename C, typename TO, typename FROM>
+__device__ __forceinline__ void split_exchange(C* v, TO&& to, FROM&& from) {
+    auto wait = [] {
+        if constexpr (WG) __syncthreads();
+        else wave_lds_fence();
+    };
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        wait();
+#pragma unroll
+        for (int k = 0; k < PT; k++) *to(k) = half ? v[k].y : v[k].x;
+        wait();
+#pragma unroll
+        for (int k = 0; k < PT; k++) (half ? v[k].y : v[k].x) = *from(k);
+    }
+}
+template <int N, typename C>
+__global__ __launch_bounds__((Row1P<N, C>::NT), 1) void k_row_uxiu_1p(C* __restrict__ Vv, const C* __restrict__ U,
+                                                                      const C* __restrict__ Xs, size_t V,
+                                                                      const C* __restrict__ tw) {
+    typedef typename scalar_of<C>::type T;
+    typedef RegFft<N> F;
+    typedef Row1P<N, C> R;
+    constexpr int PT = F::PT, N3 = F::N3, SPT = R::SPT, SUB = R::SUB;
+    static_assert(SPT * R::NT == N && 4 * SPT == PT, "row tiling");
+    __shared__ T lds[4 * R::PL];
     const size_t row0 = (size_t)blockIdx.x * N;
+    // the slots of the exchanges: a thread's points j + T r, its sub-sequence, the order inside it,
+    // and a thread's sites (site y of plane p at (y / T) SUB + y mod T)
+    auto pl = [&] { return lds + opaque_v((int)threadIdx.x) / F::T * R::PL; };
+    auto idx = [] { return opaque_v((int)threadIdx.x) % F::T; };
 #pragma unroll 1
     for (int half = 0; half < 2; half++) {
-        C h[4][SPT];
+        C v[PT];
+        {
+            const int t = opaque_v((int)threadIdx.x), j = t % F::T;
+            const C* src = Xs + (size_t)(4 * half + t / F::T) * V + row0 + reg_freq<N>(j / N3, j % N3, 0);
 #pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const C* src = Xs + (size_t)(4 * half + p) * V + row0;
-            const int tl = opaque_v(tid);
-#pragma unroll
-            for (int q = 0; q < SPT; q++) lds[lpos<1, PN, 4>(tl + q * NT, 0)] = src[tl + q * NT];
-            __syncthreads();
-            lds_fft<N, 1, 1, PN, NT, +1, 4>(lds, tw_fft(tw), opaque_v(tid));
-            const int tr = opaque_v(tid);
-#pragma unroll
-            for (int q = 0; q < SPT; q++) h[p][q] = lds[lpos<1, PN, 4>(tr + q * NT, 0)];
-            __syncthreads();
+            for (int q = 0; q < PT; q++) v[q] = src[reg_freq_q<N>(q)];
         }
-        const int tu = opaque_v(tid);
+        {
+            const int j = idx(), g = j / N3, m = j % N3;
+            T* sub = pl() + g * SUB;
+            T* own = pl() + j;
+            if (half) __syncthreads();
+#pragma unroll
+            for (int u = 0; u < F::NU; u++) dft_reg<N3, +1>(v + u * N3);
+            split_exchange<PT, false>(
+                v, [&](int k) { return sub + (m + N3 * (k / N3)) * N3 + ((k % N3) ^ m); },
+                [&](int b) { return sub + b * N3 + (m ^ (b % N3)); });
+            twiddle_powers<PT, +1>(v, tw_fft(tw), PT * m);
+            dft_reg<PT, +1>(v);
+            split_exchange<PT, true>(
+                v, [&](int a) { return sub + m + N3 * a; }, [&](int k) { return own + k * SUB; });
+            twiddle_powers<PT, +1>(v, tw_fft(tw), j);
+            dft_reg<PT, +1>(v);
+        }
+        {
+            T* own = pl() + idx();
+            const int t = opaque_v((int)threadIdx.x);
+            T* site = lds + t / F::T * SUB + t % F::T;
+            split_exchange<PT, true>(
+                v, [&](int r) { return own + r * SUB; },
+                [&](int k) { return site + k % 4 * R::PL + k / 4 * 4 * SUB; });
+        }
+        // v[4 q + p]: plane p of site threadIdx + q NT
+        const int tu = opaque_v((int)threadIdx.x);
 #pragma unroll
         for (int q = 0; q < SPT; q++) {
-            const size_t i = row0 + tu + q * NT;
+            const size_t i = row0 + tu + q * R::NT;
             T hh[8];
 #pragma unroll
             for (int p = 0; p < 4; p++) {
-                hh[2 * p] = h[p][q].x;
-                hh[2 * p + 1] = h[p][q].y;
+                hh[2 * p] = v[4 * q + p].x;
+                hh[2 * p + 1] = v[4 * q + p].y;
             }
             typename site_mat<C>::type u;
             load_u(u, U, V, i);
-            T v[8];
-            uxiu_gen(u, hh, v);
+            T w[8];
+            uxiu_gen(u, hh, w);
 #pragma unroll
-            for (int p = 0; p < 4; p++) h[p][q] = mkc<C>(v[2 * p], v[2 * p + 1]);
+            for (int p = 0; p < 4; p++) v[4 * q + p] = mkc<C>(w[2 * p], w[2 * p + 1]);
         }
+        {
+            T* own = pl() + idx();
+            const int t = opaque_v((int)threadIdx.x);
+            T* site = lds + t / F::T * SUB + t % F::T;
+            split_exchange<PT, true>(
+                v, [&](int k) { return site + k % 4 * R::PL + k / 4 * 4 * SUB; },
+                [&](int r) { return own + r * SUB; });
+        }
+        {
+            const int j = idx(), g = j / N3, m = j % N3;
+            T* sub = pl() + g * SUB;
+            T* own = pl() + j;
+            dft_reg<PT, -1>(v);
+            twiddle_powers<PT, -1>(v, tw_fft(tw), j);
+            split_exchange<PT, true>(
+                v, [&](int k) { return own + k * SUB; }, [&](int a) { return sub + m + N3 * a; });
+            dft_reg<PT, -1>(v);
+            twiddle_powers<PT, -1>(v, tw_fft(tw), PT * m);
+            split_exchange<PT, false>(
+                v, [&](int b) { return sub + b * N3 + (m ^ (b % N3)); },
+                [&](int k) { return sub + (m + N3 * (k / N3)) * N3 + ((k % N3) ^ m); });
 #pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const int tl = opaque_v(tid);
+            for (int u = 0; u < F::NU; u++) dft_reg<N3, -1>(v + u * N3);
+        }
+        {
+            const int t = opaque_v((int)threadIdx.x), j = t % F::T;
+            C* dst = Vv + (size_t)(4 * half + t / F::T) * V + row0 + reg_freq<N>(j / N3, j % N3, 0);
 #pragma unroll
-            for (int q = 0; q < SPT; q++) lds[lpos<1, PN, 4>(tl + q * NT, 0)] = h[p][q];
-            __syncthreads();
-            lds_fft<N, 1, 1, PN, NT, -1, 4>(lds, tw_fft(tw), opaque_v(tid));
-            C* dst = Vv + (size_t)(4 * half + p) * V + row0;
-            const int ts = opaque_v(tid);
-#pragma unroll
-            for (int q = 0; q < SPT; q++) dst[ts + q * NT] = lds[lpos<1, PN, 4>(ts + q * NT, 0)];
-            __syncthreads();
+            for (int q = 0; q < PT; q++) dst[reg_freq_q<N>(q)] = v[q];
         }
     }
 }
