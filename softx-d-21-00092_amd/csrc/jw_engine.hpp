@@ -1410,16 +1410,16 @@ static hipError_t step_fused_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     const size_t V = c->V;
     const C* tw = twiddles<C>(c);
     hipError_t e;
-    // The next step's noise rides on the update pass in FP64 for N <= 512,
-    // where that measured faster (steps/s, fixed / correlated coupling, fused
-    // against separate: N = 256 10032 / 10783 against 9785 / 10571; 512 7258 /
-    // 7134 against 6670 / 6579); at 1024 and 2048 the separate pass is faster
-    // (1916 / 1742 against 1746 / 1597; 471 / 426 against 463 / 420), and in
-    // FP32 the separate pass, at two workgroups per CU, is faster everywhere.
+    // The next step's noise rides on the update pass up to N = 1024, where that is
+    // faster: its instructions hide under the update's memory time, and a launch goes (us a
+    // step, fixed coupling, separate -> fused, FP64 / FP32: N = 64 26.8 -> 23.8 / 24.7 ->
+    // 22.3; 256 57.0 -> 53.9 / 42.1 -> 40.3; 512 95.9 -> 91.3 / 64.2 -> 61.2; 1024 365 ->
+    // 353 / 187 -> 182).  At 2048 it is slower in FP64 (1449 -> 1507), whose update then
+    // runs with one workgroup a CU, and the same in FP32 (766 -> 763, correlated 894 -> 897).
     // Momentum-space noise (a.kspace): no noise pass; the first column pass
     // draws the spectra and writes the position-space noise's row spectra back
     // for the correlated row pass.
-    constexpr bool fuse_noise = sizeof(C) == sizeof(double2) && N <= 512;
+    constexpr bool fuse_noise = N <= 1024;
     const int first_noise = a.kspace ? 0 : fuse_noise ? a.first_noise : 1;
     const int next_noise = a.kspace ? 0 : fuse_noise ? a.next_noise : 0;
     if (first_noise) {
