@@ -1,6 +1,6 @@
 // jw_engine.hpp -- fused generator-basis Langevin step for 64 <= N <= 2048,
 // templated on the storage type C (double2: FP64 form, float2: mixed form);
-// instantiated by jw_step_f64.hip and jw_step_f32.hip.
+// one object per size and type (jw_step_n.hip, jw_step_multi.hip).
 //
 // One step (main_optimized.cpp:243-304 in the generator basis) as five passes
 // over HBM instead of the reference's 8 nine-component FFTs and 5 site loops:
@@ -15,19 +15,24 @@
 // U as its rows 0 and 1, UPlanes below).  With the spectra drawn per mode the
 // noise pass goes and column A reads nothing and writes 12 planes.
 //
-// Row passes: one workgroup per lattice row, four planes at a time in LDS.
+// Transforms run with their data in registers (jw_regfft.hpp).  Row passes: one
+// workgroup per lattice row and four planes, LDS holding the row between the transform
+// and the site algebra.
 //
 // The intermediate planes (xi, V, A, B spectra) between a row pass and a
-// column pass are stored in one of two layouts (template parameter BF):
-//   BF = 0   row-major, site (x, y) at x N + y.  Column passes then take strips
-//            of W adjacent columns (X and Y tiles together in LDS), workgroups
+// column pass are stored in one of these layouts (template parameter BF):
+//   BF = 0   row-major, row spectra in the order of freq_of_pos.  Column passes take
+//            strips of W adjacent columns, X and Y in registers (k_col_reg), workgroups
 //            mapped so that strips sharing cache lines run on the same XCD.
+//   BF = 3   the same in frequency order: the large lattices, the matrix-core stages.
+//   BF = 2   the x and y directions interleaved site by site (k_col_kmult).
 //   BF = 4, 8  blocks of BF rows: (x, y) at ((x / BF) N + y) BF + x mod BF, so
 //            that one 128-byte segment holds 8 / BF adjacent columns of BF
 //            consecutive rows.  A column pass then reads and writes whole
 //            segments (8 / BF columns per workgroup, one plane at a time, all
 //            four plane pairs in one workgroup); row passes touch BF-row
 //            segments whose rows are processed on one XCD at neighbouring times.
+//   BF = 1, 16, 32  row-major, one plane at a time over 64-, 32- or 16-byte strips.
 // U always stays row-major.
 #pragma once
 
@@ -55,7 +60,7 @@ template <int N, typename C>
 __device__ __forceinline__ int row_slot_of(int y) {
     return (y / RowE<N>::T) * RowT<N, C>::SUB + y % RowE<N>::T;
 }
-// Row-major column passes hold the X and Y tiles of one W-column strip together
+// The column passes in LDS (k_col_kmult) hold the X and Y tiles of one W-column strip together
 // in LDS (2 W N complex values plus one padding row in eight, 144 KB at most in
 // FP64): W = min(16, 4096 / N) for both forms (wider FP32 strips measured
 // slower: one workgroup per CU and spills in the correlated variant).
@@ -497,8 +502,9 @@ __global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_uxiu_co
 //   receive the row spectra of the position-space noise.
 // X, Y: row spectra of plane p; one workgroup per strip of W columns and plane
 // pair.  BF = 0: columns in the order of freq_of_pos, and sa's likewise; otherwise
-// (the large lattices) column c is frequency c.  A thread holds PT points of one column of X and of Y; LDS holds one
-// plane of the strip for the exchanges, and the (4 sin^2, sin) table of kx.
+// (the large lattices) column c is frequency c.  A thread holds PT points of one column
+// of X and of Y; LDS holds one plane of the strip for the exchanges, and the
+// (4 sin^2, sin) table of kx.
 //
 // What bounds it: the loaded pass moves 12 planes at 3.1-3.2 TB/s (FP64 and FP32
 // at N = 2048; the bare access pattern reaches 4.6 TB/s), the drawing pass is
@@ -528,6 +534,24 @@ struct ColR {
     static_assert(W >= 1 && NT >= 64 && NT * REGS <= 512 * 256, "column strip");
 };
 
+// Planes that a column pass of a large lattice writes for row passes (BF = 3; Z, and X, Y
+// where they are drawn): tiles of TR rows by the strip's W columns, 64 bytes each, so that a
+// workgroup writes whole 64-byte pieces.  In row-major planes a strip's row segments are 16
+// bytes (N = 8192 in FP32; 32 at 4096), the other strips' parts of a line come after
+// the line has left L2, and 2.4 times the bytes went to memory.  us per launch, row-major
+// -> tiles: N = 8192 FP32 drawing 9500 -> 5010, loaded (which reads row-major planes)
+// 6180 -> 4490, against U xi~ U^dagger 4600 -> 5000 on tiles.  Two drawn fixed-coupling steps
+// at N = 4096, FP64 14.8 -> 13.5 ms, FP32 10.0 -> 9.1.  at(x, c) is the offset of row x's
+// column c; columns W apart are TR W elements apart.
+template <int N, typename C>
+struct Tile {
+    static constexpr int W = ColR<N, C>::W, TR = 64 / (int)sizeof(C) / W;
+    static_assert(TR >= 1 && RegFft<N>::T % TR == 0, "tile");
+    static __device__ __forceinline__ size_t at(int x, int c) {
+        return ((size_t)(x / TR) * (N / W) + c / W) * (TR * W) + (x % TR) * W + c % W;
+    }
+};
+
 // v, defined only once d is: what is computed from it is not started before
 template <typename T>
 __device__ __forceinline__ int after(int v, T d) {
@@ -555,6 +579,14 @@ __device__ __forceinline__ void col_reg_body(C* lds, double2* kt, BlockIx bi, C*
     // the thread's first element: uniform plane and row offsets, one 32-bit offset per thread
     auto at = [&]() -> unsigned {
         const int t = opaque_v(bi.tid);
+        return (unsigned)((t / W) * N + col0 + t % W);
+    };
+    // where it goes: tiles on the large lattices' planes, except over planes that other
+    // strips still read
+    auto ot = [&](bool over) -> unsigned {
+        const int t = opaque_v(bi.tid);
+        if constexpr (BF == 3)
+            if (!over) return (unsigned)Tile<N, C>::at(t / W, col0 + t % W);
         return (unsigned)((t / W) * N + col0 + t % W);
     };
     if constexpr (CR::TAB) {
@@ -619,17 +651,17 @@ __device__ __forceinline__ void col_reg_body(C* lds, double2* kt, BlockIx bi, C*
     reg_fft_inv<N, W, true>(x, lds, tw_fft(tw), opaque_v(bi.tid));
     {
         C* const O = CORR ? X : Z;
-        const unsigned o = at();
+        const unsigned o = ot(CORR && !GEN);
 #pragma unroll
         for (int r = 0; r < PT; r++) (O + r * RS)[o] = x[r];
     }
     if constexpr (CORR) {
         reg_fft_inv<N, W, false>(y, lds, tw_fft(tw), opaque_v(bi.tid));
-        const unsigned oy = at();
+        const unsigned oy = ot(!GEN);
 #pragma unroll
         for (int r = 0; r < PT; r++) (Y + r * RS)[oy] = y[r];
         reg_fft_inv<N, W, false>(z, lds, tw_fft(tw), opaque_v(bi.tid));
-        const unsigned oz = at();
+        const unsigned oz = ot(false);
 #pragma unroll
         for (int r = 0; r < PT; r++) (Z + r * RS)[oz] = z[r];
     }

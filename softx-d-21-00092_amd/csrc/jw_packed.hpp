@@ -95,6 +95,27 @@ __global__ __launch_bounds__(RowN<N>::NT) void k_fft_rows_reg(C* __restrict__ da
     for (int r = 0; r < F::PT; r++) row[DIR < 0 ? freq(r) : site(r)] = cscale(v[r], (T)scale);
 }
 
+// inverse row transforms of tiled planes (Tile) into row-major ones; the rows of a tile
+// run on one XCD.  Bound by memory; four FP32 planes at N = 8192 1.13 ms (1.05 in place on
+// row-major ones, whose column passes took 6.2 ms longer a step).
+template <int N, typename C>
+__global__ __launch_bounds__(RowN<N>::NT) void k_rows_inv_tiled(C* __restrict__ out, const C* __restrict__ in, size_t V,
+                                                                const C* __restrict__ tw) {
+    typedef RegFft<N> F;
+    __shared__ C lds[RowN<N>::RPW * RowT<N, C>::PL];
+    const int x = xcd_strip(blockIdx.x, N / RowN<N>::RPW) * RowN<N>::RPW + threadIdx.x / F::T;
+    C* buf = lds + (threadIdx.x / F::T) * RowT<N, C>::PL;
+    const int j = threadIdx.x % F::T;
+    C v[F::PT];
+    const C* src = in + blockIdx.y * V + Tile<N, C>::at(x, reg_freq<N>(j / F::N3, j % F::N3, 0));
+#pragma unroll
+    for (int q = 0; q < F::PT; q++) v[q] = src[reg_freq_q<N>(q) * Tile<N, C>::TR];
+    reg_fft_inv<N, 1, true>(v, buf, tw_fft(tw), opaque_v(j));
+    C* dst = out + blockIdx.y * V + (size_t)x * N + j;
+#pragma unroll
+    for (int r = 0; r < F::PT; r++) dst[r * F::T] = v[r];
+}
+
 template <int N, int DIR, typename C>
 __global__ __launch_bounds__((ColR<N, C>::NT)) void k_fft_cols_reg(C* __restrict__ data, size_t plane_stride,
                                                                    const C* __restrict__ tw, double scale) {
@@ -379,7 +400,7 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
 // rebuilt on load), as in the fused step.  Per step, in complex planes moved:
 //   [position-space noise: noise W 8, forward row FFT R 8 W 8]
 //   column A                     R 8 (0 drawn) W 4 (+8 correlated or drawn)
-//   inverse row FFT of A         R 4 W 4
+//   inverse row FFT of A         R 4 W 4   (after U xi U^dagger where A is in tiles)
 //   correlated or drawn noise, k_row_uxiu_1p (not in FP64 at N = 8192):
 //     inverse row FFT of xi~, U xi~ U^dagger, forward row FFT of V  R 20 W 8
 //   otherwise: [inverse row FFT of xi~ R 8 W 8]
@@ -391,7 +412,8 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
 // 88 planes with the noise drawn per mode (114 in FP64 at N = 8192),
 // against 66 for the fused step of N <= 2048.  Column strips: k_col_reg on planes in
 // natural order (layout 3 of its parameter), 16-byte row segments in FP32 at N = 8192, 32 at
-// N = 4096; one plane at a time over 16-byte segments (BF = 32) in FP64 at N = 8192.
+// N = 4096, which writes tiles of 64 bytes (Tile) where row passes read; one plane at a
+// time over 16-byte segments (BF = 32) in FP64 at N = 8192.
 // ===========================================================================
 // U xi~ U^dagger of the large-lattice step as one pass over a lattice row, where
 // four planes of a row do not fit LDS: the four planes of a direction are in the
@@ -402,7 +424,7 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
 // read once per direction), and back.  In place of the inverse row FFT of xi~ (R 8 W 8),
 // the site pass (R 14 W 8) and the forward row FFT of V (R 8 W 8): R 20 W 8.
 // Bound by memory and by its own exchanges in turn (one workgroup a CU): FP32 at N = 8192
-// 4.6 ms (10.7 GB), where a plane at a time through LDS stages took 7.7 ms.  Against the
+// 4.6 ms (10.7 GB; 5.0 from tiles), where a plane at a time through LDS stages took 7.7 ms.  Against the
 // three passes, two steps at N = 4096 with drawn correlated noise: FP64 18.3 -> 15.5 ms, FP32
 // 10.8 -> 10.0.  FP64 at N = 8192 fits neither LDS nor registers and keeps the three passes.
 template <int N, typename C>
@@ -431,7 +453,8 @@ __device__ __forceinline__ void split_exchange(C* v, TO&& to, FROM&& from) {
         for (int k = 0; k < PT; k++) (half ? v[k].y : v[k].x) = *from(k);
     }
 }
-template <int N, typename C>
+// TILED: xi~ in tiles (Tile), the rows of a tile on one XCD.
+template <int N, int TILED, typename C>
 __global__ __launch_bounds__((Row1P<N, C>::NT), 1) void k_row_uxiu_1p(C* __restrict__ Vv, const C* __restrict__ U,
                                                                       const C* __restrict__ Xs, size_t V,
                                                                       const C* __restrict__ tw) {
@@ -441,7 +464,8 @@ __global__ __launch_bounds__((Row1P<N, C>::NT), 1) void k_row_uxiu_1p(C* __restr
     constexpr int PT = F::PT, N3 = F::N3, SPT = R::SPT, SUB = R::SUB;
     static_assert(SPT * R::NT == N && 4 * SPT == PT, "row tiling");
     __shared__ T lds[4 * R::PL];
-    const size_t row0 = (size_t)blockIdx.x * N;
+    const int x = TILED ? xcd_strip(blockIdx.x, N) : (int)blockIdx.x;
+    const size_t row0 = (size_t)x * N;
     // the slots of the exchanges: a thread's points j + T r, its sub-sequence, the order inside it,
     // and a thread's sites (site y of plane p at (y / T) SUB + y mod T)
     auto pl = [&] { return lds + opaque_v((int)threadIdx.x) / F::T * R::PL; };
@@ -451,9 +475,10 @@ __global__ __launch_bounds__((Row1P<N, C>::NT), 1) void k_row_uxiu_1p(C* __restr
         C v[PT];
         {
             const int t = opaque_v((int)threadIdx.x), j = t % F::T;
-            const C* src = Xs + (size_t)(4 * half + t / F::T) * V + row0 + reg_freq<N>(j / N3, j % N3, 0);
+            const int f = reg_freq<N>(j / N3, j % N3, 0);
+            const C* src = Xs + (size_t)(4 * half + t / F::T) * V + (TILED ? Tile<N, C>::at(x, f) : row0 + f);
 #pragma unroll
-            for (int q = 0; q < PT; q++) v[q] = src[reg_freq_q<N>(q)];
+            for (int q = 0; q < PT; q++) v[q] = src[reg_freq_q<N>(q) * (TILED ? Tile<N, C>::TR : 1)];
         }
         {
             const int j = idx(), g = j / N3, m = j % N3;
@@ -551,12 +576,27 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
         KTimer t(c, K_COL_KMULT);
         JW_TRY((col_pass<N, BF>(c, ZA, Xi, Xi + 4 * V, a.sa_k, a.sqrt_coupling, a.corr, 1, a.ns, a.kspace, a.corr)));
     }
-    JW_TRY((launch_rows<N, C>(c, ZA, 4, 0, 1.0, tw)));
+    // BF = 3: column passes write tiles, which the row transforms take out of place, into
+    // the planes of xi~ once U xi~ U^dagger has read them
+    const C *HA = ZA, *HB = ZB;
+    auto rows_inv = [&](C* Z, C* to, const C*& H) -> hipError_t {
+        if constexpr (BF == 3) {
+            KTimer t(c, K_FFT_ROWS);
+            hipLaunchKernelGGL((k_rows_inv_tiled<N, C>), dim3(N / RowN<N>::RPW, 4), dim3(RowN<N>::NT), 0, c->stream, to, Z, V, tw);
+            H = to;
+            return hipGetLastError();
+        } else {
+            return launch_rows<N, C>(c, Z, 4, 0, 1.0, tw);
+        }
+    };
     bool one_pass = false;
     if constexpr (Row1P<N, C>::ok) {
         if (wb) {
             KTimer t(c, K_UXIU);
-            hipLaunchKernelGGL((k_row_uxiu_1p<N, C>), dim3(N), dim3(Row1P<N, C>::NT), 0, c->stream, Vv, U, Xi, V, tw);
+            if (BF == 3 && a.kspace)
+                hipLaunchKernelGGL((k_row_uxiu_1p<N, BF == 3, C>), dim3(N), dim3(Row1P<N, C>::NT), 0, c->stream, Vv, U, Xi, V, tw);
+            else
+                hipLaunchKernelGGL((k_row_uxiu_1p<N, 0, C>), dim3(N), dim3(Row1P<N, C>::NT), 0, c->stream, Vv, U, Xi, V, tw);
             JW_TRY(hipGetLastError());
             one_pass = true;
         }
@@ -571,14 +611,15 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
         }
         JW_TRY((launch_rows<N, C>(c, Vv, 8, 1, 1.0, tw)));
     }
+    JW_TRY(rows_inv(ZA, Xi, HA));
     {
         KTimer t(c, K_COL_KMULT);
         JW_TRY((col_pass<N, BF>(c, ZB, Vv, Vv + 4 * V, a.sa_k, a.sqrt_coupling, 0, 1, a.ns, 0, 0)));
     }
-    JW_TRY((launch_rows<N, C>(c, ZB, 4, 0, 1.0, tw)));
+    JW_TRY(rows_inv(ZB, Xi + 4 * V, HB));
     {
         KTimer t(c, K_UPDATE);
-        hipLaunchKernelGGL((k_update_packed<C, 1>), dim3(g), dim3(256), 0, c->stream, U, ZA, ZB, V, a.sqrt_step,
+        hipLaunchKernelGGL((k_update_packed<C, 1>), dim3(g), dim3(256), 0, c->stream, U, HA, HB, V, a.sqrt_step,
                            a.reunit, a.whole);
         JW_TRY(hipGetLastError());
     }
