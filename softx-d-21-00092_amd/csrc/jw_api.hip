@@ -164,7 +164,7 @@ int evolve_generator_basis(jw_ctx* c, jw_field* U, int nsteps, bool fused, bool 
         if (!ok) return fail(JW_ERR_STATE, "pending injection has %d normals per site, need 16", c->inj_per_site);
         if (fused || large) {
             const jw::StepArgs sa{ns, sa_pos, sa_k, kc == 0, corr, ss, 0, 1, it == 0, it < nsteps - 1, c->noise_kspace,
-                                  it == nsteps - 1};
+                                  it == nsteps - 1 ? U->d : nullptr};
             if (fused) HIP_CHECK(jw::step_fused(c, U->d, Xi, Vv, ZA, ZB, sa));
             else HIP_CHECK(jw::step_large(c, U->d, Xi, Vv, ZA, ZB, sa));
             continue;
@@ -369,7 +369,7 @@ hipError_t batch_group_step(jw_batch* b, BatchGroup& g, int coupling, double ste
                     b->d_step};
     const jw::StepArgs a{ns,      sa_pos,      sa_k,  coupling == JW_SQRT_COUPLING_CONSTANT,
                          coupling == JW_CORRELATED_NOISE_COUPLING, sqrt(step), reunit, count, first_noise, next_noise,
-                         b->kspace, 0};
+                         b->kspace, nullptr};
     if (b->fp32)
         return jw::step_fused_f32(g.ctx, (jw::cplxf*)U, (jw::cplxf*)g.Xi, (jw::cplxf*)g.Vv, (jw::cplxf*)g.ZA,
                                   (jw::cplxf*)g.ZB, a);
@@ -403,7 +403,7 @@ int batch_step_all(jw_batch* b, int coupling, double step, const jw::Alpha& al, 
                                    b->fp32 ? (const void*)g.ctx->twf : (const void*)g.ctx->tw};
         }
         const jw::StepArgs a{ga[0].ns, nullptr, nullptr, coupling == JW_SQRT_COUPLING_CONSTANT,
-                             coupling == JW_CORRELATED_NOISE_COUPLING, sqrt(step), reunit, 1, 1, 0, b->kspace, 0};
+                             coupling == JW_CORRELATED_NOISE_COUPLING, sqrt(step), reunit, 1, 1, 0, b->kspace, nullptr};
         HIP_CHECK(b->fp32 ? jw::step_multi_f32(b->stream, ga, ng, a) : jw::step_multi(b->stream, ga, ng, a));
     } else {
         HIP_CHECK(hipEventRecord(b->fork, b->stream));
@@ -1107,7 +1107,7 @@ int jw_evolve_mixed(jw_ctx* c, jw_field* U, int coupling, int kernel, double ste
         const int reunit = reunit_every > 0 && ((it + 1) % reunit_every == 0 || it == nsteps - 1);
         const jw::StepArgs sa{ns,      sa_pos,        sa_k,           coupling == JW_SQRT_COUPLING_CONSTANT,
                               corr,    sqrt(step),    reunit,         1,
-                              it == 0, it < nsteps - 1, c->noise_kspace, 0};
+                              it == 0, it < nsteps - 1, c->noise_kspace, large && it == nsteps - 1 ? U->d : nullptr};
         const hipError_t he = fused ? jw::step_fused_f32(c, U32, Xi, Vv, ZA, ZB, sa)
                               : large ? jw::step_large_f32(c, U32, Xi, Vv, ZA, ZB, sa)
                                     : jw::step_unfused_f32(c, U32, Xi, Vv, ZA, ZB, ns, sa_pos, sa_k,
@@ -1115,7 +1115,7 @@ int jw_evolve_mixed(jw_ctx* c, jw_field* U, int coupling, int kernel, double ste
                                                            sqrt(step), reunit);
         if (he != hipSuccess) rc = fail(JW_ERR_HIP, "%s", hipGetErrorString(he));
     }
-    if (rc == JW_OK && jw::u_convert(c, U32, U->d, 0, uplanes) != hipSuccess) rc = fail(JW_ERR_HIP, "U conversion failed");
+    if (rc == JW_OK && !large && jw::u_convert(c, U32, U->d, 0, uplanes) != hipSuccess) rc = fail(JW_ERR_HIP, "U conversion failed");
     c->layout = saved_layout;
     return rc;
 }

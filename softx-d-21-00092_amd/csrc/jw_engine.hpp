@@ -1484,7 +1484,7 @@ static hipError_t step_fused_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     {
         KTimer t(c, kcls[3]);
         hipLaunchKernelGGL((k_row_update<N, BF, C>), dim3(N, 1, a.nbatch), dim3(RowE<N>::NT), 0, c->stream, U, ZA, ZB, V,
-                           a.sqrt_step, a.reunit, a.whole, tw, next_noise, Xi, a.ns, a.sa_pos);
+                           a.sqrt_step, a.reunit, a.whole != nullptr, tw, next_noise, Xi, a.ns, a.sa_pos);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return hipSuccess;

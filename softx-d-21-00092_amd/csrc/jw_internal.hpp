@@ -152,7 +152,8 @@ struct StepArgs {
     int first_noise;         // generate this step's xi first (else the previous update did)
     int next_noise;          // the update pass also generates the next step's xi
     int kspace;              // xi drawn per mode in the first column pass (no noise pass)
-    int whole;               // write row 2 of U as well (FP64 field, last step of a call)
+    cplx* whole;             // the field that this step, a call's last, leaves whole: row 2 of U as well (FP64), or all
+                             // nine planes in FP64 instead of U (FP32 on a large lattice); otherwise nullptr
 };
 hipError_t step_fused(jw_ctx* c, cplx* U, cplx* Xi, cplx* Vv, cplx* ZA, cplx* ZB, const StepArgs& a);
 hipError_t step_fused_f32(jw_ctx* c, cplxf* U, cplxf* Xi, cplxf* Vv, cplxf* ZA, cplxf* ZB, const StepArgs& a);

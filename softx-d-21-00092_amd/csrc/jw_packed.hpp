@@ -316,9 +316,11 @@ __global__ __launch_bounds__(256) void k_uxiu_packed(C* __restrict__ Vv, const C
     }
 }
 
+// whole: a call's last step leaves all nine planes there, in FP64 (U itself, or the field
+// of a mixed call, whose own pass back, R 6 FP32 W 9 FP64, took 2.4 ms at N = 8192 after 2.5 here)
 template <typename C, int U6 = 0>
-__global__ __launch_bounds__(256) void k_update_packed(C* __restrict__ U, const C* __restrict__ ZA,
-                                                       const C* __restrict__ ZB, size_t V, double ss, int reunit, int whole) {
+__global__ __launch_bounds__(256) void k_update_packed(C* U, const C* __restrict__ ZA, const C* __restrict__ ZB, size_t V,
+                                                       double ss, int reunit, cplx* whole) {
     GRID_STRIDE(i, V) {
         double ha[8], hb[8];
 #pragma unroll
@@ -333,12 +335,15 @@ __global__ __launch_bounds__(256) void k_update_packed(C* __restrict__ U, const 
         load_u_d<U6>(u, U, V, i);
         m3 r = mmul(mmul(eb, u), ea);
         if (reunit) r = su3_project(r);
+        if (U6 && whole) {      // rows 0 and 1 as the storage type holds them
 #pragma unroll
-        for (int k = 0; k < (U6 ? 6 : 9); k++) U[k * V + i] = mkc<C>(r.m[k].x, r.m[k].y);
-        if (U6 && whole) {      // a call's last step leaves all nine entries
+            for (int k = 0; k < 6; k++) r.m[k] = to_d(mkc<C>(r.m[k].x, r.m[k].y));
             row2_of(r.m);
 #pragma unroll
-            for (int k = 6; k < 9; k++) U[k * V + i] = mkc<C>(r.m[k].x, r.m[k].y);
+            for (int k = 0; k < 9; k++) whole[k * V + i] = r.m[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < (U6 ? 6 : 9); k++) U[k * V + i] = mkc<C>(r.m[k].x, r.m[k].y);
         }
     }
 }
@@ -383,7 +388,7 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
     JW_TRY(fft2d_t(c, ZB, 4, 0, s));
     {
         KTimer t(c, K_UPDATE);
-        hipLaunchKernelGGL(k_update_packed<C>, dim3(g), dim3(256), 0, c->stream, U, ZA, ZB, V, ss, reunit, 0);
+        hipLaunchKernelGGL(k_update_packed<C>, dim3(g), dim3(256), 0, c->stream, U, ZA, ZB, V, ss, reunit, (cplx*)nullptr);
         JW_TRY(hipGetLastError());
     }
 #undef JW_TRY
