@@ -95,7 +95,9 @@ __device__ __forceinline__ m3 mmul(const m3& a, const m3& b) {
 }
 
 // the same in FP32 (the mixed-precision form's products of exponentials and
-// links: its fields carry FP32 rounding anyway)
+// links: its fields carry FP32 rounding anyway).  Each product is rounded by itself and
+// then added: with the products accumulated by fused multiply-adds, the small ones next
+// to the exponential's diagonal take two roundings of the sum's size instead of one.
 struct m3f { cplxf m[9]; };
 
 __device__ __forceinline__ m3f mmul(const m3f& a, const m3f& b) {
@@ -104,10 +106,8 @@ __device__ __forceinline__ m3f mmul(const m3f& a, const m3f& b) {
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++) {
-            cplxf s = cmul(a.m[3 * i], b.m[j]);
-            s = cmad(s, a.m[3 * i + 1], b.m[3 + j]);
-            s = cmad(s, a.m[3 * i + 2], b.m[6 + j]);
-            c.m[3 * i + j] = s;
+            const cplxf s = cadd(cmul(a.m[3 * i], b.m[j]), cmul(a.m[3 * i + 1], b.m[3 + j]));
+            c.m[3 * i + j] = cadd(s, cmul(a.m[3 * i + 2], b.m[6 + j]));
         }
     return c;
 }
