@@ -415,7 +415,8 @@ hipError_t correlator(jw_ctx* c, const cplx* U, cplx* planes, double* corr) {
     return hipGetLastError();
 }
 
-// average_and_symmetrize on reals, sites s0 .. s0 + n - 1 into host memory (same operations)
+// average_and_symmetrize on reals, sites s0 .. s0 + n - 1 into host memory (same operations).
+// Launched from the lanes' host threads, so untimed: a KTimer writes the context's counters.
 __global__ __launch_bounds__(256) void k_symmetrize_real(const double* __restrict__ in, double* __restrict__ out, int N, size_t s0,
                                                          size_t n) {
 #pragma clang fp contract(off)
@@ -430,7 +431,6 @@ __global__ __launch_bounds__(256) void k_symmetrize_real(const double* __restric
 }
 
 hipError_t symmetrize_real(jw_ctx* c, const double* in, double* out, size_t s0, size_t n) {
-    KTimer t(c, K_OBS);
     hipLaunchKernelGGL(k_symmetrize_real, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, in, out, c->N, s0, n);
     return hipGetLastError();
 }
