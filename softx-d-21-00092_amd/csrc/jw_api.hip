@@ -595,12 +595,19 @@ int jw_create(jw_ctx** out, int N, int device) {
         return fail(JW_ERR_HIP, "stream creation failed");
     }
     // twiddles exp(-2 pi i m/N) rounded from long double (FP64 and FP32)
-    std::vector<cplx> tw(N);
-    std::vector<float2> twf(N);
-    for (int m = 0; m < N; m++) {
-        long double ang = -2.0L * 3.141592653589793238462643383279502884L * (long double)m / (long double)N;
-        tw[m] = make_double2((double)cosl(ang), (double)sinl(ang));
-        twf[m] = make_float2((float)cosl(ang), (float)sinl(ang));
+    const std::vector<int> ex = jw::reg_tables(N);
+    const size_t nt = ex.size();
+    std::vector<cplx> tw(nt);
+    std::vector<float2> twf(nt);
+    for (size_t i = 0; i < nt; i++) {
+        if (i >= (size_t)N) {
+            tw[i] = tw[ex[i]];
+            twf[i] = twf[ex[i]];
+            continue;
+        }
+        long double ang = -2.0L * 3.141592653589793238462643383279502884L * (long double)i / (long double)N;
+        tw[i] = make_double2((double)cosl(ang), (double)sinl(ang));
+        twf[i] = make_float2((float)cosl(ang), (float)sinl(ang));
     }
     // momenta.h:90-125 per axis: 4 pow(sin(pi k/N), 2) and sin(2 pi k/N)
     std::vector<double> q4(N), sb(N);
@@ -608,13 +615,13 @@ int jw_create(jw_ctx** out, int N, int device) {
         q4[k] = 4.0 * pow(sin(M_PI * k / (1.0 * N)), 2.0);
         sb[k] = sin(2.0 * M_PI * k / (1.0 * N));
     }
-    if (hipMalloc(&c->tw, N * sizeof(cplx)) != hipSuccess || hipMalloc(&c->q4, N * sizeof(double)) != hipSuccess ||
-        hipMalloc(&c->sb, N * sizeof(double)) != hipSuccess || hipMalloc(&c->twf, N * sizeof(float2)) != hipSuccess) {
+    if (hipMalloc(&c->tw, nt * sizeof(cplx)) != hipSuccess || hipMalloc(&c->q4, N * sizeof(double)) != hipSuccess ||
+        hipMalloc(&c->sb, N * sizeof(double)) != hipSuccess || hipMalloc(&c->twf, nt * sizeof(float2)) != hipSuccess) {
         jw_destroy(c);
         return fail(JW_ERR_ALLOC, "table allocation failed");
     }
-    hipMemcpy(c->tw, tw.data(), N * sizeof(cplx), hipMemcpyHostToDevice);
-    hipMemcpy(c->twf, twf.data(), N * sizeof(float2), hipMemcpyHostToDevice);
+    hipMemcpy(c->tw, tw.data(), nt * sizeof(cplx), hipMemcpyHostToDevice);
+    hipMemcpy(c->twf, twf.data(), nt * sizeof(float2), hipMemcpyHostToDevice);
     hipMemcpy(c->q4, q4.data(), N * sizeof(double), hipMemcpyHostToDevice);
     hipMemcpy(c->sb, sb.data(), N * sizeof(double), hipMemcpyHostToDevice);
     *out = c;

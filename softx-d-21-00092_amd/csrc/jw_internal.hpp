@@ -6,6 +6,8 @@
 #include <stdint.h>
 #include <stddef.h>
 
+#include <vector>
+
 #include "../../include/jimwlk.h"
 
 // intermediate-plane layout of the fused step unless jw_set_fused selects one:
@@ -33,6 +35,22 @@ struct NoiseSrc {
     const uint32_t* stepp; // device step counter (read instead of step when set)
 };
 
+// Points a thread holds of a transform of length N >= 64 in registers (jw_regfft.hpp)
+constexpr int reg_points(int N) { return N == 64 ? 4 : (N <= 512 ? 8 : (N <= 4096 ? 16 : 32)); }
+// The twiddle table of such a transform: exponent i of w_N at entry i < N, then the
+// exponents of its steps 1 and 3 in the order in which their threads read them
+inline std::vector<int> reg_tables(int N) {
+    std::vector<int> e;
+    for (int i = 0; i < N; i++) e.push_back(i);
+    if (N < 64) return e;
+    const int PT = reg_points(N), T = N / PT, N3 = T / PT;
+    for (int k = 1; k < PT; k++)
+        for (int j = 0; j < T; j++) e.push_back(j * k);
+    for (int k = 1; k < PT; k++)
+        for (int m = 0; m < N3; m++) e.push_back(PT * m * k);
+    return e;
+}
+
 struct Alpha {
     double lambda_L, mu0_over_lambda, freeze_c, beta0;
 };
@@ -50,7 +68,7 @@ struct jw_ctx {
     size_t V;
     int device;
     hipStream_t stream;
-    jw::cplx* tw;          // tw[m] = exp(-2 pi i m / N), m < N
+    jw::cplx* tw;          // tw[i] = exp(-2 pi i e_i / N), e = reg_tables(N): e_i = i for i < N
     float2* twf;           // the same in FP32 (mixed-precision form)
     double* q4;            // q4[k] = 4 pow(sin(pi k / N), 2)   (momenta.h:111)
     double* sb;            // sb[k] = sin(2 pi k / N)           (momenta.h:119-120)

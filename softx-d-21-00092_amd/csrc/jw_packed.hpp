@@ -142,10 +142,16 @@ __global__ __launch_bounds__((ColR<N, C>::NT)) void k_fft_cols_reg(C* __restrict
     for (int r = 0; r < F::PT; r++) (data + (DIR < 0 ? rq(r) : r * RS))[e] = cscale(v[r], (T)scale);
 }
 
-template <int N, typename C>
+// REG: the transforms in registers.  The FP32 2-D transforms (the unfused sequence of the
+// mixed form) and the row passes beside the 16-byte column strips keep the radix-8 passes in
+// LDS: the 16- and 32-point factors' constants, rounded to FP32, cost more error there than
+// the passes saved (rms of forward, multiply, inverse, LDS / registers: N = 1024 2.23e-7 /
+// 2.29e-7, 2048 2.34e-7 / 2.41e-7, 4096 2.48e-7 / 2.59e-7; FP64 4.38e-16 / 4.11e-16,
+// 4.57e-16 / 4.51e-16, 5.04e-16 / 4.69e-16).
+template <int N, bool REG, typename C>
 static hipError_t launch_rows(jw_ctx* c, C* p, int np, int dir, double scale, const C* tw) {
     KTimer t(c, K_FFT_ROWS);
-    if constexpr (N >= 64) {
+    if constexpr (REG && N >= 64) {
         dim3 grid(N / RowN<N>::RPW, np), block(RowN<N>::NT);
         if (dir) hipLaunchKernelGGL((k_fft_rows_reg<N, -1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
         else hipLaunchKernelGGL((k_fft_rows_reg<N, +1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
@@ -158,10 +164,10 @@ static hipError_t launch_rows(jw_ctx* c, C* p, int np, int dir, double scale, co
     return hipGetLastError();
 }
 
-template <int N, typename C>
+template <int N, bool REG, typename C>
 static hipError_t launch_cols(jw_ctx* c, C* p, int np, int dir, double scale, const C* tw) {
     KTimer t(c, K_FFT_COLS);
-    if constexpr (N >= 64) {
+    if constexpr (REG && N >= 64) {
         dim3 grid(N / ColR<N, C>::W, np), block(ColR<N, C>::NT);
         if (dir) hipLaunchKernelGGL((k_fft_cols_reg<N, -1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
         else hipLaunchKernelGGL((k_fft_cols_reg<N, +1, C>), grid, block, 0, c->stream, p, c->V, tw, scale);
@@ -199,14 +205,14 @@ static const C* twiddles_of(const jw_ctx* c) {
 
 template <typename C>
 static hipError_t fft_rows_t(jw_ctx* c, C* planes, int nplanes, int dir, double scale) {
-#define CALL_ROWS(n) launch_rows<n, C>(c, planes, nplanes, dir, scale, twiddles_of<C>(c))
+#define CALL_ROWS(n) launch_rows<n, sizeof(C) == sizeof(double2), C>(c, planes, nplanes, dir, scale, twiddles_of<C>(c))
     JW_SIZE_SWITCH(c->N, CALL_ROWS)
 #undef CALL_ROWS
 }
 
 template <typename C>
 static hipError_t fft_cols_t(jw_ctx* c, C* planes, int nplanes, int dir, double scale) {
-#define CALL_COLS(n) launch_cols<n, C>(c, planes, nplanes, dir, scale, twiddles_of<C>(c))
+#define CALL_COLS(n) launch_cols<n, sizeof(C) == sizeof(double2), C>(c, planes, nplanes, dir, scale, twiddles_of<C>(c))
     JW_SIZE_SWITCH(c->N, CALL_COLS)
 #undef CALL_COLS
 }
@@ -495,11 +501,11 @@ __global__ __launch_bounds__((Row1P<N, C>::NT), 1) void k_row_uxiu_1p(C* __restr
             split_exchange<PT, false>(
                 v, [&](int k) { return sub + (m + N3 * (k / N3)) * N3 + ((k % N3) ^ m); },
                 [&](int b) { return sub + b * N3 + (m ^ (b % N3)); });
-            twiddle_powers<PT, +1>(v, tw_fft(tw), PT * m);
+            twiddle<N, 3, +1>(v, tw_fft(tw), m);
             dft_reg<PT, +1>(v);
             split_exchange<PT, true>(
                 v, [&](int a) { return sub + m + N3 * a; }, [&](int k) { return own + k * SUB; });
-            twiddle_powers<PT, +1>(v, tw_fft(tw), j);
+            twiddle<N, 1, +1>(v, tw_fft(tw), j);
             dft_reg<PT, +1>(v);
         }
         {
@@ -541,11 +547,11 @@ __global__ __launch_bounds__((Row1P<N, C>::NT), 1) void k_row_uxiu_1p(C* __restr
             T* sub = pl() + g * SUB;
             T* own = pl() + j;
             dft_reg<PT, -1>(v);
-            twiddle_powers<PT, -1>(v, tw_fft(tw), j);
+            twiddle<N, 1, -1>(v, tw_fft(tw), j);
             split_exchange<PT, true>(
                 v, [&](int k) { return own + k * SUB; }, [&](int a) { return sub + m + N3 * a; });
             dft_reg<PT, -1>(v);
-            twiddle_powers<PT, -1>(v, tw_fft(tw), PT * m);
+            twiddle<N, 3, -1>(v, tw_fft(tw), m);
             split_exchange<PT, false>(
                 v, [&](int b) { return sub + b * N3 + (m ^ (b % N3)); },
                 [&](int k) { return sub + (m + N3 * (k / N3)) * N3 + ((k % N3) ^ m); });
@@ -567,6 +573,7 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     const C* tw = twiddles_of<C>(c);
     const unsigned g = grid_for(V, 256);
     const int wb = a.corr || a.kspace;      // xi~ written back by column A
+    constexpr bool REG = BF == 3 || sizeof(C) == sizeof(double2);
     hipError_t e;
 #define JW_TRY(x) if ((e = (x)) != hipSuccess) return e
     if (!a.kspace) {
@@ -575,7 +582,7 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
             hipLaunchKernelGGL(k_gen_noise_packed<C>, dim3(g), dim3(256), 0, c->stream, Xi, V, a.ns, a.sa_pos);
             JW_TRY(hipGetLastError());
         }
-        JW_TRY((launch_rows<N, C>(c, Xi, 8, 1, 1.0, tw)));
+        JW_TRY((launch_rows<N, REG, C>(c, Xi, 8, 1, 1.0, tw)));
     }
     {
         KTimer t(c, K_COL_KMULT);
@@ -591,7 +598,7 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
             H = to;
             return hipGetLastError();
         } else {
-            return launch_rows<N, C>(c, Z, 4, 0, 1.0, tw);
+            return launch_rows<N, REG, C>(c, Z, 4, 0, 1.0, tw);
         }
     };
     bool one_pass = false;
@@ -607,14 +614,14 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
         }
     }
     if (!one_pass) {
-        if (wb) JW_TRY((launch_rows<N, C>(c, Xi, 8, 0, 1.0, tw)));
+        if (wb) JW_TRY((launch_rows<N, REG, C>(c, Xi, 8, 0, 1.0, tw)));
         {
             KTimer t(c, K_UXIU);
             hipLaunchKernelGGL((k_uxiu_packed<C, 1>), dim3(g), dim3(256), 0, c->stream, Vv, U, wb ? Xi : nullptr, V,
                                a.ns, a.sa_pos);
             JW_TRY(hipGetLastError());
         }
-        JW_TRY((launch_rows<N, C>(c, Vv, 8, 1, 1.0, tw)));
+        JW_TRY((launch_rows<N, REG, C>(c, Vv, 8, 1, 1.0, tw)));
     }
     JW_TRY(rows_inv(ZA, Xi, HA));
     {
