@@ -18,6 +18,7 @@ import numpy as np
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB = os.path.join(HERE, "liboracle.so")
 REF_LIB = os.path.join(HERE, "_ref", "libjw_ref.so")
+REF_SRC = "/root/reference/su3_matrix.h"      # one of the reference's sources, where they are present
 
 SQRT, NOISE, HATTA, FIXED, CORRELATED = 0, 1, 2, 3, 4
 LINEAR, SIN = 0, 1
@@ -38,7 +39,7 @@ def alpha(lambda_L=6.0, mu0_over_lambda=2.5, freeze_c=0.2, beta0=9.0):
 def build(ref=True):
     """Compile liboracle.so (and _ref/libjw_ref.so when the reference tree exists)."""
     subprocess.run(["make", "-s", "-C", HERE, "-B", "oracle"], check=True)
-    if ref and os.path.isfile("/root/reference/su3_matrix.h"):
+    if ref and os.path.isfile(REF_SRC):
         subprocess.run(["make", "-s", "-C", HERE, "-B", "ref"], check=True)
 
 
@@ -283,8 +284,11 @@ class Reference:
 
     def __init__(self, path=REF_LIB):
         if not os.path.exists(path):
-            # a test that asks for it is skipped, as in a tree without the reference
-            raise unittest.SkipTest(f"reference build missing: {path}")
+            # without the reference's sources a test that asks for it is skipped; with them a
+            # library that was not built is an error
+            if not os.path.isfile(REF_SRC):
+                raise unittest.SkipTest(f"reference build missing: {path}")
+            raise RuntimeError(f"reference build missing: {path}")
         self.L = ctypes.CDLL(path)
         assert self.L.ref_lattice_size() == self.N
 
