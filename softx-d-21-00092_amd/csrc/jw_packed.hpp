@@ -1,8 +1,8 @@
 // jw_packed.hpp -- the unfused passes of the generator-basis step, templated on
 // the storage type C (double2: FP64 form, float2: mixed form): the 2-D FFT
 // row and column passes and the per-site kernels (noise, kernel multiply,
-// U xi U^dagger, update).  Site algebra is FP64 in both forms.  Used where the
-// fused passes are not (N outside 64..2048, the LINEAR kernel's 9-component
+// U xi U^dagger, update).  Site algebra is FP64 in both forms, but for U xi U^dagger of
+// the mixed form at N = 8192.  Used where the fused passes are not (N outside 64..2048, the LINEAR kernel's 9-component
 // transforms, jw_set_fused(ctx, 0)).
 #pragma once
 
@@ -436,8 +436,9 @@ static hipError_t step_unfused_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, co
 // the site pass (R 14 W 8) and the forward row FFT of V (R 8 W 8): R 20 W 8.
 // Bound by memory and by its own exchanges in turn (one workgroup a CU): FP32 at N = 8192
 // 4.6 ms (10.7 GB; 5.0 from tiles), where a plane at a time through LDS stages took 7.7 ms.  Against the
-// three passes, two steps at N = 4096 with drawn correlated noise: FP64 18.3 -> 15.5 ms, FP32
-// 10.8 -> 10.0.  FP64 at N = 8192 fits neither LDS nor registers and keeps the three passes.
+// three passes, two steps at N = 4096 with drawn correlated noise: FP64 18.3 -> 15.5 ms, mixed
+// 10.8 -> 10.0 (with FP64 products here as there: 4.3 ms a step, 4.2 with FP32 ones, which
+// put a long step 5% further from FP64).  FP64 at N = 8192 fits neither LDS nor registers and keeps the three passes.
 template <int N, typename C>
 struct Row1P {
     typedef RegFft<N> F;
@@ -445,6 +446,10 @@ struct Row1P {
     static constexpr int NT = 4 * F::T, SPT = N / NT;
     static constexpr int SUB = RegLds<N, 1, T>::SUB, PL = RegLds<N, 1, T>::ELEMS;
     static constexpr bool ok = sizeof(C) == sizeof(float2) || N == 4096;
+    // the products' type: FP64 at N = 4096 in both forms, as in the separate passes; FP32 at 8192
+    static constexpr bool FP64 = N == 4096;
+    typedef typename std::conditional<FP64, m3, m3f>::type M;
+    typedef typename std::conditional<FP64, double, float>::type S;
 };
 // v[k] -> LDS at to(k), v[k] <- LDS from from(k), the real parts and then the imaginary
 // parts; WG: over the workgroup (otherwise inside each wave).  Ends with its reads.
@@ -521,15 +526,15 @@ __global__ __launch_bounds__((Row1P<N, C>::NT), 1) void k_row_uxiu_1p(C* __restr
 #pragma unroll
         for (int q = 0; q < SPT; q++) {
             const size_t i = row0 + tu + q * R::NT;
-            T hh[8];
+            typename R::S hh[8], w[8];
 #pragma unroll
             for (int p = 0; p < 4; p++) {
                 hh[2 * p] = v[4 * q + p].x;
                 hh[2 * p + 1] = v[4 * q + p].y;
             }
-            typename site_mat<C>::type u;
-            load_u(u, U, V, i);
-            T w[8];
+            typename R::M u;
+            if constexpr (R::FP64) load_u_d<1>(u, U, V, i);
+            else load_u(u, U, V, i);
             uxiu_gen(u, hh, w);
 #pragma unroll
             for (int p = 0; p < 4; p++) v[4 * q + p] = mkc<C>(w[2 * p], w[2 * p + 1]);

@@ -51,3 +51,8 @@ def mixed_error(jw, N, space, step, rows):
 
 def test_mixed_8192_errs_no_more_than_radix_8(jw):
     assert mixed_error(jw, 8192, jw.NOISE_MOMENTUM, 1e-4, 8) <= 1.005 * 2.7275e-8
+
+
+# a step this long lets the error of U xi U^dagger through: with its products in FP32 1.52e-6
+def test_mixed_4096_keeps_fp64_products(jw):
+    assert mixed_error(jw, 4096, jw.NOISE_POSITION, 1.0, 4) <= 1.005 * 1.4459e-6
