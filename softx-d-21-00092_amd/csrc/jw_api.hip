@@ -640,7 +640,7 @@ void jw_destroy(jw_ctx* c) {
     if (c->sa16) hipFree(c->sa16);
     if (c->sap) hipFree(c->sap);
     if (c->inj) hipFree(c->inj);
-    jw::lanes_free(c);
+    jw::staging_free(c);
     if (c->ws) hipFree(c->ws);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;

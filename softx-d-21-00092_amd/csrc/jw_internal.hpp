@@ -90,11 +90,14 @@ struct jw_ctx {
     int inj_per_site;      // 0 when no injection is pending
     // Philox stream state for the generators
     uint32_t seed, traj, step;
-    // pinned staging of the host transfers (jw_host.hpp): up to JW_LANES buffers of
-    // lane_cap bytes, allocated on first use, freed with the context
+    // staging of the host transfers (jw_host.hpp), allocated on first use, freed with the
+    // context: one device buffer and up to JW_LANES pinned ones of lane_cap bytes
+    void* stage;
+    size_t stage_cap;
+    int staged;            // transfers that went through the device buffer
     void* lane_pin[JW_LANES];
     hipEvent_t lane_ev[JW_LANES];
-    size_t lane_cap;
+    size_t lane_cap[JW_LANES];
     // workspace: generator-basis planes (packed) and scratch complex planes
     jw::cplx* ws;
     size_t ws_planes;
