@@ -72,13 +72,15 @@ int ensure_sa(jw_ctx* c, int variant, const jw::Alpha& a) {
     return JW_OK;
 }
 
-// the current sa table in 16-row blocks (for the blocked column pass)
-int ensure_sa16(jw_ctx* c) {
+// the current sa table in 16-row blocks (for the one-plane column passes), its columns
+// in the order of the row-major row spectra (perm) or of frequency
+int ensure_sa16(jw_ctx* c, bool perm) {
     if (!c->sa16 && hipMalloc(&c->sa16, c->V * sizeof(double)) != hipSuccess)
         return fail(JW_ERR_ALLOC, "coupling table allocation failed");
-    if (c->sa16_gen == c->sa_gen) return JW_OK;
-    HIP_CHECK(jw::block16(c, c->sa16, c->sa));
+    if (c->sa16_gen == c->sa_gen && c->sa16_perm == perm) return JW_OK;
+    HIP_CHECK(jw::block16(c, c->sa16, c->sa, perm));
     c->sa16_gen = c->sa_gen;
+    c->sa16_perm = perm;
     return JW_OK;
 }
 
@@ -126,19 +128,19 @@ int check_field(const jw_field* f, const jw_ctx* c, int t, const char* name) {
     return JW_OK;
 }
 
-// the column passes of layouts 1, 4 and 8 read the 16-row-blocked sqrt(alpha) table
+// the column passes of layouts 1, 4, 8, 16 and 32 read the 16-row-blocked sqrt(alpha) table
 bool uses_sa16(int layout) { return layout == 1 || layout == 4 || layout == 8 || layout >= 16; }
-// and the register-held column pass of the row-major fused step the one in its
-// column order (the matrix-core stages read the plain table)
-bool uses_sap(const jw_ctx* c, bool fused, bool mfma) { return fused && c->layout == 0 && !mfma; }
+// row spectra in the order in which the row transform ends (RowOrder in jw_engine.hpp)
+bool row_order_fft(bool fused, int layout) { return fused && (layout == 0 || layout == 1 || layout == 16); }
 
 // sqrt(alpha) in k for the fused or large-lattice passes of c->layout (ensure_sa done)
-int k_table(jw_ctx* c, bool fused, bool mfma, const double** sa_k) {
+int k_table(jw_ctx* c, bool fused, const double** sa_k) {
     *sa_k = c->sa;
+    const bool perm = row_order_fft(fused, c->layout);
     if (uses_sa16(c->layout)) {
-        if (int e = ensure_sa16(c)) return e;
+        if (int e = ensure_sa16(c, perm)) return e;
         *sa_k = c->sa16;
-    } else if (uses_sap(c, fused, mfma)) {
+    } else if (perm) {
         if (int e = ensure_sap(c)) return e;
         *sa_k = c->sap;
     }
@@ -215,9 +217,11 @@ int evolve_sin(jw_ctx* c, jw_field* U, int coupling, double step, const jw_alpha
     if ((fused || large) && sa_k) {
         int rc = JW_OK;
         if (!tabs) {
-            rc = k_table(c, fused, false, &sa_k);
-        } else if (uses_sa16(c->layout) || uses_sap(c, fused, false)) {
-            const hipError_t he = uses_sa16(c->layout) ? jw::block16(c, tabs + V, tabs) : jw::perm_columns(c, tabs + V, tabs);
+            rc = k_table(c, fused, &sa_k);
+        } else if (uses_sa16(c->layout) || row_order_fft(fused, c->layout)) {
+            const bool perm = row_order_fft(fused, c->layout);
+            const hipError_t he = uses_sa16(c->layout) ? jw::block16(c, tabs + V, tabs, perm)
+                                                       : jw::perm_columns(c, tabs + V, tabs);
             if (he != hipSuccess) rc = fail(JW_ERR_HIP, "coupling table: %s", hipGetErrorString(he));
             sa_k = tabs + V;
         }
@@ -357,7 +361,7 @@ int batch_tables(BatchGroup& g, int coupling, const jw::Alpha& al, const double*
         *sa_pos = c->sa;
     } else if (coupling == JW_SQRT_COUPLING_CONSTANT || coupling == JW_CORRELATED_NOISE_COUPLING) {
         if (int e = ensure_sa(c, 0, al)) return e;
-        if (int e = k_table(c, true, c->fft_mfma != 0, sa_k)) return e;
+        if (int e = k_table(c, true, sa_k)) return e;
     }
     return JW_OK;
 }
@@ -1098,7 +1102,7 @@ int jw_evolve_mixed(jw_ctx* c, jw_field* U, int coupling, int kernel, double ste
     const int saved_layout = c->layout;
     if (c->layout < 0) c->layout = default_layout(c->N, 1, c->fft_mfma);
     int rc = JW_OK;
-    if ((fused || large) && sa_k) rc = k_table(c, fused, c->fft_mfma != 0, &sa_k);
+    if ((fused || large) && sa_k) rc = k_table(c, fused, &sa_k);
     // the fused and large-lattice passes hold rows 0 and 1 of U (row 2 rebuilt),
     // the unfused sequence all nine entries
     const int uplanes = fused || large ? 6 : 9;

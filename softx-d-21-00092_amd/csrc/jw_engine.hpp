@@ -24,7 +24,8 @@
 //   BF = 0   row-major, row spectra in the order of freq_of_pos.  Column passes take
 //            strips of W adjacent columns, X and Y in registers (k_col_reg), workgroups
 //            mapped so that strips sharing cache lines run on the same XCD.
-//   BF = 3   the same in frequency order: the large lattices, the matrix-core stages.
+//   BF = 3   the same in frequency order: the large lattices.
+//   BF = 5   row-major for the matrix-core stages (k_col_kmult).
 //   BF = 2   the x and y directions interleaved site by site (k_col_kmult).
 //   BF = 4, 8  blocks of BF rows: (x, y) at ((x / BF) N + y) BF + x mod BF, so
 //            that one 128-byte segment holds 8 / BF adjacent columns of BF
@@ -33,6 +34,7 @@
 //            four plane pairs in one workgroup); row passes touch BF-row
 //            segments whose rows are processed on one XCD at neighbouring times.
 //   BF = 1, 16, 32  row-major, one plane at a time over 64-, 32- or 16-byte strips.
+// Row spectra on row-major planes up to N = 2048 are in the order of freq_of_pos.
 // U always stays row-major.
 #pragma once
 
@@ -86,12 +88,12 @@ __device__ __forceinline__ int xcd_strip(int b, int nstrips) {
     return (b % 8) * (nstrips / 8) + b / 8;
 }
 
-// offset of site (x, y) in an intermediate plane of layout BF (0 and 2
-// row-major, 1 row-major for the 64-byte-strip column pass, 3 row-major in frequency
-// order: the matrix-core column stages and the large lattices, 4 and 8 row blocks)
+// offset of site (x, y) in an intermediate plane of layout BF (4 and 8 row blocks, the
+// others row-major)
+constexpr bool row_blocks_of(int BF) { return BF == 4 || BF == 8; }
 template <int N, int BF>
 __device__ __forceinline__ size_t lay(int x, int y) {
-    if constexpr (BF <= 3 || BF >= 16) return (size_t)x * N + y;
+    if constexpr (!row_blocks_of(BF)) return (size_t)x * N + y;
     else return ((size_t)(x / BF) * N + y) * BF + (x % BF);
 }
 
@@ -106,25 +108,30 @@ __device__ __forceinline__ size_t pat(int q, int x, int y, size_t V) {
     else return (size_t)q * V + lay<N, BF>(x, y);
 }
 
-// Row spectra on row-major planes (BF = 0) are stored in the order in which the
+// Row spectra on row-major planes are stored in the order in which the
 // row transform ends: position s = q T + j holds the frequency of v[q] in thread j,
 // so that a wave writes and reads whole contiguous runs (in frequency order its
-// 64 elements are eight runs of 8; FP32 U xi~ U^dagger at N = 2048 242 against 195 us).  The column
-// pass takes columns independently and needs only their frequency.
+// 64 elements are eight runs of 8; FP32 U xi~ U^dagger at N = 2048 242 against 195 us).  A column
+// pass takes columns independently and needs only their frequency.  Interleaved and
+// blocked planes keep frequency order, as do the large lattices.
+template <int N, int BF>
+struct RowOrder {
+    static constexpr bool fft = N <= 2048 && (BF == 0 || BF == 1 || BF == 5 || BF == 16);
+};
 template <int N, int BF>
 __device__ __forceinline__ int freq_of_pos(int s) {
     typedef RegFft<N> F;
-    if constexpr (BF != 0) return s;
+    if constexpr (!RowOrder<N, BF>::fft) return s;
     else return reg_freq<N>(s % F::T / F::N3, s % F::N3, 0) + reg_freq_q<N>(s / F::T);
 }
 // position of v[q] in thread j: pos0(j) + posq(q)
 template <int N, int BF>
 __device__ __forceinline__ int pos0(int j) {
-    return BF == 0 ? j : reg_freq<N>(j / RegFft<N>::N3, j % RegFft<N>::N3, 0);
+    return RowOrder<N, BF>::fft ? j : reg_freq<N>(j / RegFft<N>::N3, j % RegFft<N>::N3, 0);
 }
 template <int N, int BF>
 __device__ __forceinline__ constexpr int posq(int q) {
-    return BF == 0 ? q * RegFft<N>::T : reg_freq_q<N>(q);
+    return RowOrder<N, BF>::fft ? q * RegFft<N>::T : reg_freq_q<N>(q);
 }
 
 // lattice row of row-pass block b.  Blocks are dealt round-robin to the 8 XCDs;
@@ -132,7 +139,7 @@ __device__ __forceinline__ constexpr int posq(int q) {
 // consecutive turns (a bijection on [0, N) for N a multiple of 8 BF).
 template <int N, int BF>
 __device__ __forceinline__ int row_of_block(int b) {
-    if constexpr (BF <= 3 || BF >= 16) return b;
+    if constexpr (!row_blocks_of(BF)) return b;
     else {
         static_assert(N % (8 * BF) == 0, "blocked layout needs N a multiple of 8 BF");
         const int t = b >> 3, xcd = b & 7;
@@ -705,7 +712,7 @@ __device__ __forceinline__ void col_kmult_body(C* lds, BlockIx bi, C* __restrict
     typedef typename scalar_of<C>::type T;
     typedef ColE<N, C, CORR> CE;
     constexpr int W = CE::W, NT = CE::NT, PER = CE::PER, PAIRS = CE::PAIRS;
-    constexpr int S2 = 2 * W;
+    constexpr int S2 = 2 * W, BF = PI ? 2 : 5;
     const int tid = bi.tid;
     const auto twl = tw_source<N, sizeof(C) == sizeof(float2)>(tw);
     const int strip = xcd_strip(bi.bx, N / W);
@@ -750,12 +757,12 @@ __device__ __forceinline__ void col_kmult_body(C* lds, BlockIx bi, C* __restrict
 #pragma unroll
     for (int q = 0; q < PAIRS; q++) {
         const int pr = tk + q * NT;
-        const int kx = pr / W, c = pr % W, ky = col0 + c;
-        const size_t k = (size_t)kx * N + ky;
+        const int kx = pr / W, c = pr % W, ky = freq_of_pos<N, BF>(col0 + c);
+        const size_t k = (size_t)kx * N + col0 + c;                 // sa is stored by position
         C vx, vy;
         if constexpr (GEN) {
             T g[4];
-            kspace_normals4((uint32_t)k, nk.step, nk.tag, bi.by, nk.seed, nk.traj, g);
+            kspace_normals4((uint32_t)(kx * N + ky), nk.step, nk.tag, bi.by, nk.seed, nk.traj, g);
             vx = mkc<C>(g[0] * (T)N, g[1] * (T)N);          // sqrt(V) = N
             vy = mkc<C>(g[2] * (T)N, g[3] * (T)N);
         } else {
@@ -931,9 +938,9 @@ __global__ __launch_bounds__((ColB<N, BF, C>::NT), (ColB<N, BF, C>::WAVES)) void
 #pragma unroll
         for (int q = 0; q < PER; q++) {
             const int pr = t + q * NT;
-            const int kx = pr % N, c = pr / N, ky = y0 + c;
+            const int kx = pr % N, c = pr / N, ky = freq_of_pos<N, BF>(y0 + c);
             const int l = lpos<1, PN, 4>(kx, c);
-            const size_t k16 = ((size_t)(kx >> 4) * N + ky) * 16 + (kx & 15);
+            const size_t k16 = ((size_t)(kx >> 4) * N + y0 + c) * 16 + (kx & 15);      // sa16 is stored by position
             C v;
             if constexpr (GEN) {
                 if (d == 0) {
@@ -1376,7 +1383,7 @@ static hipError_t col_pass(jw_ctx* c, C* Z, C* X, C* Y, const double* sa_k, int 
     const size_t V = c->V;
     const C* tw = twiddles<C>(c);
 #define JW_COL_ARGS Z, X, Y, V, sqrt_coupling, c->q4, c->sb, sa_k, tw, ns, noise_scale
-    if constexpr (BF == 3 && N <= 2048) {
+    if constexpr (BF == 5) {
         // split-BF16 matrix-core radix-16 stages (FP32 storage)
         const dim3 grid(N / ColE<N, C>::W, 4, nbatch);
         if (gen)
@@ -1497,7 +1504,7 @@ hipError_t step_fused_layout(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, const 
     switch (c->layout) {
         case 0:
             if constexpr (sizeof(C) == sizeof(float2))
-                if (c->fft_mfma) return step_fused_n<N, 3>(c, U, Xi, Vv, ZA, ZB, a, kcls);
+                if (c->fft_mfma) return step_fused_n<N, 5>(c, U, Xi, Vv, ZA, ZB, a, kcls);
             return step_fused_n<N, 0>(c, U, Xi, Vv, ZA, ZB, a, kcls);
         case 1: return step_fused_n<N, 1>(c, U, Xi, Vv, ZA, ZB, a, kcls);
         case 2: return step_fused_n<N, 2>(c, U, Xi, Vv, ZA, ZB, a, kcls);

@@ -77,10 +77,12 @@ struct jw_ctx {
     int sa_variant;        // -1 none, 0 kernel formula, 1 noise formula
     jw::Alpha sa_params;
     unsigned sa_gen;       // bumped whenever sa is rebuilt
-    // k-space sqrt(alpha) in 16-row blocks for the blocked column pass:
-    // sa16[((kx / 16) N + ky) 16 + kx mod 16] = sa[kx N + ky]
+    // k-space sqrt(alpha) in 16-row blocks for the one-plane column passes:
+    // sa16[((kx / 16) N + s) 16 + kx mod 16] = sa[kx N + ky], ky = s, or the
+    // frequency of position s in a row-major row spectrum (sa16_perm)
     double* sa16;
     unsigned sa16_gen;     // sa_gen it was built from (0: never)
+    bool sa16_perm;
     // k-space sqrt(alpha) with ky in the order of the fused step's row-major row
     // spectra: sap[kx N + s] = sa[kx N + frequency of position s]
     double* sap;
@@ -202,7 +204,7 @@ hipError_t u_convert(jw_ctx* c, cplxf* u32, cplx* u64, int to_f32, int planes);
 // row 2 of a 9-plane FP64 U rebuilt from rows 0 and 1 (on stream s)
 hipError_t u_rebuild(jw_ctx* c, cplx* U, hipStream_t s);
 hipError_t step_inc(hipStream_t s, uint32_t* step);
-hipError_t block16(jw_ctx* c, double* out, const double* in);
+hipError_t block16(jw_ctx* c, double* out, const double* in, bool perm);
 hipError_t perm_columns(jw_ctx* c, double* out, const double* in);
 
 // observables

@@ -20,9 +20,28 @@ __global__ __launch_bounds__(256) void k_block16(double* __restrict__ out, const
     }
 }
 
-hipError_t block16(jw_ctx* c, double* out, const double* in) {
+// the same with its columns in the order of the row-major row spectra
+template <int N>
+__global__ __launch_bounds__(256) void k_block16_perm(double* __restrict__ out, const double* __restrict__ in) {
+    GRID_STRIDE(i, (size_t)N * N) {
+        const int kx = (int)(i / N), s = (int)(i % N);
+        out[((size_t)(kx >> 4) * N + s) * 16 + (kx & 15)] = in[(size_t)kx * N + freq_of_pos<N, 0>(s)];
+    }
+}
+
+hipError_t block16(jw_ctx* c, double* out, const double* in, bool perm) {
     if (c->N % 16) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_block16, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, out, in, c->N);
+    if (!perm) {
+        hipLaunchKernelGGL(k_block16, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, out, in, c->N);
+        return hipGetLastError();
+    }
+#define JW_BLOCK(n, C) \
+    case n: hipLaunchKernelGGL(k_block16_perm<n>, dim3(grid_for(c->V, 256)), dim3(256), 0, c->stream, out, in); break;
+    switch (c->N) {
+        JW_FUSED_SIZES(JW_BLOCK, cplx)
+        default: return hipErrorInvalidValue;
+    }
+#undef JW_BLOCK
     return hipGetLastError();
 }
 
