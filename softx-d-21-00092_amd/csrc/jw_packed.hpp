@@ -645,8 +645,9 @@ static hipError_t step_large_n(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
 }
 
 // the column strips of a large lattice: the register-held strips of layout 0 (FP32
-// at both sizes, FP64 at N = 4096), or one plane at a time over 16-byte segments
-// (layout 32; FP64 at N = 8192 has no other)
+// at both sizes, FP64 at N = 4096), X and Y in LDS for the matrix-core stages on layout 0 (mixed,
+// N = 4096), or one plane at a time over 16-byte segments (layout 32; FP64 at N = 8192 has
+// no other)
 template <typename C>
 static hipError_t step_large_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, const StepArgs& a) {
     if (a.nbatch != 1) return hipErrorInvalidValue;
@@ -657,6 +658,8 @@ static hipError_t step_large_t(jw_ctx* c, C* U, C* Xi, C* Vv, C* ZA, C* ZB, cons
     }
     if (c->N == 4096) {
         if (c->layout == 32) return step_large_n<4096, 32>(c, U, Xi, Vv, ZA, ZB, a);
+        if constexpr (sizeof(C) == sizeof(float2))
+            if (c->fft_mfma) return step_large_n<4096, 5>(c, U, Xi, Vv, ZA, ZB, a);
         return step_large_n<4096, 3>(c, U, Xi, Vv, ZA, ZB, a);
     }
     return hipErrorInvalidValue;
