@@ -1484,7 +1484,10 @@ int jw_batch_evolve(jw_batch* b, int coupling, int kernel, double step, const jw
     // previous call's graph (still running on b->stream) reads, and replaces
     // that graph: wait for the previous call's work first.
     if (!same_key) HIP_CHECK(hipStreamSynchronize(b->stream));
-    if (int e = batch_tune(b, coupling, step, al)) return e;
+    // one launch per kernel class runs row-major planes and FP32 butterflies: no layout to
+    // choose, and none but theirs for the coupling tables
+    if (b->launch == 1) batch_rowmajor(b);
+    else if (int e = batch_tune(b, coupling, step, al)) return e;
     if (b->launch < 0)
         if (int e = batch_tune_launch(b, coupling, step, al)) return e;
     if (b->graph && !same_key) {
