@@ -348,6 +348,10 @@ const char* jw_kernel_name(int which);
 int jw_calibration_copy(jw_ctx* ctx, int nplanes);
 /* exp(i s H(h)) for n generator vectors h (8 reals each) -> n 3x3 matrices (18 reals). */
 int jw_su3_exp_gen(jw_ctx* ctx, const double* host_h8, double s, double* host_out18, int n);
+/* The normals that the noise streams form from Philox words, four words to an item: 12
+ * reals, the pair of two 53-bit uniforms in FP64 and in FP32 (jw_noise_philox), then the two
+ * pairs of 32-bit uniforms in FP64 and in FP32 (JW_NOISE_MOMENTUM). */
+int jw_box_muller(jw_ctx* ctx, const uint32_t* host_words4, double* host_out12, int n);
 
 #ifdef __cplusplus
 }

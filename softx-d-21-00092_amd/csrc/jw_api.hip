@@ -1295,6 +1295,28 @@ int jw_su3_exp_gen(jw_ctx* c, const double* h8, double s, double* out18, int n) 
     return JW_OK;
 }
 
+int jw_box_muller(jw_ctx* c, const uint32_t* words, double* out12, int n) {
+    if (!c || !words || !out12 || n < 0) return fail(JW_ERR_ARG, "bad argument");
+    if (n == 0) return JW_OK;
+    const size_t wb = 4 * sizeof(uint32_t) * n, ob = 12 * sizeof(double) * n;
+    uint32_t* dw = nullptr;
+    double* dout = nullptr;
+    HIP_CHECK(hipMalloc(&dw, wb));
+    if (hipMalloc(&dout, ob) != hipSuccess) {
+        hipFree(dw);
+        return fail(JW_ERR_ALLOC, "allocation failed");
+    }
+    hipError_t e = hipMemcpyAsync(dw, words, wb, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = jw::box_muller_batch(c, dw, dout, n);
+    if (e == hipSuccess) e = hipMemcpyAsync(out12, dout, ob, hipMemcpyDeviceToHost, c->stream);
+    const hipError_t s = hipStreamSynchronize(c->stream);
+    hipFree(dw);
+    hipFree(dout);
+    if (e != hipSuccess || s != hipSuccess)
+        return fail(JW_ERR_HIP, "Box-Muller kernel: %s", hipGetErrorString(e != hipSuccess ? e : s));
+    return JW_OK;
+}
+
 
 // ---------------------------------------------------------------- batches
 int jw_batch_create(jw_batch** out, int device, int ngroups, const int* N, const int* count, int fp32) {

@@ -404,10 +404,7 @@ __device__ __forceinline__ void polar_quarter(double rr, uint32_t q, double r, d
     z1 = rs * si;
 }
 
-__device__ __forceinline__ void box_muller_pair(uint32_t site, uint32_t step, uint32_t tag, uint32_t call,
-                                                uint32_t seed, uint32_t traj, double& z0, double& z1) {
-    uint32_t c[4] = {site, step, tag, call};
-    philox4x32_10(c, seed, traj);
+__device__ __forceinline__ void box_muller53(const uint32_t c[4], double& z0, double& z1) {
     // u0 = (a + 1/2) 2^-53 with a the upper 53 bits of (c0, c1), rounded once
     const double u0 = fma((double)c[0], 0x1.0p-32, fma((double)(c[1] >> 11), 0x1.0p-53, 0x1.0p-54));
     const double rr = sqrt_pos(-2.0 * log_unit(u0));
@@ -416,6 +413,13 @@ __device__ __forceinline__ void box_muller_pair(uint32_t site, uint32_t step, ui
     const double r = fma((double)(int32_t)(c[2] - (q << 30)), 0x1.0p-30,
                          fma((double)(c[3] >> 11), 0x1.0p-51, 0x1.0p-52));
     polar_quarter(rr, q, r, z0, z1);
+}
+
+__device__ __forceinline__ void box_muller_pair(uint32_t site, uint32_t step, uint32_t tag, uint32_t call,
+                                                uint32_t seed, uint32_t traj, double& z0, double& z1) {
+    uint32_t c[4] = {site, step, tag, call};
+    philox4x32_10(c, seed, traj);
+    box_muller53(c, z0, z1);
 }
 
 // sqrt(-2 log u) in FP32 from w = u (lo: u < 1/2) or w = 1 - u.  One logarithm for
@@ -442,10 +446,7 @@ __device__ __forceinline__ float radius_f(bool lo, float w) {
 // x = 2 u1 - 1 in (-1, 1): sincospi(x + 1) = -sincospi(x), on the hardware
 // sine and cosine.  Each normal agrees with the FP64 pair to a few FP32 ulps
 // of max(|z|, 1).
-__device__ __forceinline__ void box_muller_pair_f(uint32_t site, uint32_t step, uint32_t tag, uint32_t call,
-                                                  uint32_t seed, uint32_t traj, float& z0, float& z1) {
-    uint32_t c[4] = {site, step, tag, call};
-    philox4x32_10(c, seed, traj);
+__device__ __forceinline__ void box_muller53(const uint32_t c[4], float& z0, float& z1) {
     // u0 = (m0 + 1/2) 2^-53 and u1 = (m1 + 1/2) 2^-53, m the upper 53 bits of a
     // word pair.  53-bit integers to FP32 through FP64 (exact there, then one
     // rounding: the same value as a direct conversion, in fewer instructions).
@@ -462,6 +463,13 @@ __device__ __forceinline__ void box_muller_pair_f(uint32_t site, uint32_t step, 
                                  (double)(int32_t)((c[3] >> 11) * 2u + 1u)) * 0x1.0p-54f;
     z0 = -rr * __builtin_amdgcn_cosf(rev);
     z1 = -rr * __builtin_amdgcn_sinf(rev);
+}
+
+__device__ __forceinline__ void box_muller_pair_f(uint32_t site, uint32_t step, uint32_t tag, uint32_t call,
+                                                  uint32_t seed, uint32_t traj, float& z0, float& z1) {
+    uint32_t c[4] = {site, step, tag, call};
+    philox4x32_10(c, seed, traj);
+    box_muller53(c, z0, z1);
 }
 
 // ---------------------------------------------------------------------------

@@ -223,5 +223,6 @@ hipError_t aos_to_planes(jw_ctx* c, cplx* planes, const cplx* aos, int t, size_t
 // instrumentation and unit-test hooks
 hipError_t calibration_copy(jw_ctx* c, const cplx* a, cplx* b, size_t n);
 hipError_t exp_batch(jw_ctx* c, const double* h8, double s, double* out18, int n);
+hipError_t box_muller_batch(jw_ctx* c, const uint32_t* words, double* out12, int n);
 
 }  // namespace jw

@@ -808,4 +808,30 @@ hipError_t exp_batch(jw_ctx* c, const double* h8, double s, double* out18, int n
     return hipGetLastError();
 }
 
+// the normals of given Philox words, four to a call: 53-bit pair in FP64 and FP32, the two
+// 32-bit pairs in FP64 and FP32
+__global__ __launch_bounds__(256) void k_box_muller_batch(const uint32_t* __restrict__ words, double* __restrict__ out, int n) {
+    GRID_STRIDE(i, (size_t)n) {
+        const uint32_t c[4] = {words[4 * i], words[4 * i + 1], words[4 * i + 2], words[4 * i + 3]};
+        double* o = out + 12 * i;
+        float f[2];
+        box_muller53(c, o[0], o[1]);
+        box_muller53(c, f[0], f[1]);
+        o[2] = f[0];
+        o[3] = f[1];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            box_muller32(c[2 * p], c[2 * p + 1], o[4 + 2 * p], o[5 + 2 * p]);
+            box_muller32(c[2 * p], c[2 * p + 1], f[0], f[1]);
+            o[8 + 2 * p] = f[0];
+            o[9 + 2 * p] = f[1];
+        }
+    }
+}
+
+hipError_t box_muller_batch(jw_ctx* c, const uint32_t* words, double* out12, int n) {
+    hipLaunchKernelGGL(k_box_muller_batch, dim3(grid_for((size_t)n, 256)), dim3(256), 0, c->stream, words, out12, n);
+    return hipGetLastError();
+}
+
 }  // namespace jw

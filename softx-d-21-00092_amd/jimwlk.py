@@ -92,6 +92,7 @@ def lib():
         L.jw_saturation_scale.argtypes = [ctypes.c_int, _dp, _dp, _dp, _dp]
         L.jw_kernel_time.argtypes = [ctypes.c_void_p, ctypes.c_int, _dp, ctypes.POINTER(ctypes.c_long)]
         L.jw_su3_exp_gen.argtypes = [ctypes.c_void_p, _dp, ctypes.c_double, _dp, ctypes.c_int]
+        L.jw_box_muller.argtypes = [ctypes.c_void_p, ctypes.c_void_p, _dp, ctypes.c_int]
         L.jw_timing.argtypes = [ctypes.c_void_p, ctypes.c_int]
         L.jw_set_fused.argtypes = [ctypes.c_void_p, ctypes.c_int]
         L.jw_set_mixed_fft.argtypes = [ctypes.c_void_p, ctypes.c_int]
@@ -345,6 +346,14 @@ class Context:
         out = np.zeros((h8.shape[0], 9), np.complex128)
         _check(lib().jw_su3_exp_gen(self.h, _p(h8), s, _p(out), h8.shape[0]))
         return out.reshape(-1, 3, 3)
+
+    def box_muller(self, words):
+        """Normals of (n, 4) Philox words: columns 0-1 and 2-3 the 53-bit pair in FP64 and FP32,
+        4-7 and 8-11 the 32-bit pairs in FP64 and FP32."""
+        words = np.ascontiguousarray(words, dtype=np.uint32).reshape(-1, 4)
+        out = np.empty((words.shape[0], 12))
+        _check(lib().jw_box_muller(self.h, words.ctypes.data, _p(out), words.shape[0]))
+        return out
 
 
 class Batch:
