@@ -326,11 +326,12 @@ int jw_saturation_scale(int nbins, const double* rbar, const double* Sbin, const
  * taking one plane at a time over 32-byte column strips (two workgroups per CU
  * in FP64); 8: one plane at a time over 16-byte strips (N = 4096 and 8192
  * only).  At N = 4096 modes 0, 1, 2 and 8 exist, at N = 8192 modes 0, 1 and 8
- * (the column strips that fit LDS); others are JW_ERR_UNSUPPORTED there
- * (2..8 for measurement). */
+ * (mode 1 there: strips held in registers in the mixed form, those of mode 8 in
+ * FP64); others are JW_ERR_UNSUPPORTED there (2..8 for measurement). */
 int jw_set_fused(jw_ctx* ctx, int mode);
 /* The column transforms of the mixed-precision form (jw_evolve_mixed, fused
- * passes, row-major layout).  mode 0 (default): FP32 radix-8/4/2 butterflies;
+ * passes, row-major layout; at N = 4096 and 8192 by default on the strips of
+ * jw_set_fused mode 8).  mode 0 (default): FP32 radix-8/4/2 butterflies;
  * 1: the radix-16 stages as DFT-matrix products on the matrix cores in split
  * BF16 (x = hi + lo, three products lo.hi + hi.lo + hi.hi accumulated in FP32,
  * v_mfma_f32_32x32x16_bf16), the remaining stage in FP32 butterflies: about

@@ -147,9 +147,10 @@ int k_table(jw_ctx* c, bool fused, const double** sa_k) {
     return JW_OK;
 }
 
-// the intermediate layout when none is selected: row-major planes, whose column pass holds its strip in registers; 16-byte strips
-// one plane at a time for FP64 at N = 8192 (two planes of one column take the
-// registers of more than a CU) and for the matrix-core stages of the large lattices
+// the intermediate layout when none is selected: row-major planes, whose column pass holds
+// its strip in registers; 16-byte strips one plane at a time for FP64 at N = 8192 (two planes
+// of one column take the registers of more than a CU) and for the matrix-core stages of the
+// large lattices
 int default_layout(int N, int fp32, int mfma) {
     if (!fp32) return N == 8192 ? 32 : 0;
     return N >= 4096 && mfma ? 32 : 0;
@@ -1231,8 +1232,8 @@ int jw_set_fused(jw_ctx* c, int mode) {
     if (!c) return fail(JW_ERR_ARG, "null context");
     static const int layouts[9] = {0, JW_DEFAULT_LAYOUT, 0, 4, 8, 1, 2, 16, 32};
     if (mode < 0 || mode > 8) return fail(JW_ERR_ARG, "fused mode %d: expected 0..8", mode);
-    // N = 4096 runs column strips of layouts 0 and 32, N = 8192 of layout 32;
-    // layout 32 exists for those two sizes only
+    // N = 4096 runs column strips of layouts 0 and 32; N = 8192 of layout 32, and of 0 in the
+    // mixed form by default (default_layout).  Layout 32 exists for those two sizes only.
     const bool large = jw::large_supported(c->N);
     if (mode > 1 && ((large && !(mode == 8 || (c->N == 4096 && mode == 2))) || (!large && mode == 8)))
         return fail(JW_ERR_UNSUPPORTED, "fused mode %d is not available at N = %d", mode, c->N);

@@ -332,9 +332,12 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
 // instead of 130 FP64 instructions per pair.  The fused multiply-adds are written out
 // and no others are formed: every kernel gives the same bits.
 
-// log u for a normal u in (0, 1]: u = 2^e m, m in [sqrt(1/2), sqrt 2);
-// log m = 2 atanh(s), s = f / (2 + f), f = m - 1, as (f - f^2/2) + s (f^2/2 + R),
-// R = s^2 P(s^2) with P fitted (relative error 9e-18 of log m)
+// log u for a normal u in (0, 1], by the argument reduction and the summation of the
+// logarithm in fdlibm (Sun Microsystems, 1993; published with its derivation, and the form
+// of the C libraries descended from it): u = 2^e m, m in [sqrt(1/2), sqrt 2), the exponent
+// taken after adding the distance of sqrt(1/2)'s upper word from one's; log m = 2 atanh(s), s =
+// f / (2 + f), f = m - 1, as (f - f^2/2) + s (f^2/2 + R).  R = s^2 P(s^2), with P
+// fitted here (relative error 9e-18 of log m), and the division by Newton steps.
 __device__ __forceinline__ double log_unit(double u) {
 #pragma clang fp contract(off)
     uint32_t hi = (uint32_t)__double2hiint(u) + (0x3ff00000u - 0x3fe6a09eu);
@@ -362,7 +365,8 @@ __device__ __forceinline__ double log_unit(double u) {
     return fma(k, 0x1.62e42fef00000p-1, fh + (fl + t));
 }
 
-// sqrt x, x >= 0 and not subnormal
+// sqrt x, x >= 0 and not subnormal: Goldschmidt's iteration (1964) from the hardware's
+// reciprocal square root, and one correction by the residual x - g^2
 __device__ __forceinline__ double sqrt_pos(double x) {
 #pragma clang fp contract(off)
     const double y = __builtin_amdgcn_rsq(x);

@@ -513,15 +513,15 @@ __global__ __launch_bounds__(RowE<N>::NT, RowWaves<C>::value) void k_row_uxiu_co
 // of X and of Y; LDS holds one plane of the strip for the exchanges, and the
 // (4 sin^2, sin) table of kx.
 //
-// What bounds it: the loaded pass moves 12 planes at 3.1-3.2 TB/s (FP64 and FP32
+// What bounds it: the loaded pass moves 12 planes at 2.7-2.8 TB/s (FP64 and FP32
 // at N = 2048; the bare access pattern reaches 4.6 TB/s), the drawing pass is
 // bound by the noise's instructions.  64-byte row segments (W = 4 FP64, 8 FP32)
 // take the bare pattern from 2.7 TB/s (16 bytes) and 3.7 (32 bytes) to 4.6, and
 // the registers of a CU hold four times the strip that the LDS-resident form
 // (k_col_kmult) could, with 4 workgroup barriers instead of about 20.
-// N = 2048, us per launch, k_col_kmult -> this: loaded FP64 420 -> 258, FP32 241 ->
-// 135; correlated FP64 660 -> 485, FP32 445 -> 212; drawing FP64 490 -> 355, FP32
-// 295 -> 171.
+// N = 2048, us per launch (kernel trace, averages), k_col_kmult -> this: loaded FP64 420 ->
+// 298, FP32 241 -> 146; correlated FP64 660 -> 546, FP32 445 -> 234; drawing FP64 490 -> 403,
+// FP32 295 -> 183.
 // ---------------------------------------------------------------------------
 template <int N, typename C>
 struct ColR {

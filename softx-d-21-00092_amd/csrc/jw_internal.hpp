@@ -105,9 +105,9 @@ struct jw_ctx {
     size_t ws_planes;
     // 1: evolve through the unfused kernel sequence even where the fused passes exist
     int unfused;
-    // fused step's intermediate-plane layout: 0 row-major (X and Y tiles of
-    // 32-byte column strips in LDS), 1 row-major (one plane at a time over
-    // 64-byte strips), 4 or 8 rows per block, -1 default
+    // fused step's intermediate-plane layout: 0 row-major (X and Y strips in registers, or
+    // in LDS for the matrix-core stages), 1, 16, 32 row-major (one plane at a time over
+    // 64-, 32- or 16-byte strips), 2 interleaved, 4 or 8 rows per block, -1 default
     int layout;
     // 1: the FP32 row-major column passes run their radix-16 stages as
     // split-BF16 DFT-matrix products on the matrix cores (jw_set_mixed_fft)

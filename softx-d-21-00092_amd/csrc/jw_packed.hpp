@@ -67,7 +67,7 @@ __global__ __launch_bounds__((ColCfg<N, C>::NT)) void k_fft_cols(C* __restrict__
         base[(size_t)(i / G::W) * N + (i % G::W)] = cscale(lds[lpos<G::W, 1, 3>(i / G::W, i % G::W)], (T)scale);
 }
 
-// From N = 64 on the transforms run in registers (jw_regfft.hpp), T threads a row or a
+// From N = 64 on the FP64 transforms run in registers (jw_regfft.hpp), T threads a row or a
 // column, and LDS is touched by one exchange over the workgroup and one inside a wave
 // instead of by every radix-8 stage; a column strip is a 64-byte segment wide.  Bound by
 // memory: nine planes of FP64 at N = 512 (2 x 38 MB), rows 17.0 -> 16.8 us, columns 22.0 ->

@@ -191,9 +191,9 @@ struct RegTw {
 // 754 us a step of fixed coupling).  rms error of forward, multiply, inverse against
 // extended precision, radix-8 passes in LDS -> here: FP64 N = 64 3.21e-16 -> 3.00e-16, 128 3.53 ->
 // 3.61, 256 3.73 -> 3.76, 512 4.21 -> 4.18, 1024 4.38 -> 4.11, 2048 4.57 -> 4.51, 4096 5.04 ->
-// 4.69, 8192 5.15 -> 4.87 (products: 4.48 at 1024, 4.82 at 2048); FP32 with the table 1.72e-7
-// -> 1.69e-7 at 64, 1.94 -> 1.85 at 128, 2.82 -> 2.06 at 4096, 3.00 -> 2.72 at 8192, with products
-// 2.82 -> 2.5 at 1024, 3.00 -> 2.6 at 2048 (2.8 and 3.1 at 4096 and 8192).
+// 4.69, 8192 5.15 -> 4.87 (products of two, no fused constants: 4.48 at 1024, 4.82 at 2048);
+// FP32 (LDS: two-level table) with the table 1.72e-7 -> 1.69e-7 at 64, 1.94 -> 1.85 at 128, 2.82 ->
+// 2.59 at 4096, 3.00 -> 2.72 at 8192, with products 2.82 -> 2.52 at 1024, 3.00 -> 2.63 at 2048.
 template <int N, typename C>
 struct TwRule {
     static constexpr bool TABLE = RegFft<N>::PT <= 8 || sizeof(C) == sizeof(double2) || N >= 4096;
